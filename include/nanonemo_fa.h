@@ -80,6 +80,20 @@ int nn_fa_bwd_strided(const void* dO, const void* q, const void* k, const void* 
                       const int64_t qo_strides[3], const int64_t kv_strides[3],
                       int dtype, float scale, void* stream);
 
+/* Forward and backward on views whose layouts differ: `strides` holds element triples {batch, head, row} for q (in the
+ * backward, of dO too), for k and v, for o and, in the backward, for dq and for dk and dv (9 and 15 values). Every
+ * stride is a positive multiple of 8 elements. For callers whose tensors are views of projections, such as a
+ * transposed (B, T, heads, D) tensor with a dense output: the .contiguous() copies of
+ * /root/reference/nanonemo/kernels/cuda/flash_attn.py:20,33 are not needed. */
+int nn_fa_fwd_views(const void* q, const void* k, const void* v, void* o, float* lse,
+                    int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D, const int64_t* strides,
+                    int dtype, float scale, void* stream);
+int nn_fa_bwd_views(const void* dO, const void* q, const void* k, const void* v, const void* o,
+                    const float* lse, void* dq, void* dk, void* dv,
+                    void* workspace, size_t workspace_bytes,
+                    int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D, const int64_t* strides,
+                    int dtype, float scale, void* stream);
+
 /* Forward with the rotary position embedding of q folded in: as nn_fa_fwd_strided, with q holding the
  * projections *before* RoPE. Each query row is rotated in registers (rotate-half, dimension i paired with
  * i + D/2, angle of the row's position: y[i] = x[i] cos - x[i+D/2] sin, y[i+D/2] = x[i] sin + x[i+D/2] cos,

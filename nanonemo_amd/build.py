@@ -52,6 +52,10 @@ HIPCC_FLAGS = [
     # no other kernel's code changes).
     "-mllvm",
     "-amdgpu-mfma-vgpr-form=1",
+    # The first 16 dwords of a kernel's arguments arrive in scalar registers with the launch instead of by a scalar load
+    # at its start: the forward 1.5-3 % faster at B=1-32, T=256-512, other kernels and shapes within noise.
+    "-mllvm",
+    "-amdgpu-kernarg-preload-count=16",
 ]
 
 

@@ -326,11 +326,18 @@ __device__ inline QBlk qblock_of(int bid, int BH, int group, int nqb) {
 }
 
 // Element strides of a [B][heads][T][D] tensor view whose D stride is 1: batch, head and row
-// (sequence position). Q, O, dO and dQ share one layout; K, V, dK and dV another.
+// (sequence position).
 struct Lay {
     long long sb, sh;
     int st;
-    __device__ size_t at(int b, int h) const { return (size_t)b * sb + (size_t)h * sh; }
+    // b, h >= 0 and the strides positive: as unsigned 32 x 64-bit products, which take fewer scalar instructions.
+    __device__ size_t at(int b, int h) const { return (uint32_t)b * (uint64_t)sb + (uint32_t)h * (uint64_t)sh; }
+};
+// The layouts of a call's tensors. q and dO share one, k and v another, dk and dv a third: a pair's copies then use one
+// set of per-lane offsets and one scalar offset (with a layout per tensor the kernels took up to 0.35 us longer at the
+// small shapes, and dK/dV has no registers for a second set).
+struct Lays {
+    Lay q, k, o, dq, dk;
 };
 
 // Wait until this wave's vector-memory operations (including LDS DMA) have completed.
@@ -399,7 +406,7 @@ template <int HD, int DT, bool ROPE>
 __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(const u16* __restrict__ Q, const u16* __restrict__ K,
                                                         const u16* __restrict__ V, u16* __restrict__ O,
                                                         float* __restrict__ LSE, int BH, int H, int KVH, int T,
-                                                        int nqb, float sl2, Lay lq, Lay lk, RopeArgs ra) {
+                                                        int nqb, float sl2, Lay lq, Lay lk, Lay lo, RopeArgs ra) {
     using E = Elem<DT>;
     NN_TL_START(kTlFwd);
     constexpr int BM = 128, BN = 128, NW = 4;
@@ -417,9 +424,8 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(const u16* __restrict__ 
     const int b = bh / H, h = bh - b * H;
     const int kvh = h / (H / KVH);
     const size_t qoff = lq.at(b, h);
-    const size_t kvoff = lk.at(b, kvh);
-    const u16* Kp = K + kvoff;
-    const u16* Vp = V + kvoff;
+    const u16* Kp = K + lk.at(b, kvh);
+    const u16* Vp = V + lk.at(b, kvh);
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_kernel(const u16* __restrict__ 
             for (int s = 0; s < NS; ++s) *reinterpret_cast<u16x8*>(qo + 16 * s + 8 * hh) = qf[s];
         }
         const float inv = 1.f / ltot;
-        u16* op = O + qoff + (size_t)qrow * lq.st;
+        u16* op = O + lo.at(b, h) + (size_t)qrow * lo.st;
 #pragma unroll
         for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
@@ -664,7 +670,7 @@ template <int HD, int DT>
 __global__ __launch_bounds__(256) void fa_bwd_pre_kernel(const u16* __restrict__ O, const u16* __restrict__ dO,
                                                          const float* __restrict__ LSE, float* __restrict__ nDvec,
                                                          float* __restrict__ nLvec, int64_t rows, int H, int T,
-                                                         float inv_scale, Lay lq) {
+                                                         float inv_scale, Lay lo, Lay lq) {
     using E = Elem<DT>;
     constexpr int TPR = HD / 8;  // threads per row
     const int64_t gtid = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -674,8 +680,8 @@ __global__ __launch_bounds__(256) void fa_bwd_pre_kernel(const u16* __restrict__
     if (row < rows) {
         const int64_t bh = row / T;
         const int t = (int)(row - bh * T), b = (int)(bh / H), h = (int)(bh - (int64_t)b * H);
-        const size_t off = lq.at(b, h) + (size_t)t * lq.st + 8 * c;
-        const u16x8 o = ld8(O + off), g = ld8(dO + off);
+        const u16x8 o = ld8(O + lo.at(b, h) + (size_t)t * lo.st + 8 * c);
+        const u16x8 g = ld8(dO + lq.at(b, h) + (size_t)t * lq.st + 8 * c);
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc = fmaf(E::to_f32(o[j]), E::to_f32(g[j]), acc);
     }
@@ -716,8 +722,8 @@ template <int HD, int DT, int WPP, bool KVL>
 __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
     const u16* __restrict__ Q, const u16* __restrict__ K, const u16* __restrict__ V, const u16* __restrict__ dO,
     const float* __restrict__ nLvec, const float* __restrict__ nDvec, u16* __restrict__ dK, u16* __restrict__ dV,
-    int BKV, int H, int KVH, int T, int nkb, int nqt, float sl2, float scale, Lay lq, Lay lk, int nsplit,
-    float* __restrict__ part, int paired) {
+    int BKV, int H, int KVH, int T, int nkb, int nqt, float sl2, float scale, Lay lq, Lay lk, Lay ldk,
+    int nsplit, float* __restrict__ part, int paired) {
     using E = Elem<DT>;
     NN_TL_START(kTlDkdv);
     constexpr int BNK = 64, BM = 64, NW = 4, NSL = BNK / 32;
@@ -1141,7 +1147,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
                     for (int sl = 0; sl < NSL; ++sl) {
                         const int key = kb0 + 32 * sl + l32;
                         if (active && key < T) {
-                            u16* row = (which == 0 ? dK : dV) + kvoff + (size_t)key * lk.st;
+                            u16* row = (which == 0 ? dK : dV) + ldk.at(b, kvh) + (size_t)key * ldk.st;
 #pragma unroll
                             for (int k = 0; k < NO; ++k)
                                 if (owned(k) / (4 * ND) == sl)
@@ -1192,7 +1198,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
                 const int ow = wave - wp + c % 4 % WPP;
                 const u32x4 vk = *row16(ow, c, 0, r & 31), vv = *row16(ow, c, 1, r & 31);
                 if (active && kb0 + r < T) {
-                    const size_t off = kvoff + (size_t)(kb0 + r) * lk.st + 8 * j;
+                    const size_t off = ldk.at(b, kvh) + (size_t)(kb0 + r) * ldk.st + 8 * j;
                     *reinterpret_cast<u32x4*>(dK + off) = vk;
                     *reinterpret_cast<u32x4*>(dV + off) = vv;
                 }
@@ -1213,7 +1219,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
 template <int DT>
 __global__ __launch_bounds__(256) void fa_bwd_dkdv_sum_kernel(const float* __restrict__ part, u16* __restrict__ dK,
                                                               u16* __restrict__ dV, int nsplit, int BKV, int KVH,
-                                                              int T, int HD, Lay lk) {
+                                                              int T, int HD, Lay ldk) {
     using E = Elem<DT>;
     const int64_t per = (int64_t)BKV * T * HD;  // elements of one gradient
     const int64_t n4 = 2 * per / 4;
@@ -1227,7 +1233,7 @@ __global__ __launch_bounds__(256) void fa_bwd_dkdv_sum_kernel(const float* __res
         f32x4 acc = *reinterpret_cast<const f32x4*>(part + e);
         for (int s = 1; s < nsplit; ++s) acc += *reinterpret_cast<const f32x4*>(part + (int64_t)s * 2 * per + e);
         const int b = bk / KVH, kvh = bk - b * KVH;
-        u16* dst = (which == 0 ? dK : dV) + lk.at(b, kvh) + (size_t)key * lk.st + col;
+        u16* dst = (which == 0 ? dK : dV) + ldk.at(b, kvh) + (size_t)key * ldk.st + col;
         *reinterpret_cast<u32x2*>(dst) = u32x2{E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
     }
 }
@@ -1247,7 +1253,8 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const u16* __restrict
                                                            const u16* __restrict__ dO, const float* __restrict__ LSE,
                                                            float* __restrict__ nLvec, float* __restrict__ nDvec,
                                                            u16* __restrict__ dQ, int BH, int H, int KVH, int T, int nqb,
-                                                           float sl2, float scale, Lay lq, Lay lk, RopeArgs ra) {
+                                                           float sl2, float scale, Lay lq, Lay lk, Lay lo, Lay ldq,
+                                                           RopeArgs ra) {
     using E = Elem<DT>;
     NN_TL_START(kTlDq);
     // LDS tiles of BT = 128 keys (one barrier and one tile wait per 128 keys), each processed as two BN = 64-key
@@ -1267,10 +1274,8 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const u16* __restrict
     const int bh = blk.bh, qb = blk.qb;
     const int b = bh / H, h = bh - b * H;
     const int kvh = h / (H / KVH);
-    const size_t qoff = lq.at(b, h);
-    const size_t kvoff = lk.at(b, kvh);
-    const u16* Kp = K + kvoff;
-    const u16* Vp = V + kvoff;
+    const u16* Kp = K + lk.at(b, kvh);
+    const u16* Vp = V + lk.at(b, kvh);
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1298,9 +1303,10 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const u16* __restrict
     const float lse = LSE[(size_t)bh * T + qc_];
     if (qw < T) {
         const DmaOffs<HD, 32, 1> rfo = dma_offsets<HD, 32, 1>(lane, 0, lq.st);
-        dma_rows<HD, 32, 1>(Q + qoff, lq.st, qw, T, kB + 32 * wave * HD, 0, rfo);
-        dma_rows<HD, 32, 1>(dO + qoff, lq.st, qw, T, vB + 32 * wave * HD, 0, rfo);
-        dma_rows<HD, 32, 1>(O + qoff, lq.st, qw, T, oS + 32 * wave * HD, 0, rfo);
+        const DmaOffs<HD, 32, 1> ofo = dma_offsets<HD, 32, 1>(lane, 0, lo.st);
+        dma_rows<HD, 32, 1>(Q + lq.at(b, h), lq.st, qw, T, kB + 32 * wave * HD, 0, rfo);
+        dma_rows<HD, 32, 1>(dO + lq.at(b, h), lq.st, qw, T, vB + 32 * wave * HD, 0, rfo);
+        dma_rows<HD, 32, 1>(O + lo.at(b, h), lo.st, qw, T, oS + 32 * wave * HD, 0, ofo);
     }
     wait_vmem();
     // The preprocessing pass, for this block's rows: D = rowsum(dO * O) from the 16-bit O (each half-wave
@@ -1419,7 +1425,7 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(const u16* __restrict
     }
 
     if (qrow < T) {
-        u16* dst = dQ + qoff + (size_t)qrow * lq.st;
+        u16* dst = dQ + ldq.at(b, h) + (size_t)qrow * ldq.st;
         if constexpr (ROPE) {
             // The gradient reaching the rotated Q, rounded to the 16-bit type as a stored dQ would be, then the
             // rotation by -theta. Element i of dq[dt] is column c = 32 dt + (i / 4) * 8 + 4 hh + i % 4; its pair
@@ -1583,12 +1589,12 @@ Workspace carve(void* base, int64_t B, int64_t H, int64_t KVH, int64_t T, int64_
 
 template <int HD, int DT>
 int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B, int64_t H, int64_t KVH,
-             int64_t T, float scale, Lay lq, Lay lk, RopeArgs ra, hipStream_t st) {
+             int64_t T, float scale, const Lays& l, RopeArgs ra, hipStream_t st) {
     const int nqb = (int)((T + 127) / 128);
     const int BH = (int)(B * H);
     auto launch = [&](auto kern) {
         kern<<<dim3(nqb * BH), dim3(256), 0, st>>>((const u16*)q, (const u16*)k, (const u16*)v, (u16*)o, lse, BH, (int)H,
-                                                   (int)KVH, (int)T, nqb, scale * kLog2e, lq, lk, ra);
+                                                   (int)KVH, (int)T, nqb, scale * kLog2e, l.q, l.k, l.o, ra);
     };
     if (ra.cosT)
         launch(fa_fwd_kernel<HD, DT, true>);
@@ -1599,18 +1605,18 @@ int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, i
 
 template <int HD, int DT>
 int pre_impl(const void* o, const void* dO, const float* lse, const Workspace& w, int64_t B, int64_t H, int64_t KVH,
-             int64_t T, float scale, Lay lq, hipStream_t st) {
+             int64_t T, float scale, const Lays& l, hipStream_t st) {
     (void)KVH;
     const int64_t rows = B * H * T;
     const int64_t blocks = (rows * (HD / 8) + 255) / 256;
     fa_bwd_pre_kernel<HD, DT><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
-        (const u16*)o, (const u16*)dO, lse, w.nD, w.nL, rows, (int)H, (int)T, 1.0f / scale, lq);
+        (const u16*)o, (const u16*)dO, lse, w.nD, w.nL, rows, (int)H, (int)T, 1.0f / scale, l.o, l.q);
     return launch_status("fa_bwd_pre_kernel");
 }
 
 template <int HD, int DT>
 int dkdv_impl(const void* q, const void* k, const void* v, const void* dO, const Workspace& w, void* dk, void* dv,
-              int64_t B, int64_t H, int64_t KVH, int64_t T, float scale, Lay lq, Lay lk, hipStream_t st) {
+              int64_t B, int64_t H, int64_t KVH, int64_t T, float scale, const Lays& l, hipStream_t st) {
     const int nkb = (int)((T + 63) / 64);  // 64-key units
     const int nqt = nkb;                   // 64-row query tiles
     const int npairs = (nkb + 1) / 2;
@@ -1624,7 +1630,7 @@ int dkdv_impl(const void* q, const void* k, const void* v, const void* dO, const
     auto launch = [&](auto kern, int ppb) {
         kern<<<dim3((unsigned)dkdv_blocks(B, KVH, T, mode, w.nsplit)), dim3(256), 0, st>>>(
             (const u16*)q, (const u16*)k, (const u16*)v, (const u16*)dO, w.nL, w.nD, (u16*)dk, (u16*)dv, BKV, (int)H,
-            (int)KVH, (int)T, nkb, nqt, scale * kLog2e, scale, lq, lk, w.nsplit, w.part, paired ? 1 : 0);
+            (int)KVH, (int)T, nkb, nqt, scale * kLog2e, scale, l.q, l.k, l.dk, w.nsplit, w.part, paired ? 1 : 0);
     };
     // K / V through LDS (KVL) for pairs at head_dim 64 up to T = 2048: measured 1-3.4 % faster there (config 2:
     // -3 %), within noise or slower at T >= 4096 and at head_dim 32, where the direct loads stay.
@@ -1642,20 +1648,20 @@ int dkdv_impl(const void* q, const void* k, const void* v, const void* dO, const
     const int64_t n4 = 2 * (int64_t)BKV * T * HD / 4;
     const int blocks = (int)std::min<int64_t>((n4 + 255) / 256, 2048);
     fa_bwd_dkdv_sum_kernel<DT><<<dim3(blocks), dim3(256), 0, st>>>(w.part, (u16*)dk, (u16*)dv, w.nsplit, BKV, (int)KVH,
-                                                                   (int)T, HD, lk);
+                                                                   (int)T, HD, l.dk);
     return launch_status("fa_bwd_dkdv_sum_kernel");
 }
 
 template <int HD, int DT>
 int dq_impl(const void* q, const void* k, const void* v, const void* o, const void* dO, const float* lse,
-            const Workspace& w, void* dq, int64_t B, int64_t H, int64_t KVH, int64_t T, float scale, Lay lq, Lay lk,
+            const Workspace& w, void* dq, int64_t B, int64_t H, int64_t KVH, int64_t T, float scale, const Lays& l,
             RopeArgs ra, hipStream_t st) {
     const int nqb = (int)((T + 127) / 128);
     const int BH = (int)(B * H);
     auto launch = [&](auto kern) {
         kern<<<dim3(nqb * BH), dim3(256), 0, st>>>((const u16*)q, (const u16*)k, (const u16*)v, (const u16*)o,
                                                    (const u16*)dO, lse, w.nL, w.nD, (u16*)dq, BH, (int)H, (int)KVH,
-                                                   (int)T, nqb, scale * kLog2e, scale, lq, lk, ra);
+                                                   (int)T, nqb, scale * kLog2e, scale, l.q, l.k, l.o, l.dq, ra);
     };
     if (ra.cosT)
         launch(fa_bwd_dq_kernel<HD, DT, true>);
@@ -1666,6 +1672,9 @@ int dq_impl(const void* q, const void* k, const void* v, const void* o, const vo
 
 // Dense [B][heads][T][D] layout.
 Lay contiguous(int64_t heads, int64_t T, int64_t D) { return Lay{(long long)(heads * T * D), (long long)(T * D), (int)D}; }
+
+// Every tensor's layout for a call in which q, o, dO and dq share one and k, v, dk and dv another.
+Lays shared_lays(Lay q, Lay k) { return Lays{q, k, q, q, k}; }
 
 // Validates caller-given element strides {batch, head, row} of a [B][heads][T][D] view with unit D
 // stride: every stride a positive multiple of 8 elements (16-byte rows, so tiles move 16 bytes
@@ -1679,6 +1688,34 @@ int take_layout(const int64_t* strides, int64_t heads, int64_t T, int64_t D, con
     if (T * st >= ((int64_t)1 << 30) || sb >= ((int64_t)1 << 40) || sh * heads >= ((int64_t)1 << 40))
         return fail(-1, "%s strides too large", what);
     *out = Lay{(long long)sb, (long long)sh, (int)st};
+    return 0;
+}
+
+// The strides a caller gives, as element triples {batch, head, row}: one triple for q, o, dO and dq and one for k, v,
+// dk and dv (null: dense), or `each`, one per layout of Lays: q (and dO), k and v, o and, for the backward, dq, dk
+// and dv.
+struct Strides {
+    const int64_t *qo = nullptr, *kv = nullptr, *each = nullptr;
+};
+int take_lays(const Strides& sd, bool bwd, int64_t H, int64_t KVH, int64_t T, int64_t D, Lays* out) {
+    if (!sd.each) {
+        Lay q = contiguous(H, T, D), k = contiguous(KVH, T, D);
+        if (sd.qo)
+            if (int e = take_layout(sd.qo, H, T, D, "q/o", &q)) return e;
+        if (sd.kv)
+            if (int e = take_layout(sd.kv, KVH, T, D, "k/v", &k)) return e;
+        *out = shared_lays(q, k);
+        return 0;
+    }
+    Lays l{};
+    const struct {
+        Lay* to;
+        int64_t heads;
+        const char* what;
+    } all[5] = {{&l.q, H, "q/dO"}, {&l.k, KVH, "k/v"}, {&l.o, H, "o"}, {&l.dq, H, "dq"}, {&l.dk, KVH, "dk/dv"}};
+    for (int i = 0; i < (bwd ? 5 : 3); ++i)
+        if (int e = take_layout(sd.each + 3 * i, all[i].heads, T, D, all[i].what, all[i].to)) return e;
+    *out = l;
     return 0;
 }
 
@@ -1701,7 +1738,7 @@ int check_ws(void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int6
 
 NNFA_API const char* nn_fa_last_error(void) { return g_last_error.c_str(); }
 
-NNFA_API int nn_fa_abi_version(void) { return 10; }
+NNFA_API int nn_fa_abi_version(void) { return 11; }
 
 NNFA_API size_t nn_fa_bwd_workspace_size(int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D) {
     if (B < 0 || H < 0 || KVH < 0 || T < 0 || D < 0) return 0;
@@ -1733,8 +1770,8 @@ int check_rope(const float* cos_table, const float* sin_table, int64_t table_row
 }
 
 int fwd_entry(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B, int64_t H, int64_t KVH,
-              int64_t T, int64_t D, int dtype, float scale, const int64_t* qo_strides, const int64_t* kv_strides,
-              void* stream, RopeArgs ra = {}, int64_t table_rows = 0) {
+              int64_t T, int64_t D, int dtype, float scale, const Strides& sd, void* stream, RopeArgs ra = {},
+              int64_t table_rows = 0) {
     g_last_error.clear();
     if (int e = check_dims(B, H, KVH, T, D, dtype)) return e;
     if (B == 0 || T == 0) return 0;
@@ -1744,65 +1781,54 @@ int fwd_entry(const void* q, const void* k, const void* v, void* o, float* lse, 
         if (int e = check_rope(ra.cosT, ra.sinT, table_rows, T)) return e;
         if (!ra.qrot || !aligned16(ra.qrot)) return fail(-1, "q_rot must be a 16-byte aligned buffer");
     }
-    Lay lq = contiguous(H, T, D), lk = contiguous(KVH, T, D);
-    if (qo_strides)
-        if (int e = take_layout(qo_strides, H, T, D, "q/o", &lq)) return e;
-    if (kv_strides)
-        if (int e = take_layout(kv_strides, KVH, T, D, "k/v", &lk)) return e;
-    return NNFA_DISPATCH(fwd_impl, D, dtype, q, k, v, o, lse, B, H, KVH, T, scale, lq, lk, ra, (hipStream_t)stream);
+    Lays l;
+    if (int e = take_lays(sd, false, H, KVH, T, D, &l)) return e;
+    return NNFA_DISPATCH(fwd_impl, D, dtype, q, k, v, o, lse, B, H, KVH, T, scale, l, ra, (hipStream_t)stream);
 }
 
-// Shared argument checks of the backward stages; fills the workspace view and the two layouts.
+// Shared argument checks of the backward stages; fills the workspace view and the layouts.
 int bwd_prologue(const void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int64_t KVH, int64_t T,
-                 int64_t D, int dtype, const int64_t* qo_strides, const int64_t* kv_strides, Workspace* w, Lay* lq,
-                 Lay* lk) {
+                 int64_t D, int dtype, const Strides& sd, Workspace* w, Lays* l) {
     g_last_error.clear();
     if (int e = check_dims(B, H, KVH, T, D, dtype)) return e;
     if (B == 0 || T == 0) return 1;  // nothing to do
     if (int e = check_ws((void*)workspace, workspace_bytes, B, H, KVH, T, D)) return e;
     *w = carve((void*)workspace, B, H, KVH, T, D);
-    *lq = contiguous(H, T, D);
-    *lk = contiguous(KVH, T, D);
-    if (qo_strides)
-        if (int e = take_layout(qo_strides, H, T, D, "q/o", lq)) return e;
-    if (kv_strides)
-        if (int e = take_layout(kv_strides, KVH, T, D, "k/v", lk)) return e;
-    return 0;
+    return take_lays(sd, true, H, KVH, T, D, l);
 }
 
 int pre_entry(const void* o, const void* dO, const float* lse, void* workspace, size_t workspace_bytes, int64_t B,
-              int64_t H, int64_t KVH, int64_t T, int64_t D, int dtype, float scale, const int64_t* qo_strides,
-              void* stream) {
+              int64_t H, int64_t KVH, int64_t T, int64_t D, int dtype, float scale, void* stream) {
     Workspace w;
-    Lay lq, lk;
-    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, qo_strides, nullptr, &w, &lq, &lk))
+    Lays l;
+    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, {}, &w, &l))
         return e > 0 ? 0 : e;
     if (!o || !dO || !lse) return fail(-1, "null pointer argument");
     if (!aligned16(o) || !aligned16(dO)) return fail(-1, "inputs must be 16-byte aligned");
     if (!(scale > 0.f)) return fail(-1, "scale must be positive");
-    return NNFA_DISPATCH(pre_impl, D, dtype, o, dO, lse, w, B, H, KVH, T, scale, lq, (hipStream_t)stream);
+    return NNFA_DISPATCH(pre_impl, D, dtype, o, dO, lse, w, B, H, KVH, T, scale, l, (hipStream_t)stream);
 }
 
 int dkdv_entry(const void* q, const void* k, const void* v, const void* dO, void* workspace,
                size_t workspace_bytes, void* dk, void* dv, int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D,
-               int dtype, float scale, const int64_t* qo_strides, const int64_t* kv_strides, void* stream) {
+               int dtype, float scale, const Strides& sd, void* stream) {
     Workspace w;
-    Lay lq, lk;
-    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, qo_strides, kv_strides, &w, &lq, &lk))
+    Lays l;
+    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, sd, &w, &l))
         return e > 0 ? 0 : e;
     if (!q || !k || !v || !dO || !dk || !dv) return fail(-1, "null pointer argument");
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(dO) || !aligned16(dk) || !aligned16(dv))
         return fail(-1, "inputs must be 16-byte aligned");
-    return NNFA_DISPATCH(dkdv_impl, D, dtype, q, k, v, dO, w, dk, dv, B, H, KVH, T, scale, lq, lk, (hipStream_t)stream);
+    return NNFA_DISPATCH(dkdv_impl, D, dtype, q, k, v, dO, w, dk, dv, B, H, KVH, T, scale, l, (hipStream_t)stream);
 }
 
 int dq_entry(const void* q, const void* k, const void* v, const void* o, const void* dO, const float* lse,
              void* workspace, size_t workspace_bytes, void* dq, int64_t B, int64_t H, int64_t KVH, int64_t T,
-             int64_t D, int dtype, float scale, const int64_t* qo_strides, const int64_t* kv_strides, void* stream,
+             int64_t D, int dtype, float scale, const Strides& sd, void* stream,
              RopeArgs ra = {}, int64_t table_rows = 0) {
     Workspace w;
-    Lay lq, lk;
-    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, qo_strides, kv_strides, &w, &lq, &lk))
+    Lays l;
+    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, sd, &w, &l))
         return e > 0 ? 0 : e;
     if (!q || !k || !v || !o || !dO || !lse || !dq) return fail(-1, "null pointer argument");
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(dO) || !aligned16(dq))
@@ -1810,18 +1836,18 @@ int dq_entry(const void* q, const void* k, const void* v, const void* o, const v
     if (!(scale > 0.f)) return fail(-1, "scale must be positive");
     if (ra.cosT || ra.sinT)
         if (int e = check_rope(ra.cosT, ra.sinT, table_rows, T)) return e;
-    return NNFA_DISPATCH(dq_impl, D, dtype, q, k, v, o, dO, lse, w, dq, B, H, KVH, T, scale, lq, lk, ra,
+    return NNFA_DISPATCH(dq_impl, D, dtype, q, k, v, o, dO, lse, w, dq, B, H, KVH, T, scale, l, ra,
                          (hipStream_t)stream);
 }
 
 int bwd_entry(const void* dO, const void* q, const void* k, const void* v, const void* o, const float* lse, void* dq,
               void* dk, void* dv, void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int64_t KVH,
-              int64_t T, int64_t D, int dtype, float scale, const int64_t* qo_strides, const int64_t* kv_strides,
-              void* stream, RopeArgs ra = {}, int64_t table_rows = 0) {
+              int64_t T, int64_t D, int dtype, float scale, const Strides& sd, void* stream, RopeArgs ra = {},
+              int64_t table_rows = 0) {
     // Every argument of the three stages is checked before the first launch.
     Workspace w;
-    Lay lq, lk;
-    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, qo_strides, kv_strides, &w, &lq, &lk))
+    Lays l;
+    if (int e = bwd_prologue(workspace, workspace_bytes, B, H, KVH, T, D, dtype, sd, &w, &l))
         return e > 0 ? 0 : e;
     if (!dO || !q || !k || !v || !o || !lse || !dq || !dk || !dv) return fail(-1, "null pointer argument");
     if (!aligned16(dO) || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(dq) ||
@@ -1832,52 +1858,50 @@ int bwd_entry(const void* dO, const void* q, const void* k, const void* v, const
         if (int e = check_rope(ra.cosT, ra.sinT, table_rows, T)) return e;
     // dQ first: it also computes -D and -lse/scale for its rows into the workspace (the preprocessing
     // pass, fused), which the dK/dV kernel reads.
-    if (int e = dq_entry(q, k, v, o, dO, lse, workspace, workspace_bytes, dq, B, H, KVH, T, D, dtype, scale, qo_strides,
-                         kv_strides, stream, ra, table_rows))
+    if (int e = dq_entry(q, k, v, o, dO, lse, workspace, workspace_bytes, dq, B, H, KVH, T, D, dtype, scale, sd, stream, ra,
+                         table_rows))
         return e;
-    return dkdv_entry(q, k, v, dO, workspace, workspace_bytes, dk, dv, B, H, KVH, T, D, dtype, scale, qo_strides,
-                      kv_strides, stream);
+    return dkdv_entry(q, k, v, dO, workspace, workspace_bytes, dk, dv, B, H, KVH, T, D, dtype, scale, sd, stream);
 }
 
 }  // namespace
 
 NNFA_API int nn_fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B, int64_t H,
                        int64_t KVH, int64_t T, int64_t D, int dtype, float scale, void* stream) {
-    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, nullptr, nullptr, stream);
+    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, {}, stream);
 }
 
 NNFA_API int nn_fa_fwd_strided(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B, int64_t H,
                                int64_t KVH, int64_t T, int64_t D, const int64_t* qo_strides, const int64_t* kv_strides,
                                int dtype, float scale, void* stream) {
     if (!qo_strides || !kv_strides) return fail(-1, "null strides");
-    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, qo_strides, kv_strides, stream);
+    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, {qo_strides, kv_strides}, stream);
 }
 
 NNFA_API int nn_fa_bwd_pre(const void* o, const void* dO, const float* lse, void* workspace, size_t workspace_bytes,
                            int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D, int dtype, float scale,
                            void* stream) {
-    return pre_entry(o, dO, lse, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale, nullptr, stream);
+    return pre_entry(o, dO, lse, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale, stream);
 }
 
 NNFA_API int nn_fa_bwd_dkdv(const void* q, const void* k, const void* v, const void* dO, void* workspace,
                             size_t workspace_bytes, void* dk, void* dv, int64_t B, int64_t H, int64_t KVH, int64_t T,
                             int64_t D, int dtype, float scale, void* stream) {
-    return dkdv_entry(q, k, v, dO, workspace, workspace_bytes, dk, dv, B, H, KVH, T, D, dtype, scale, nullptr, nullptr,
+    return dkdv_entry(q, k, v, dO, workspace, workspace_bytes, dk, dv, B, H, KVH, T, D, dtype, scale, {},
                       stream);
 }
 
 NNFA_API int nn_fa_bwd_dq(const void* q, const void* k, const void* v, const void* o, const void* dO, const float* lse,
                           void* workspace, size_t workspace_bytes, void* dq, int64_t B, int64_t H, int64_t KVH,
                           int64_t T, int64_t D, int dtype, float scale, void* stream) {
-    return dq_entry(q, k, v, o, dO, lse, workspace, workspace_bytes, dq, B, H, KVH, T, D, dtype, scale, nullptr,
-                    nullptr, stream);
+    return dq_entry(q, k, v, o, dO, lse, workspace, workspace_bytes, dq, B, H, KVH, T, D, dtype, scale, {}, stream);
 }
 
 NNFA_API int nn_fa_bwd(const void* dO, const void* q, const void* k, const void* v, const void* o, const float* lse,
                        void* dq, void* dk, void* dv, void* workspace, size_t workspace_bytes, int64_t B, int64_t H,
                        int64_t KVH, int64_t T, int64_t D, int dtype, float scale, void* stream) {
     return bwd_entry(dO, q, k, v, o, lse, dq, dk, dv, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale,
-                     nullptr, nullptr, stream);
+                     {}, stream);
 }
 
 NNFA_API int nn_fa_bwd_strided(const void* dO, const void* q, const void* k, const void* v, const void* o,
@@ -1886,7 +1910,23 @@ NNFA_API int nn_fa_bwd_strided(const void* dO, const void* q, const void* k, con
                                const int64_t* kv_strides, int dtype, float scale, void* stream) {
     if (!qo_strides || !kv_strides) return fail(-1, "null strides");
     return bwd_entry(dO, q, k, v, o, lse, dq, dk, dv, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale,
-                     qo_strides, kv_strides, stream);
+                     {qo_strides, kv_strides}, stream);
+}
+
+NNFA_API int nn_fa_fwd_views(const void* q, const void* k, const void* v, void* o, float* lse, int64_t B, int64_t H,
+                             int64_t KVH, int64_t T, int64_t D, const int64_t* strides, int dtype, float scale,
+                             void* stream) {
+    if (!strides) return fail(-1, "null strides");
+    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, {nullptr, nullptr, strides}, stream);
+}
+
+NNFA_API int nn_fa_bwd_views(const void* dO, const void* q, const void* k, const void* v, const void* o,
+                             const float* lse, void* dq, void* dk, void* dv, void* workspace, size_t workspace_bytes,
+                             int64_t B, int64_t H, int64_t KVH, int64_t T, int64_t D, const int64_t* strides, int dtype,
+                             float scale, void* stream) {
+    if (!strides) return fail(-1, "null strides");
+    return bwd_entry(dO, q, k, v, o, lse, dq, dk, dv, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale,
+                     {nullptr, nullptr, strides}, stream);
 }
 
 NNFA_API int nn_fa_fwd_rope_strided(const void* q, const void* k, const void* v, void* o, float* lse, void* q_rot,
@@ -1896,7 +1936,7 @@ NNFA_API int nn_fa_fwd_rope_strided(const void* q, const void* k, const void* v,
     if (!qo_strides || !kv_strides) return fail(-1, "null strides");
     const RopeArgs ra{cos_table, sin_table, (u16*)q_rot};
     if (!cos_table || !sin_table || !q_rot) return fail(-1, "null RoPE table or q_rot");
-    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, qo_strides, kv_strides, stream, ra, table_rows);
+    return fwd_entry(q, k, v, o, lse, B, H, KVH, T, D, dtype, scale, {qo_strides, kv_strides}, stream, ra, table_rows);
 }
 
 NNFA_API int nn_fa_bwd_rope_strided(const void* dO, const void* q_rot, const void* k, const void* v, const void* o,
@@ -1909,7 +1949,7 @@ NNFA_API int nn_fa_bwd_rope_strided(const void* dO, const void* q_rot, const voi
     if (!cos_table || !sin_table) return fail(-1, "null RoPE table");
     const RopeArgs ra{cos_table, sin_table, nullptr};
     return bwd_entry(dO, q_rot, k, v, o, lse, dq, dk, dv, workspace, workspace_bytes, B, H, KVH, T, D, dtype, scale,
-                     qo_strides, kv_strides, stream, ra, table_rows);
+                     {qo_strides, kv_strides}, stream, ra, table_rows);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1970,8 +2010,7 @@ NNFA_API int nn_fa_bwd_noalloc(const void* dO, const void* q, const void* k, con
                     "use nn_fa_bwd with a caller workspace", need, kNoAllocScratchBytes);
     void* ws = nullptr;
     if (int e = scratch_ptr(stream, &ws)) return e;
-    return bwd_entry(dO, q, k, v, o, lse, dq, dk, dv, ws, kNoAllocScratchBytes, B, H, KVH, T, D, dtype, scale, nullptr,
-                     nullptr, stream);
+    return bwd_entry(dO, q, k, v, o, lse, dq, dk, dv, ws, kNoAllocScratchBytes, B, H, KVH, T, D, dtype, scale, {}, stream);
 }
 
 #if NN_TIMELINE

@@ -45,6 +45,11 @@ SIGNATURES: dict[str, tuple] = {
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i64, _i64, _i64, _i64, _i64p, _i64p, _int, _f32,
          _vp],
     ),
+    "nn_fa_fwd_views": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64p, _int, _f32, _vp]),
+    "nn_fa_bwd_views": (
+        _int,
+        [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i64, _i64, _i64, _i64, _i64, _i64p, _int, _f32, _vp],
+    ),
     "nn_fa_fwd_rope_strided": (
         _int,
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64p, _i64p, _int, _f32, _vp],
@@ -86,7 +91,7 @@ SIGNATURES: dict[str, tuple] = {
     "nn_rmsnorm_last_error": (ctypes.c_char_p, []),
 }
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 
 @cache

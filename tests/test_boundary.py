@@ -150,6 +150,55 @@ def test_strided_c_abi_rejects_bad_strides_before_any_launch(qs, ks, msg):
 
 
 @pytest.mark.parametrize(
+    "which, strides, msg",
+    [
+        (0, (4096, 1024, 60), "q/dO strides must be positive multiples of 8"),
+        (1, (4096, 0, 64), "k/v strides must be positive multiples of 8"),
+        (2, (4096, 1024, 32), "o row stride is smaller than head_dim"),
+        (3, (4096, 1024, 1 << 27), "dq strides too large"),
+        (4, (-4096, 1024, 64), "dk/dv strides must be positive multiples of 8"),
+    ],
+)
+def test_views_c_abi_rejects_bad_strides_before_any_launch(which, strides, msg):
+    L = lib()
+    each = [(4096, 1024, 64)] * 5
+    each[which] = strides
+    arr = lambda n: (ctypes.c_int64 * (3 * n))(*(x for t in each[:n] for x in t))  # noqa: E731
+    if which < 3:
+        rc = L.nn_fa_fwd_views(16, 16, 16, 16, 16, 1, 4, 2, 16, 64, arr(3), 1, 0.125, None)
+        assert rc != 0 and msg in L.nn_fa_last_error().decode()
+    rc = L.nn_fa_bwd_views(16, 16, 16, 16, 16, 16, 16, 16, 16, 256, 1 << 30, 1, 4, 2, 16, 64, arr(5), 1, 0.125, None)
+    assert rc != 0 and msg in L.nn_fa_last_error().decode()
+    rc = L.nn_fa_fwd_views(16, 16, 16, 16, 16, 1, 4, 2, 16, 64, None, 1, 0.125, None)
+    assert rc != 0 and "null strides" in L.nn_fa_last_error().decode()
+
+
+def test_which_views_are_read_in_place():
+    from nanonemo_amd.kernels.hip.flash_attn import _readable, _stride_array, _strides
+
+    B, T, H, D = 2, 5, 3, 32
+    buf = torch.zeros(B, T, H + 2, D, dtype=torch.float16)
+    view = buf[:, :, 1 : 1 + H].transpose(1, 2)  # heads inside a wider projection
+    assert _strides(view) == (T * (H + 2) * D, D, (H + 2) * D) and _readable(view)[0] is view
+    assert list(_stride_array(view, torch.zeros(B, H, T, D))) == [*_strides(view), H * T * D, T * D, D]
+    copied = {
+        "expanded heads": buf[:, :, :1].transpose(1, 2).expand(B, H, T, D),
+        "hd not innermost": torch.zeros(B, H, D, T, dtype=torch.float16).transpose(2, 3),
+        "odd row stride": torch.zeros(B, H, T, D + 4, dtype=torch.float16)[..., :D],
+        "overlapping rows": torch.zeros(B * H * T * D, dtype=torch.float16).as_strided((B, H, T, D), (H * T * 8, T * 8, 8, 1)),
+        "misaligned": torch.zeros(B, T, H, D + 8, dtype=torch.float16)[..., 4 : 4 + D].transpose(1, 2),
+    }
+    for what, t in copied.items():
+        assert _strides(t) is None, what
+        assert _readable(t)[0].is_contiguous() and torch.equal(_readable(t)[0], t), what
+    # a pair must share its strides; a size-1 dimension's stride does not count
+    dense = torch.zeros(B, H, T, D, dtype=torch.float16)
+    assert all(t.is_contiguous() for t in _readable(view, dense))
+    one = torch.zeros(1, 1, H, D, dtype=torch.float16).as_strided((1, H, 1, D), (7, D, 3, 1))
+    assert _strides(one) == (H * D, D, D)
+
+
+@pytest.mark.parametrize(
     "kw, msg",
     [
         (dict(D=56), "head_dim must be a multiple of 16"),

@@ -147,3 +147,40 @@ def test_bthd_compiles_without_graph_breaks():
     assert torch.equal(out, eager)
     for a, b in zip((p.grad for p in params), grads):
         torch.testing.assert_close(a, b, rtol=1e-2, atol=1e-2)
+
+
+def _as(t: torch.Tensor, how: str) -> torch.Tensor:
+    """t (B, h, T, D) with another memory order: "dense", "proj" (a transposed projection), "wide" (heads inside a wider
+    projection, the rest NaN), "odd" (a row stride the kernels cannot read, so the op copies)."""
+    B, h, T, D = t.shape
+    if how == "dense":
+        return t.clone()
+    if how == "odd":
+        return torch.full((B, h, T, D + 4), float("nan"), dtype=t.dtype, device=t.device)[..., :D].copy_(t)
+    pad = 2 if how == "wide" else 0
+    buf = torch.full((B, T, h + pad, D), float("nan"), dtype=t.dtype, device=t.device)
+    return buf[:, :, pad // 2 : pad // 2 + h].transpose(1, 2).copy_(t)
+
+
+@pytest.mark.parametrize("orders", [("proj",) * 4, ("wide", "proj", "wide", "dense"), ("dense", "wide", "wide", "proj"), ("odd", "odd", "proj", "wide")])
+@pytest.mark.parametrize("B, H, KVH, T, hd", [*SHAPES, (2, 12, 1, 1024, 64), (9, 12, 12, 129, 64)])
+def test_views_bit_identical_to_dense(B, H, KVH, T, hd, orders):
+    # flash_attn and both ops read strided q, k, v and d_o in place; the last two shapes split dK/dV and use one
+    # wave per pair.
+    dtype = torch.bfloat16 if hd == 64 else torch.float16
+    print(f"\n[case] views {orders} B={B} H={H} KVH={KVH} T={T} hd={hd} {dtype}", flush=True)
+    fa = _fa()
+    ts = [t.to(DEV) for t in make_inputs(B, H, KVH, T, hd, dtype, seed=7)]
+    ref = _bhtd(*ts)
+    q, k, v, do = (_as(t, how) for t, how in zip(ts, orders))
+    for t in (q, k, v):
+        t.requires_grad_()
+    o = fa.flash_attn(q, k, v)
+    got = (o.detach(), *torch.autograd.grad(o, (q, k, v), do))
+    oo, lse = torch.ops.nanonemo.flash_attn(q.detach(), k.detach(), v.detach())
+    ops = (oo, *torch.ops.nanonemo.flash_attn_bwd(do, q.detach(), k.detach(), v.detach(), oo, lse))
+    torch.cuda.synchronize()
+    assert torch.equal(lse, ref[1])
+    for name, a, b, r in zip(("o", "dq", "dk", "dv"), got, ops, (ref[0], *ref[2:])):
+        assert a.is_contiguous() and b.is_contiguous(), name
+        assert torch.equal(a, r) and torch.equal(b, r), f"{name} differs from the dense path"
