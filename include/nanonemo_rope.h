@@ -43,6 +43,13 @@ int nn_rope_qk_bwd(const void* dq_out, void* dq, const void* dk_out, void* dk,
                    const int64_t q_strides[3], const int64_t k_strides[3], int64_t table_rows,
                    int dtype, void* stream);
 
+/* Either rotation with strides of its own for every tensor: `strides` holds {batch, position, head} triples for q,
+ * q_out, k and k_out (12 values); inverse != 0 is the backward. An output may be its own input. For projections that
+ * share a buffer. */
+int nn_rope_qk_views(const void* q, void* q_out, const void* k, void* k_out, const float* cos_table,
+                     const float* sin_table, int64_t B, int64_t T, int64_t H, int64_t KVH, int64_t D,
+                     const int64_t* strides, int64_t table_rows, int dtype, int inverse, void* stream);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char* nn_rope_last_error(void);
 

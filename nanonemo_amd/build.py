@@ -20,7 +20,7 @@ from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
-SRCS = [PKG / "csrc" / "flash_attn.hip", PKG / "csrc" / "rope.hip", PKG / "csrc" / "rmsnorm.hip"]
+SRCS = [PKG / "csrc" / f"{n}.hip" for n in ("flash_attn", "rope", "rmsnorm", "linear")]
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libnanonemo_fa.so"
 # Block timelines for `bench.py --timeline`: the attention kernels built with NN_TIMELINE=1, so that every block

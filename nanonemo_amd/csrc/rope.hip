@@ -10,8 +10,8 @@
 // The backward applies the inverse rotation (angle -theta) to the incoming gradient.
 //
 // Layout: x is a [B][T][heads][D] view with element strides {batch, row (position), head} and unit D
-// stride; q and k may have different head counts and strides; outputs are written with the same
-// strides as their inputs. The tables are dense fp32 [T_max][half]. The kernel is HBM-bound: each
+// stride; q and k may have different head counts and strides; each output has strides of its own, and
+// may be its input (a thread reads the elements it writes, and only those). The tables are dense fp32 [T_max][half]. The kernel is HBM-bound: each
 // thread moves 8 pairs (two 16-byte loads and two 16-byte stores of 16-bit data).
 #include <hip/hip_runtime.h>
 #include <stdarg.h>
@@ -77,7 +77,8 @@ struct Vec8 {
 struct Side {  // one of q / k
     const char* x;
     char* y;
-    long long sb, st, sh;  // element strides: batch, position, head
+    long long sb, st, sh;     // element strides of x: batch, position, head
+    long long ysb, yst, ysh;  // and of y
 };
 
 // One rounding per product and per sum, as the reference's separate torch ops do: no contraction
@@ -118,6 +119,8 @@ __global__ __launch_bounds__(256) void rope_qk_kernel(Side q, Side k, const floa
     char* yp = isq ? q.y : k.y;
     const long long off = b * (isq ? q.sb : k.sb) + (long long)t * (isq ? q.st : k.st) +
                           (long long)h * (isq ? q.sh : k.sh) + i0;
+    const long long yoff = b * (isq ? q.ysb : k.ysb) + (long long)t * (isq ? q.yst : k.yst) +
+                           (long long)h * (isq ? q.ysh : k.ysh) + i0;
     float x1[8], x2[8], c[8], sn[8], y1[8], y2[8];
     V::load(xp + off * V::bytes, x1);
     V::load(xp + (off + half) * V::bytes, x2);
@@ -135,8 +138,8 @@ __global__ __launch_bounds__(256) void rope_qk_kernel(Side q, Side k, const floa
             y2[j] = sub(mul(x2[j], c[j]), mul(x1[j], sn[j]));
         }
     }
-    V::store(yp + off * V::bytes, y1);
-    V::store(yp + (off + half) * V::bytes, y2);
+    V::store(yp + yoff * V::bytes, y1);
+    V::store(yp + (yoff + half) * V::bytes, y2);
 }
 
 thread_local std::string g_err;
@@ -153,15 +156,17 @@ int fail(const char* fmt, ...) {
 
 bool aligned(const void* p, int n) { return ((uintptr_t)p % n) == 0; }
 
-int check_side(const void* x, const void* y, int64_t heads, const int64_t* strides, int64_t D, int esize,
-               const char* what) {
+int take_side(const void* x, void* y, int64_t heads, const int64_t* strides, const int64_t* out_strides,
+              const char* what, Side* s) {
     if (heads < 0) return fail("invalid %s head count", what);
+    *s = Side{};
     if (heads == 0) return 0;
-    if (!x || !y || !strides) return fail("null %s argument", what);
+    if (!x || !y || !strides || !out_strides) return fail("null %s argument", what);
     for (int i = 0; i < 3; ++i)
-        if (strides[i] <= 0 || strides[i] % 8) return fail("%s strides must be positive multiples of 8 elements", what);
+        if (strides[i] <= 0 || strides[i] % 8 || out_strides[i] <= 0 || out_strides[i] % 8)
+            return fail("%s strides must be positive multiples of 8 elements", what);
     if (!aligned(x, 16) || !aligned(y, 16)) return fail("%s must be 16-byte aligned", what);
-    (void)D;
+    *s = Side{(const char*)x, (char*)y, strides[0], strides[1], strides[2], out_strides[0], out_strides[1], out_strides[2]};
     return 0;
 }
 
@@ -186,7 +191,8 @@ int launch(const Side& q, const Side& k, const float* cosT, const float* sinT, i
 
 int rope_entry(const void* q, void* q_out, const void* k, void* k_out, const float* cos_table, const float* sin_table,
                int64_t B, int64_t T, int64_t H, int64_t KVH, int64_t D, const int64_t* q_strides,
-               const int64_t* k_strides, int64_t table_rows, int dtype, bool inverse, void* stream) {
+               const int64_t* qo_strides, const int64_t* k_strides, const int64_t* ko_strides, int64_t table_rows,
+               int dtype, bool inverse, void* stream) {
     g_err.clear();
     if (B < 0 || T < 0 || D <= 0) return fail("invalid sizes");
     if (D % 16) return fail("head_dim must be a multiple of 16");
@@ -195,13 +201,11 @@ int rope_entry(const void* q, void* q_out, const void* k, void* k_out, const flo
     if (B == 0 || T == 0 || (H == 0 && KVH == 0)) return 0;
     if (!cos_table || !sin_table) return fail("null table");
     if (!aligned(cos_table, 16) || !aligned(sin_table, 16)) return fail("tables must be 16-byte aligned");
-    const int es = dtype == kF32 ? 4 : 2;
-    if (int e = check_side(q, q_out, H, q_strides, D, es, "q")) return e;
-    if (int e = check_side(k, k_out, KVH, k_strides, D, es, "k")) return e;
+    Side sq, sk;
+    if (int e = take_side(q, q_out, H, q_strides, qo_strides, "q", &sq)) return e;
+    if (int e = take_side(k, k_out, KVH, k_strides, ko_strides, "k", &sk)) return e;
     const long long rows = (long long)B * T * (H + KVH);
     if (rows * (D / 16) >= ((int64_t)1 << 31) || T * (D / 2) >= ((int64_t)1 << 31)) return fail("sizes too large");
-    Side sq{(const char*)q, (char*)q_out, H ? q_strides[0] : 0, H ? q_strides[1] : 0, H ? q_strides[2] : 0};
-    Side sk{(const char*)k, (char*)k_out, KVH ? k_strides[0] : 0, KVH ? k_strides[1] : 0, KVH ? k_strides[2] : 0};
     const int half = (int)(D / 2);
     const hipStream_t st = (hipStream_t)stream;
     switch (dtype) {
@@ -217,16 +221,24 @@ NNROPE_API int nn_rope_qk(const void* q, void* q_out, const void* k, void* k_out
                           const float* sin_table, int64_t B, int64_t T, int64_t H, int64_t KVH, int64_t D,
                           const int64_t* q_strides, const int64_t* k_strides, int64_t table_rows, int dtype,
                           void* stream) {
-    return rope_entry(q, q_out, k, k_out, cos_table, sin_table, B, T, H, KVH, D, q_strides, k_strides, table_rows,
-                      dtype, false, stream);
+    return rope_entry(q, q_out, k, k_out, cos_table, sin_table, B, T, H, KVH, D, q_strides, q_strides, k_strides,
+                      k_strides, table_rows, dtype, false, stream);
 }
 
 NNROPE_API int nn_rope_qk_bwd(const void* dq_out, void* dq, const void* dk_out, void* dk, const float* cos_table,
                               const float* sin_table, int64_t B, int64_t T, int64_t H, int64_t KVH, int64_t D,
                               const int64_t* q_strides, const int64_t* k_strides, int64_t table_rows, int dtype,
                               void* stream) {
-    return rope_entry(dq_out, dq, dk_out, dk, cos_table, sin_table, B, T, H, KVH, D, q_strides, k_strides, table_rows,
-                      dtype, true, stream);
+    return rope_entry(dq_out, dq, dk_out, dk, cos_table, sin_table, B, T, H, KVH, D, q_strides, q_strides, k_strides,
+                      k_strides, table_rows, dtype, true, stream);
+}
+
+NNROPE_API int nn_rope_qk_views(const void* q, void* q_out, const void* k, void* k_out, const float* cos_table,
+                                const float* sin_table, int64_t B, int64_t T, int64_t H, int64_t KVH, int64_t D,
+                                const int64_t* strides, int64_t table_rows, int dtype, int inverse, void* stream) {
+    if (!strides) return fail("null strides");
+    return rope_entry(q, q_out, k, k_out, cos_table, sin_table, B, T, H, KVH, D, strides, strides + 3, strides + 6,
+                      strides + 9, table_rows, dtype, inverse != 0, stream);
 }
 
 NNROPE_API const char* nn_rope_last_error(void) { return g_err.c_str(); }

@@ -1,0 +1,137 @@
+"""The model's linear layers under 16-bit autocast, with weight gradients from this build's kernel
+(include/nanonemo_linear.h).
+
+``projections(x, layers)`` applies bias-free ``nn.Linear`` layers that share an input: one product against their
+stacked 16-bit weights, and in the backward one product for the input's gradient and one ``nn_linear_wgrad`` call for
+every weight's, summed and returned in fp32. PyTorch's autocast runs a product per layer each way, rounds every weight
+gradient to 16 bits and casts it back, and adds the input's gradients in 16 bits; the gradient products over
+thousands of tokens into a small matrix are also where the library is slowest (768 x 768 over 8192 tokens: 50 us, of
+which 10 would do).
+
+``can_project(x, layers)`` says whether the call can take this path: plain CUDA tensors and untouched fp32
+``nn.Linear`` layers under 16-bit autocast, in eager mode. Everything else (hooks, parametrizations, other module or
+tensor types, torch.compile, torch.func, forward-mode AD, no autocast) keeps calling the modules. A backward that is
+itself recorded (create_graph) runs differentiable torch products instead of the kernel.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import torch
+from torch import Tensor, nn
+from torch.autograd import forward_ad
+from torch.nn.modules import module as _module
+
+from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check_linear, eager, lib, on_device, stream_of
+
+_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
+# Above this many elements of dW the library's product fills the chip by itself and is the faster one (8192 tokens:
+# 2048 x 2048 at 16384 tokens 140 us here against 165 with its cast, 4096 x 4096 334 against 245).
+_WGRAD_MOST = 6_000_000
+
+
+def plain(m: nn.Module, x: Tensor, width: int) -> bool:
+    """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width."""
+    if type(m) is not nn.Linear or m.bias is not None or "forward" in m.__dict__:
+        return False
+    if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+        return False
+    w = m.weight
+    return (type(w) is nn.Parameter and w.dtype is torch.float32 and w.device == x.device and w.is_contiguous()
+            and w.shape[1] == width and w.shape[0] % 8 == 0 and width % 8 == 0 and w.data_ptr() % 16 == 0)
+
+
+def eligible(x: Tensor) -> bool:
+    """Whether a layer called on x now may run on this build's kernels (see above), whatever its modules."""
+    if not eager(x) or not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") not in _DTYPES:
+        return False
+    if x.dim() < 2 or x.numel() == 0 or not x.is_floating_point() or x.dtype is torch.float64:
+        return False
+    return not (torch.jit.is_tracing() or forward_ad._current_level >= 0 or _module._has_any_global_hook())
+
+
+def can_project(x: Tensor, *layers: nn.Module) -> bool:
+    """Whether ``projections`` can stand for calling the layers on x (see above)."""
+    return eligible(x) and all(plain(m, x, x.shape[-1]) for m in layers)
+
+
+def wgrad(dy: Tensor, x: Tensor, rows: list[int]) -> list[Tensor]:
+    """dy^T x for dy (T, sum(rows)) and x (T, K), 16-bit with unit column strides: fp32, one (rows[i], K) tensor each."""
+    (T, N), K = dy.shape, x.shape[1]
+    if N * K > _WGRAD_MOST:
+        dw = torch.mm(dy.t(), x, out_dtype=torch.float32)
+        return [dw] if len(rows) == 1 else [t.contiguous() for t in dw.split(rows)]
+    out = [torch.empty((r, K), dtype=torch.float32, device=x.device) for r in rows]
+    L, n = lib(), len(rows)
+    ws_bytes = L.nn_linear_wgrad_workspace_size(T, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    with on_device(x):
+        rc = L.nn_linear_wgrad(
+            dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), T, N, K, n,
+            (ctypes.c_void_p * n)(*(t.data_ptr() for t in out)), (ctypes.c_int64 * n)(*rows),
+            ws.data_ptr() if ws_bytes else None, ws_bytes, _DTYPES[x.dtype], stream_of(x),
+        )
+    check_linear(rc)
+    return out
+
+
+def cast_weights(dtype: torch.dtype, *groups: tuple[Tensor, ...]) -> list[Tensor]:
+    """Each group of fp32 (N_i, K) weights stacked into one (sum N_i, K) tensor of a 16-bit dtype, in one launch."""
+    ws = [w for group in groups for w in group]
+    out, dst = [], []
+    for group in groups:
+        t = torch.empty((sum(w.shape[0] for w in group), group[0].shape[1]), dtype=dtype, device=group[0].device)
+        at = t.data_ptr()
+        for w in group:
+            dst.append(at)
+            at += 2 * w.numel()
+        out.append(t)
+    n = len(ws)
+    with on_device(ws[0]):
+        rc = lib().nn_linear_cast(
+            n, (ctypes.c_void_p * n)(*(w.data_ptr() for w in ws)), (ctypes.c_void_p * n)(*dst),
+            (ctypes.c_int64 * n)(*(w.numel() for w in ws)), _DTYPES[dtype], stream_of(ws[0]),
+        )
+    check_linear(rc)
+    return out
+
+
+def stacked(grads: tuple[Tensor | None, ...], rows: list[int], like: Tensor) -> Tensor:
+    """The gradients (T, rows[i]) side by side, zeros for an unused output."""
+    if len(grads) == 1:
+        return grads[0].contiguous()
+    return torch.cat([like.new_zeros(like.shape[0], r) if g is None else g for g, r in zip(grads, rows)], dim=1)
+
+
+class _Projections(torch.autograd.Function):
+    """y_i = x W_i^T: x (T, K) 16-bit, W_i fp32, y_i the column ranges of one (T, sum N_i) product."""
+
+    @staticmethod
+    def forward(ctx, x, *ws):
+        (w16,) = cast_weights(x.dtype, ws)
+        ctx.save_for_backward(x, w16, *ws)
+        ctx.set_materialize_grads(False)
+        y = x @ w16.t()
+        return (y,) if len(ws) == 1 else y.split([w.shape[0] for w in ws], dim=1)
+
+    @staticmethod
+    def backward(ctx, *dys):
+        x, w16, *ws = ctx.saved_tensors
+        rows = [w.shape[0] for w in ws]
+        need_w = any(ctx.needs_input_grad[1:])
+        dy = stacked(dys, rows, x)
+        if torch.is_grad_enabled():  # a recorded backward
+            wd = torch.cat([w.to(x.dtype) for w in ws])
+            dx = dy @ wd if ctx.needs_input_grad[0] else None
+            dws = (dy.t() @ x).float().split(rows) if need_w else [None] * len(ws)
+        else:
+            dx = dy @ w16 if ctx.needs_input_grad[0] else None
+            dws = wgrad(dy, x, rows) if need_w else [None] * len(ws)
+        return dx, *(g if n else None for g, n in zip(dws, ctx.needs_input_grad[1:]))
+
+
+def projections(x: Tensor, *layers: nn.Linear) -> tuple[Tensor, ...]:
+    """The layers' outputs on x (..., K), in the autocast dtype, as (..., N_i) column ranges of one product."""
+    flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
+    return tuple(y.view(*x.shape[:-1], y.shape[1]) for y in _Projections.apply(flat, *(m.weight for m in layers)))

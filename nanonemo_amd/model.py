@@ -78,6 +78,22 @@ class ModelConfig:
     def head_dim(self) -> int:
         return self.d_model // self.n_heads
 
+    @property
+    def any_hip(self) -> bool:
+        """Whether the model runs on this build's kernels; its linear layers then do too (kernels/hip/linear.py)."""
+        return self.attn_kernel != "torch" or self.rope_kernel != "torch" or self.norm_kernel != "torch"
+
+
+def _project(cfg: ModelConfig, x: torch.Tensor, *layers: nn.Module) -> tuple[torch.Tensor, ...]:
+    """The layers' outputs on x, on this build's linear layers where the model uses this build's kernels and the call
+    can take them."""
+    if cfg.any_hip and x.is_cuda:
+        from nanonemo_amd.kernels.hip import linear
+
+        if linear.can_project(x, *layers):
+            return linear.projections(x, *layers)
+    return tuple(layer(x) for layer in layers)
+
 
 class RMSNorm(nn.Module):
     """x / rms(x) * w, reduced in fp32 (as layers.py:23-33) and returned in x's dtype."""
@@ -155,19 +171,27 @@ class Attention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
         B, T, _ = x.shape
-        q = self.wq(x).view(B, T, self.H, self.hd)
-        k = self.wk(x).view(B, T, self.KVH, self.hd)
-        v = self.wv(x).view(B, T, self.KVH, self.hd)
+        if self.cfg.attn_kernel == "hip_bthd" and self.cfg.rope_kernel != "torch" and x.is_cuda:
+            from nanonemo_amd.kernels.hip import layers
+
+            call = (x, cos, sin, self.H, self.KVH)
+            ws = (self.wq, self.wk, self.wv, self.wo)
+            if layers.can_fuse(*call, self.hd, *ws):  # the whole layer in this build's kernels, as one autograd node
+                return layers.attention_layer(*call, *ws)
+        q, k, v = _project(self.cfg, x, self.wq, self.wk, self.wv)
+        q = q.view(B, T, self.H, self.hd)
+        k = k.view(B, T, self.KVH, self.hd)
+        v = v.view(B, T, self.KVH, self.hd)
         if self.cfg.rope_kernel == "fused":  # k rotated here, q inside the attention op
             k = self._rope_k(k, cos, sin)
-            return self.wo(self._fa.flash_attn_bthd_rope(q, k, v, cos, sin).view(B, T, -1))
+            return _project(self.cfg, self._fa.flash_attn_bthd_rope(q, k, v, cos, sin).view(B, T, -1), self.wo)[0]
         hip_rope = self.cfg.rope_kernel == "hip"
         if hip_rope:  # in the projection layout, q and k in one launch
             q, k = self._rope_qk(q, k, cos, sin)
         if self.cfg.attn_kernel == "hip_bthd":
             if not hip_rope:
                 q, k = rope(q, cos, sin, seq_dim=1), rope(k, cos, sin, seq_dim=1)
-            return self.wo(self._fa.flash_attn_bthd(q, k, v).view(B, T, -1))
+            return _project(self.cfg, self._fa.flash_attn_bthd(q, k, v).view(B, T, -1), self.wo)[0]
         q, k, v = q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)  # (B, heads, T, hd) views
         if not hip_rope:
             q, k = rope(q, cos, sin, seq_dim=2), rope(k, cos, sin, seq_dim=2)
@@ -183,7 +207,7 @@ class Attention(nn.Module):
                 backend = {"math": SDPBackend.MATH, "mem_efficient": SDPBackend.EFFICIENT_ATTENTION}[self.cfg.attn_backend]
                 with sdpa_kernel(backend):
                     y = F.scaled_dot_product_attention(q, kr, vr, is_causal=True)
-        return self.wo(y.transpose(1, 2).reshape(B, T, -1))
+        return _project(self.cfg, y.transpose(1, 2).reshape(B, T, -1), self.wo)[0]
 
 
 class MLP(nn.Module):

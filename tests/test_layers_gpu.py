@@ -1,0 +1,96 @@
+"""GPU tests of the fused layers (kernels/hip/layers.py) against the same modules run one by one."""
+
+from __future__ import annotations
+
+import copy
+
+import pytest
+import torch
+
+from nanonemo_amd.model import Attention, ModelConfig, rope_tables
+
+pytestmark = pytest.mark.gpu
+
+
+def _attention(H, KVH, hd, T, **kw):
+    torch.manual_seed(0)
+    cfg = ModelConfig(n_layers=1, d_model=H * hd, n_heads=H, n_kv_heads=KVH, max_seq_len=T, attn_kernel="hip_bthd", **kw)
+    return Attention(cfg).cuda(), tuple(t.cuda() for t in rope_tables(hd, T, 10000.0))
+
+
+def _modules_only(m):
+    """The same module with a no-op hook on each linear layer, which keeps every call on the modules."""
+    m = copy.copy(m)
+    m._modules = {n: copy.deepcopy(c) for n, c in m._modules.items()}
+    for c in m._modules.values():
+        c.register_forward_hook(lambda *_: None)
+    return m
+
+
+def _run(m, args, dy, dtype):
+    with torch.autocast("cuda", dtype=dtype):
+        y = m(*args)
+    return (y.detach(), *torch.autograd.grad(y, (args[0], *m.parameters()), dy))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+# From T = 3: at T = 1 the softmax is constant and the exact gradients of wq and wk are 0, so two correct results differ
+# by all of their rounding noise.
+@pytest.mark.parametrize("B, T, H, KVH, hd", [(2, 200, 12, 4, 64), (1, 3, 4, 1, 32), (3, 65, 2, 2, 64), (1, 1030, 8, 2, 32)])
+def test_attention_layer_matches_its_modules(B, T, H, KVH, hd, dtype):
+    from nanonemo_amd.kernels.hip import layers
+
+    print(f"\n[case] attention layer B={B} T={T} H={H} KVH={KVH} hd={hd} {dtype}", flush=True)
+    m, (cos, sin) = _attention(H, KVH, hd, T, rope_kernel="hip")
+    x = torch.randn(B, T, H * hd, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(B, T, H * hd, device="cuda").to(dtype)
+    ref_m = _modules_only(m)
+    with torch.autocast("cuda", dtype=dtype):
+        assert layers.can_fuse(x, cos, sin, H, KVH, hd, m.wq, m.wk, m.wv, m.wo)
+        assert not layers.can_fuse(x, cos, sin, H, KVH, hd, ref_m.wq, ref_m.wk, ref_m.wv, ref_m.wo)
+    got, ref = _run(m, (x, cos, sin), dy, dtype), _run(ref_m, (x, cos, sin), dy, dtype)
+    # the same 16-bit products with other sums; the reference rounds weight gradients and partial input gradients too
+    tol = 2e-2 if dtype == torch.bfloat16 else 3e-3
+    for name, a, b in zip(("y", "dx", "dwq", "dwk", "dwv", "dwo"), got, ref):
+        assert a.shape == b.shape and a.dtype == b.dtype, name
+        torch.testing.assert_close(a, b, rtol=tol, atol=tol * b.abs().max().item(), msg=name)
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        assert torch.equal(m(x, cos, sin), got[0])
+
+
+def test_attention_layer_frozen_parts_and_repeated_backward():
+    m, (cos, sin) = _attention(4, 2, 64, 70, rope_kernel="hip")
+    x = torch.randn(2, 70, 256, device="cuda", requires_grad=True)  # fp32 in, cast by the layer
+    m.wk.weight.requires_grad_(False)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = m(x, cos, sin)
+    y.float().square().sum().backward(retain_graph=True)
+    first = [t.grad.clone() for t in (x, m.wq.weight, m.wv.weight, m.wo.weight)]
+    assert x.grad.dtype == torch.float32 and m.wk.weight.grad is None
+    y.float().square().sum().backward()
+    for a, t in zip(first, (x, m.wq.weight, m.wv.weight, m.wo.weight)):
+        assert torch.equal(a + a, t.grad)
+    for p in m.parameters():
+        p.requires_grad_(False)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        (gx,) = torch.autograd.grad(m(x, cos, sin).float().square().sum(), x)
+    assert torch.equal(gx, first[0])
+    m.wo.weight.requires_grad_(True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        (gw,) = torch.autograd.grad(m(x.detach(), cos, sin).float().square().sum(), m.wo.weight)
+    assert torch.equal(gw, first[3])
+
+
+def test_attention_layer_recorded_backward():
+    # the gradient of wo's gradient norm with respect to the attention's inputs, which passes through the attention's
+    # first derivative only: as with the modules
+    m, (cos, sin) = _attention(4, 2, 32, 33, rope_kernel="hip")
+    x = torch.randn(2, 33, 128, device="cuda", requires_grad=True)
+    out = []
+    for mod in (m, _modules_only(m)):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = mod(x, cos, sin)
+        (gw,) = torch.autograd.grad(y.float().sum(), mod.wo.weight, create_graph=True)
+        out.append(torch.autograd.grad(gw.square().sum(), x))
+    for a, b in zip(*out):
+        torch.testing.assert_close(a, b, rtol=5e-2, atol=5e-2 * b.abs().max().item())
