@@ -28,6 +28,13 @@ size_t nn_linear_wgrad_workspace_size(int64_t T, int64_t N, int64_t K);
  * 16-byte aligned), in one launch: a layer's weights at the start of its forward. */
 int nn_linear_cast(int n, const float* const* src, void* const* dst, const int64_t* count, int dtype, void* stream);
 
+/* SwiGLU: h = silu(g) u with silu(g) = g / (1 + exp(-g)), in fp32 with one rounding. gu is [T][2 F] (a row's F values
+ * of g, then its F values of u: the stacked product of the gate and up layers), h is [T][F]; dense, 16-byte aligned,
+ * F a multiple of 8. The backward writes dgu = (dh u silu'(g), dh silu(g)), [T][2 F].
+ * Replaces F.silu(gate) * up (/root/reference/nanonemo/model/layers.py:130-137). */
+int nn_swiglu_fwd(const void* gu, void* h, int64_t T, int64_t F, int dtype, void* stream);
+int nn_swiglu_bwd(const void* dh, const void* gu, void* dgu, int64_t T, int64_t F, int dtype, void* stream);
+
 const char* nn_linear_last_error(void);
 
 #ifdef __cplusplus

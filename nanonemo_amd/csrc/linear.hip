@@ -1,5 +1,6 @@
-// Weight gradients of linear layers for MI355X (gfx950): dW = dY^T X, fp32 sums and result.
+// Linear-layer kernels for MI355X (gfx950): weight gradients, weight casts and the SwiGLU activation.
 //
+// Weight gradients: dW = dY^T X, fp32 sums and result.
 // The contraction runs over the tokens, which are the rows of both operands, so both MFMA operands are columns of
 // row-major tiles: tiles move global -> LDS by DMA (tiles.h) and are read with ds_read_b64_tr_b16; nothing is
 // transposed in memory. A weight gradient of this model is a small matrix with a long contraction (768 x 768 over
@@ -235,6 +236,59 @@ __global__ __launch_bounds__(256) void cast_kernel(Casts c) {
                                                   Elem<DT>::pack2(y[0], y[1]), Elem<DT>::pack2(y[2], y[3])};
 }
 
+// SwiGLU forward and backward, eight columns per thread: every input is read once and every output written once, where
+// PyTorch's silu, mul and their backwards move 2.5 times the bytes (8192 x 2048: 34 us forward and 50 backward).
+// HBM-bound; 8192 x 2048: forward 15 us (100 MB, 6.8 TB/s, partly from the last-level cache), backward 24 us (168 MB, 7.0);
+// 32768 x 2048: 68 us (5.9 TB/s) and 116 us (5.8); a 1 GiB device copy runs at 5.1 TB/s.
+template <int DT>
+__device__ inline void widen8(const u16* p, float* v) {
+    const u16x8 w = ld8(p);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = Elem<DT>::to_f32(w[e]);
+}
+template <int DT>
+__device__ inline void round8(u16* p, const float* v) {
+    *reinterpret_cast<u32x4*>(p) = u32x4{Elem<DT>::pack2(v[0], v[1]), Elem<DT>::pack2(v[2], v[3]),
+                                         Elem<DT>::pack2(v[4], v[5]), Elem<DT>::pack2(v[6], v[7])};
+}
+__device__ inline float sigmoid(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
+template <int DT>
+__global__ __launch_bounds__(256) void swiglu_fwd_kernel(const u16* __restrict__ gu, u16* __restrict__ h, int n, int vpr) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int row = i / vpr;
+    const u16* p = gu + ((size_t)i + (size_t)row * vpr) * 8;  // row 2 F + column
+    float g[8], u[8];
+    widen8<DT>(p, g);
+    widen8<DT>(p + (size_t)vpr * 8, u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = g[e] * sigmoid(g[e]) * u[e];
+    round8<DT>(h + (size_t)i * 8, g);
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void swiglu_bwd_kernel(const u16* __restrict__ dh, const u16* __restrict__ gu,
+                                                         u16* __restrict__ dgu, int n, int vpr) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int row = i / vpr;
+    const size_t at = ((size_t)i + (size_t)row * vpr) * 8, up = at + (size_t)vpr * 8;
+    float d[8], g[8], u[8];
+    widen8<DT>(dh + (size_t)i * 8, d);
+    widen8<DT>(gu + at, g);
+    widen8<DT>(gu + up, u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float s = sigmoid(g[e]);
+        const float dg = d[e] * u[e] * (s * fmaf(g[e], 1.f - s, 1.f));  // silu'(g) = s (1 + g (1 - s))
+        u[e] = d[e] * (g[e] * s);
+        g[e] = dg;
+    }
+    round8<DT>(dgu + at, g);
+    round8<DT>(dgu + up, u);
+}
+
 // ------------------------------------------------------------------------------------------
 // Host side.
 // ------------------------------------------------------------------------------------------
@@ -349,4 +403,37 @@ NNLIN_API int nn_linear_cast(int n, const float* const* src, void* const* dst, c
     else
         cast_kernel<kF16><<<grid, dim3(256), 0, (hipStream_t)stream>>>(c);
     return launched("cast_kernel");
+}
+
+namespace {
+int check_swiglu(int64_t T, int64_t F, int dtype, const void* a, const void* b, const void* c) {
+    g_err.clear();
+    if (T < 0 || F < 8 || F % 8) return fail("F must be a positive multiple of 8");
+    if (dtype != kF16 && dtype != kBF16) return fail("dtype must be float16 or bfloat16");
+    if (T * (F / 8) >= ((int64_t)1 << 31) - 256) return fail("sizes too large");
+    if (T && (!a || !b || !c || !aligned16(a) || !aligned16(b) || !aligned16(c))) return fail("tensors must be 16-byte aligned");
+    return 0;
+}
+}  // namespace
+
+NNLIN_API int nn_swiglu_fwd(const void* gu, void* h, int64_t T, int64_t F, int dtype, void* stream) {
+    if (int e = check_swiglu(T, F, dtype, gu, h, h)) return e;
+    if (T == 0) return 0;
+    const int n = (int)(T * (F / 8));
+    auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream>>>((const u16*)gu, (u16*)h, n, (int)(F / 8));
+        return launched("swiglu_fwd_kernel");
+    };
+    return dtype == kBF16 ? go(swiglu_fwd_kernel<kBF16>) : go(swiglu_fwd_kernel<kF16>);
+}
+
+NNLIN_API int nn_swiglu_bwd(const void* dh, const void* gu, void* dgu, int64_t T, int64_t F, int dtype, void* stream) {
+    if (int e = check_swiglu(T, F, dtype, dh, gu, dgu)) return e;
+    if (T == 0) return 0;
+    const int n = (int)(T * (F / 8));
+    auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream>>>((const u16*)dh, (const u16*)gu, (u16*)dgu, n, (int)(F / 8));
+        return launched("swiglu_bwd_kernel");
+    };
+    return dtype == kBF16 ? go(swiglu_bwd_kernel<kBF16>) : go(swiglu_bwd_kernel<kF16>);
 }

@@ -1,15 +1,18 @@
-"""The model's attention layer as one call under 16-bit autocast: projections, rotary embedding, attention and output
-projection, forward and backward (/root/reference/nanonemo/model/layers.py:77-116).
+"""The model's attention layer and MLP as one call each under 16-bit autocast, forward and backward
+(/root/reference/nanonemo/model/layers.py:77-116,119-137).
 
-The layer's own memory order lets every kernel read what the one before it wrote: q, k and v are column ranges of one
+Attention: projections, rotary embedding, attention and output projection. The layer's own memory order lets every kernel read what the one before it wrote: q, k and v are column ranges of one
 product's (B T, (H + 2 KVH) hd) output, the rotation writes q to a tensor of its own and k over itself, the attention
 reads k and v where they lie (nn_fa_fwd_views), and the backward writes dq, dk and dv as column ranges of one buffer,
 rotates them back in place and hands it to one product for the input's gradient and one call for the three weights'.
 That is 6 launches forward and 9 to 11 backward, where the modules take 27 in all: a cast, a product and a rounding
 per weight each way, three input gradients added in 16 bits.
 
-``can_fuse`` holds for the calls that ``linear.can_project`` describes, with every module of the layer untouched;
-the others run module by module. A backward that is itself recorded replays the layer through PyTorch's linear layers
+MLP: one product for gate and up, SwiGLU on its two halves (nn_swiglu_*), the down product; backward, one call for
+the gate's and up's weight gradients and one product for the input's gradient. 4 launches forward and 6 to 8 backward
+instead of 21.
+
+``can_fuse`` and ``can_fuse_mlp`` hold for the calls that ``linear.can_project`` describes, with every module of the layer untouched; the others run module by module. A backward that is itself recorded replays the layer through PyTorch's linear layers
 and the package's differentiable functions, so that what those support is what it supports.
 """
 
@@ -22,7 +25,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check, check_rope, lib, on_device, stream_of
+from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check, check_linear, check_rope, lib, on_device, stream_of
 from nanonemo_amd.kernels.hip.flash_attn import flash_attn_bthd
 from nanonemo_amd.kernels.hip.linear import cast_weights, eligible, plain, wgrad
 from nanonemo_amd.kernels.hip.rope import rope_qk
@@ -142,3 +145,59 @@ def attention_layer(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: i
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(B * T, d)
     y = _AttentionLayer.apply(flat, cos, sin, B, T, heads, kv_heads, wq.weight, wk.weight, wv.weight, wo.weight)
     return y.view(B, T, -1)
+
+
+def can_fuse_mlp(x: Tensor, w_gate, w_up, w_down) -> bool:
+    """Whether ``mlp_layer`` can stand for the MLP's modules called on x."""
+    if not eligible(x) or x.dim() < 2:
+        return False
+    d = x.shape[-1]
+    if not (plain(w_gate, x, d) and plain(w_up, x, d)):
+        return False
+    F_ = w_gate.weight.shape[0]
+    return w_up.weight.shape[0] == F_ and plain(w_down, x, F_) and not torch.cuda.is_current_stream_capturing()
+
+
+class _MlpLayer(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w_gate, w_up, w_down):
+        wgu, wd = cast_weights(x.dtype, (w_gate, w_up), (w_down,))
+        gu = x @ wgu.t()
+        T, F_ = x.shape[0], w_gate.shape[0]
+        h = torch.empty((T, F_), dtype=x.dtype, device=x.device)
+        with on_device(x):
+            check_linear(lib().nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F_, _DTYPES[x.dtype], stream_of(x)))
+        y = h @ wd.t()
+        ctx.save_for_backward(x, gu, h, wgu, wd, w_gate, w_up, w_down)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, gu, h, wgu, wd, w_gate, w_up, w_down = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():
+            return _replayed(_modular_mlp, (x, w_gate, w_up, w_down), need, dy, (), at=1)
+        dy = dy.contiguous()
+        dwd = wgrad(dy, h, [w_down.shape[0]])[0] if need[3] else None
+        if not (need[0] or need[1] or need[2]):
+            return None, None, None, dwd
+        dh = dy @ wd
+        dgu = torch.empty_like(gu)
+        T, F_ = h.shape
+        with on_device(x):
+            check_linear(lib().nn_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), T, F_, _DTYPES[x.dtype], stream_of(x)))
+        dx = dgu @ wgu if need[0] else None
+        dwg, dwu = wgrad(dgu, x, [F_, F_]) if need[1] or need[2] else (None, None)
+        return dx, dwg if need[1] else None, dwu if need[2] else None, dwd
+
+
+def _modular_mlp(x, w_gate, w_up, w_down):
+    """The MLP through differentiable functions, in x's dtype."""
+    return F.linear(F.silu(F.linear(x, w_gate.to(x.dtype))) * F.linear(x, w_up.to(x.dtype)), w_down.to(x.dtype))
+
+
+def mlp_layer(x: Tensor, w_gate: nn.Linear, w_up: nn.Linear, w_down: nn.Linear) -> Tensor:
+    """w_down(silu(w_gate x) * w_up x) on x (..., d) in the autocast dtype, for calls that can_fuse_mlp."""
+    flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
+    y = _MlpLayer.apply(flat, w_gate.weight, w_up.weight, w_down.weight)
+    return y.view(*x.shape[:-1], y.shape[1])

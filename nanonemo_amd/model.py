@@ -218,8 +218,15 @@ class MLP(nn.Module):
         self.w_gate = nn.Linear(cfg.d_model, cfg.d_ff, bias=False)
         self.w_up = nn.Linear(cfg.d_model, cfg.d_ff, bias=False)
         self.w_down = nn.Linear(cfg.d_ff, cfg.d_model, bias=False)
+        self.any_hip = cfg.any_hip
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if self.any_hip and x.is_cuda:
+            from nanonemo_amd.kernels.hip import layers
+
+            ws = (self.w_gate, self.w_up, self.w_down)
+            if layers.can_fuse_mlp(x, *ws):
+                return layers.mlp_layer(x, *ws)
         return self.w_down(F.silu(self.w_gate(x)) * self.w_up(x))
 
 

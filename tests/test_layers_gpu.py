@@ -7,7 +7,7 @@ import copy
 import pytest
 import torch
 
-from nanonemo_amd.model import Attention, ModelConfig, rope_tables
+from nanonemo_amd.model import MLP, Attention, ModelConfig, rope_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +94,57 @@ def test_attention_layer_recorded_backward():
         out.append(torch.autograd.grad(gw.square().sum(), x))
     for a, b in zip(*out):
         torch.testing.assert_close(a, b, rtol=5e-2, atol=5e-2 * b.abs().max().item())
+
+
+def _mlp(d, ff):
+    torch.manual_seed(0)
+    return MLP(ModelConfig(n_layers=1, d_model=d, n_heads=1, n_kv_heads=1, d_ff=ff, attn_kernel="hip_bthd")).cuda()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape, d, ff", [((2, 200), 96, 264), ((1, 1), 64, 8), ((700,), 768, 2048), ((3, 5, 7), 40, 72)])
+def test_mlp_layer_matches_its_modules(shape, d, ff, dtype):
+    from nanonemo_amd.kernels.hip import layers
+
+    print(f"\n[case] MLP layer {shape} d={d} ff={ff} {dtype}", flush=True)
+    m = _mlp(d, ff)
+    x = torch.randn(*shape, d, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(*shape, d, device="cuda").to(dtype)
+    ref_m = _modules_only(m)
+    with torch.autocast("cuda", dtype=dtype):
+        assert layers.can_fuse_mlp(x, m.w_gate, m.w_up, m.w_down)
+        assert not layers.can_fuse_mlp(x, ref_m.w_gate, ref_m.w_up, ref_m.w_down)
+    got, ref = _run(m, (x,), dy, dtype), _run(ref_m, (x,), dy, dtype)
+    # the same 16-bit products with other sums; the reference rounds silu(g), each gradient product and dW too
+    tol = 2e-2 if dtype == torch.bfloat16 else 3e-3
+    for name, a, b in zip(("y", "dx", "dw_gate", "dw_up", "dw_down"), got, ref):
+        assert a.shape == b.shape and a.dtype == b.dtype, name
+        torch.testing.assert_close(a, b, rtol=tol, atol=tol * b.abs().max().item(), msg=name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T, F", [(1, 8), (3, 104), (129, 2048)])
+def test_swiglu_matches_float64(T, F, dtype):
+    from nanonemo_amd.kernels.hip import lib
+    from nanonemo_amd.kernels.hip.layers import _DTYPES
+
+    g = torch.Generator(device="cuda").manual_seed(T + F)
+    gu = (4 * torch.randn(T, 2 * F, device="cuda", generator=g)).to(dtype)
+    edge = torch.tensor([0.0, -0.0, 60.0, -60.0, -1000.0, 1000.0, float("inf"), float("nan")], device="cuda").to(dtype)
+    gu[-1, :8] = edge
+    dh = torch.randn(T, F, device="cuda", generator=g).to(dtype)
+    h, dgu = torch.empty_like(dh), torch.empty_like(gu)
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib().nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F, _DTYPES[dtype], st) == 0
+    assert lib().nn_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), T, F, _DTYPES[dtype], st) == 0
+    x = gu.double().requires_grad_()
+    ref = torch.nn.functional.silu(x[:, :F]) * x[:, F:]
+    (rg,) = torch.autograd.grad(ref, x, dh.double())
+    # one rounding to the 16-bit type (2^-9 / 2^-12 relative, subnormals below), and a few fp32 ones
+    eps, tiny = (2.0**-8, 1e-37) if dtype == torch.bfloat16 else (2.0**-11, 2.0**-24)
+    big = torch.finfo(dtype).max
+    for a, b in ((h, ref.detach()), (dgu, rg)):
+        ok = b.isfinite() & (b.abs() < big)
+        # silu'(g) cancels near its zero at g = -1.28: its fp32 error is a few 2^-24 of 1
+        assert ((a.double() - b)[ok].abs() <= eps * b[ok].abs() + tiny + 1e-6).all()
+        assert torch.equal(a.isnan(), b.isnan())
