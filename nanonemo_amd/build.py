@@ -3,8 +3,7 @@
 Replaces the reference's JIT build (/root/reference/nanonemo/kernels/cuda/__init__.py:15-18, which runs
 nvcc through torch.utils.cpp_extension.load on first use): here ``hipcc`` compiles
 ``nanonemo_amd/csrc/*.hip`` once, in-tree, into ``nanonemo_amd/lib/libnanonemo_fa.so``, a plain C-ABI
-shared library with no torch types in its signatures (include/nanonemo_fa.h, include/nanonemo_rope.h, include/nanonemo_rmsnorm.h). The library is loaded
-with ctypes (nanonemo_amd/kernels/hip/__init__.py), so the same .so runs on any box with the ROCm
+shared library with no torch types in its signatures (include/*.h). The library is loaded with ctypes (nanonemo_amd/kernels/hip/__init__.py), so the same .so runs on any box with the ROCm
 runtime.
 
     python -m nanonemo_amd.build
@@ -16,11 +15,13 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 ROOT = PKG.parent
-SRCS = [PKG / "csrc" / f"{n}.hip" for n in ("flash_attn", "rope", "rmsnorm", "linear")]
+SRCS = [PKG / "csrc" / f"{n}.hip" for n in ("flash_attn", "rope", "rmsnorm", "linear", "loss")]
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libnanonemo_fa.so"
 # Block timelines for `bench.py --timeline`: the attention kernels built with NN_TIMELINE=1, so that every block
@@ -36,16 +37,11 @@ HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
     "-std=c++17",
-    "-shared",
     "-fPIC",
     "-Xclang",
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
-    # Device code never relies on NaN semantics (masked scores are -inf, never NaN); without this
-    # every fmaxf of an MFMA result is preceded by a canonicalising v_max_f32 x, x.
-    "-Xarch_device",
-    "-fno-honor-nans",
     # Select MFMAs in their VGPR form and let register allocation move accumulators to AGPRs where it
     # must: the dK / dV kernel then keeps dK^T / dV^T in AGPRs while S and dP stay in VGPRs, where
     # the softmax reads them, instead of copying every S / dP element out of an AGPR (2-3 % faster;
@@ -57,6 +53,11 @@ HIPCC_FLAGS = [
     "-mllvm",
     "-amdgpu-kernarg-preload-count=16",
 ]
+# Device code never relies on NaN semantics (masked scores are -inf, never NaN), except the cross entropy's, which
+# must show NaN and infinite logits; without this every fmaxf of an MFMA result is preceded by a canonicalising
+# v_max_f32 x, x.
+NO_NANS = ["-Xarch_device", "-fno-honor-nans"]
+HONOR_NANS = {"loss"}
 
 
 def hipcc() -> str:
@@ -66,40 +67,38 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found (looked at $HIPCC, /opt/rocm/bin/hipcc and PATH)")
 
 
-def _start(srcs: list[Path], lib: Path, verbose: bool, defines: tuple[str, ...] = ()):
-    LIB_DIR.mkdir(parents=True, exist_ok=True)
-    tmp = lib.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, *defines, f"-I{ROOT / 'include'}", "-o", str(tmp), *(str(s) for s in srcs)]
+def _run(cmd: list[str], verbose: bool) -> None:
+    """One hipcc command; raises with its output if it fails."""
     if verbose:
         print(" ".join(cmd), flush=True)
-    return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True), tmp, lib
-
-
-def _finish(job, verbose: bool) -> Path:
-    proc, tmp, lib = job
-    out, _ = proc.communicate()
+    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     noise = "'-packed-fp32-ops' is not a recognized feature"
-    log = "\n".join(l for l in out.splitlines() if noise not in l)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed for {lib.name} ({proc.returncode}):\n{log}")
+    log = "\n".join(l for l in p.stdout.splitlines() if noise not in l)
+    if p.returncode != 0:
+        raise RuntimeError(f"hipcc failed ({p.returncode}): {' '.join(cmd)}\n{log}")
     if verbose and log.strip():
         print(log, flush=True)
-    os.replace(tmp, lib)  # atomic: a process that already mapped the old file keeps it
-    return lib
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile the HIP library and the timeline build of the attention kernels, in parallel (always
+    """Compile the HIP library and the timeline build of the attention kernels, every source in parallel (always
     recompiles); return the library's path."""
-    jobs = [_start(SRCS, LIB, verbose), _start(TIMELINE_SRCS, TIMELINE_LIB, verbose, ("-DNN_TIMELINE=1",))]
-    errors = []
-    for job in jobs:
-        try:
-            _finish(job, verbose)
-        except RuntimeError as e:
-            errors.append(str(e))
-    if errors:
-        raise RuntimeError("\n".join(errors))
+    LIB_DIR.mkdir(parents=True, exist_ok=True)
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor() as pool:
+        jobs = []
+        for lib, srcs, defines in ((LIB, SRCS, []), (TIMELINE_LIB, TIMELINE_SRCS, ["-DNN_TIMELINE=1"])):
+            for src in srcs:
+                obj = str(Path(tmp) / f"{lib.stem}_{src.stem}.o")
+                flags = [*HIPCC_FLAGS, *([] if src.stem in HONOR_NANS else NO_NANS), *defines]
+                cmd = [hipcc(), "-c", *flags, f"-I{ROOT / 'include'}", "-o", obj, str(src)]
+                jobs.append((lib, obj, pool.submit(_run, cmd, verbose)))
+        errors = [str(e) for e in (job.exception() for _, _, job in jobs) if e]
+        if errors:
+            raise RuntimeError("\n".join(errors))
+        for lib in (LIB, TIMELINE_LIB):
+            out = lib.with_suffix(".so.tmp")
+            _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-o", str(out), *(obj for to, obj, _ in jobs if to == lib)], verbose)
+            os.replace(out, lib)  # atomic: a process that already mapped the old file keeps it
     return LIB
 
 

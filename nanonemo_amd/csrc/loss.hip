@@ -1,0 +1,235 @@
+// Cross entropy of a large vocabulary for MI355X (gfx950), forward and backward.
+//
+// A row of logits (50304 bf16 values, 100 KB) is read once by the forward, which keeps only the row's logsumexp, and
+// once by the backward, which writes the gradient in the logits' own type. PyTorch's cross entropy on .float() logits
+// writes and reads an fp32 copy, its log-softmax and their gradients: 11.5 GB for 8192 rows where 2.5 GB will do.
+// HBM-bound. Measured at 8192 x 50304 bf16: forward 148 us (5.6 TB/s), backward 327 us (5.0 TB/s, a device
+// copy's rate); the passes they replace take 3.2 ms.
+// Built with NaN semantics (unlike the other kernels): a NaN or infinite logit reaches the loss and the gradient as in
+// PyTorch.
+#include <hip/hip_runtime.h>
+#include <stdarg.h>
+#include <stdint.h>
+#include <stdio.h>
+
+#include <string>
+#include <type_traits>
+
+#include "nanonemo_loss.h"
+#include "tiles.h"
+
+#define NNLOSS_API extern "C" __attribute__((visibility("default")))
+
+namespace {
+
+constexpr int kF32 = 2;
+constexpr int kThreads = 256;
+constexpr long long kIgnore = -100;
+
+// Logits of type DT in groups of 16 bytes, as fp32.
+template <int DT>
+struct Row {
+    static constexpr int W = DT == kF32 ? 4 : 8;
+    using T = std::conditional_t<DT == kF32, float, u16>;
+    static __device__ float one(T x) {
+        if constexpr (DT == kF32)
+            return x;
+        else
+            return Elem<DT>::to_f32(x);
+    }
+    static __device__ T round(float x) {
+        if constexpr (DT == kF32)
+            return x;
+        else
+            return (T)(Elem<DT>::pack2(x, 0.f) & 0xffffu);
+    }
+    static __device__ void load(const T* p, float* v) {
+        if constexpr (DT == kF32) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = x[e];
+        } else {
+            const u16x8 x = ld8(p);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = Elem<DT>::to_f32(x[e]);
+        }
+    }
+    static __device__ void store(T* p, const float* v) {
+        if constexpr (DT == kF32)
+            *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+        else
+            *reinterpret_cast<u32x4*>(p) = u32x4{Elem<DT>::pack2(v[0], v[1]), Elem<DT>::pack2(v[2], v[3]),
+                                                 Elem<DT>::pack2(v[4], v[5]), Elem<DT>::pack2(v[6], v[7])};
+    }
+    // Values before the row's first 16-byte boundary (rows of an odd vocabulary start anywhere).
+    static __device__ int head(const T* row, int V) { return min(V, (int)((16 - ((uintptr_t)row & 15)) & 15) / (int)sizeof(T)); }
+};
+
+constexpr float kL2e = 1.4426950408889634f;
+// exp(x - m), the difference rounded once; 0 for x = -inf whatever a finite m.
+__device__ inline float exp_diff(float x, float m) { return __builtin_amdgcn_exp2f((x - m) * kL2e); }
+
+struct MaxSum {  // s = sum of exp(x - m); m = -inf, s = 0 when empty
+    float m, s;
+};
+__device__ inline float base_of(float m) { return m == -INFINITY ? 0.f : m; }  // exp(x - base) is 0 where every x is -inf
+__device__ inline MaxSum merge(MaxSum a, MaxSum b) {
+    const float m = fmaxf(a.m, b.m), c = base_of(m);
+    return {m, a.s * exp_diff(a.m, c) + b.s * exp_diff(b.m, c)};
+}
+
+// One block per row. A NaN in the row makes s NaN (fmaxf drops it from m); an infinity makes x - m NaN there.
+template <int DT>
+__global__ __launch_bounds__(kThreads) void ce_fwd_kernel(const void* __restrict__ logits, const long long* __restrict__ targets,
+                                                          float* __restrict__ lse, float* __restrict__ rows, int V) {
+    using R = Row<DT>;
+    using T = typename R::T;
+    const T* row = reinterpret_cast<const T*>(logits) + (size_t)blockIdx.x * V;
+    const int head = R::head(row, V), nv = (V - head) / R::W, tail = head + nv * R::W, tid = threadIdx.x;
+    MaxSum a{-INFINITY, 0.f};
+    auto one = [&](float x) { a = merge(a, MaxSum{x, x == -INFINITY ? 0.f : exp_diff(x, x)}); };
+    if (tid < head) one(R::one(row[tid]));
+    if (tid < V - tail) one(R::one(row[tail + tid]));
+    const T* body = row + head;
+    for (int i = tid; i < nv; i += kThreads) {
+        float v[R::W];
+        R::load(body + (size_t)i * R::W, v);
+        float m = a.m;
+#pragma unroll
+        for (int e = 0; e < R::W; ++e) m = fmaxf(m, v[e]);
+        const float c = base_of(m);
+        float s = a.s * exp_diff(a.m, c);
+#pragma unroll
+        for (int e = 0; e < R::W; ++e) s += exp_diff(v[e], c);
+        a = {m, s};
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) a = merge(a, MaxSum{__shfl_xor(a.m, d), __shfl_xor(a.s, d)});
+    __shared__ MaxSum part[kThreads / 64];
+    if ((tid & 63) == 0) part[tid >> 6] = a;
+    __syncthreads();
+    if (tid == 0) {
+        a = part[0];
+#pragma unroll
+        for (int w = 1; w < kThreads / 64; ++w) a = merge(a, part[w]);
+        const float l = a.m + logf(a.s);
+        const long long t = targets[blockIdx.x];
+        lse[blockIdx.x] = l;
+        rows[blockIdx.x] = t == kIgnore ? 0.f : t >= 0 && t < V ? l - R::one(row[t]) : NAN;
+    }
+}
+
+// loss = sum of the rows' losses / n and inv = 1 / n, n the rows whose target is not -100: one block, fixed order, fp64 sums.
+__global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__ rows, const long long* __restrict__ targets,
+                                                       float* __restrict__ loss, float* __restrict__ inv, int R) {
+    double s = 0.0;
+    int n = 0;
+    for (int i = threadIdx.x; i < R; i += 1024) {
+        s += rows[i];
+        n += targets[i] != kIgnore;
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        s += __shfl_xor(s, d);
+        n += __shfl_xor(n, d);
+    }
+    __shared__ double ps[16];
+    __shared__ int pn[16];
+    if ((threadIdx.x & 63) == 0) {
+        ps[threadIdx.x >> 6] = s;
+        pn[threadIdx.x >> 6] = n;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s = 0.0;
+        n = 0;
+        for (int w = 0; w < 16; ++w) {
+            s += ps[w];
+            n += pn[w];
+        }
+        *loss = (float)(s / n);
+        *inv = (float)(1.0 / n);
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void ce_bwd_kernel(const void* __restrict__ logits, const long long* __restrict__ targets,
+                                                          const float* __restrict__ lse, const float* __restrict__ inv,
+                                                          const float* __restrict__ grad, void* __restrict__ dlogits, int V) {
+    using R = Row<DT>;
+    using T = typename R::T;
+    const size_t off = (size_t)blockIdx.x * V;
+    const T* row = reinterpret_cast<const T*>(logits) + off;
+    T* dst = reinterpret_cast<T*>(dlogits) + off;
+    const long long t = targets[blockIdx.x];
+    const bool counts = t != kIgnore;
+    const float g = counts ? grad[0] * inv[0] : 0.f, l = lse[blockIdx.x];
+    auto of = [&](float x, int j) { return counts ? (exp_diff(x, l) - (j == t ? 1.f : 0.f)) * g : 0.f; };
+    const int head = R::head(row, V), nv = (V - head) / R::W, tail = head + nv * R::W, tid = threadIdx.x;
+    if (tid < head) dst[tid] = R::round(of(R::one(row[tid]), tid));
+    if (tid < V - tail) dst[tail + tid] = R::round(of(R::one(row[tail + tid]), tail + tid));
+    for (int i = tid; i < nv; i += kThreads) {
+        const int j = head + i * R::W;
+        float v[R::W];
+        R::load(row + j, v);
+#pragma unroll
+        for (int e = 0; e < R::W; ++e) v[e] = of(v[e], j + e);
+        R::store(dst + j, v);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// Host side.
+// ------------------------------------------------------------------------------------------
+thread_local std::string g_err;
+
+int fail(const char* what) {
+    g_err = what;
+    return -1;
+}
+
+int launched(const char* what) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        g_err = std::string(what) + " launch failed: " + hipGetErrorString(e);
+        return (int)e;
+    }
+    return 0;
+}
+
+int check_sizes(int64_t R, int64_t V, int dtype, const void* a, const void* b) {
+    g_err.clear();
+    if (R < 1 || V < 1 || R >= ((int64_t)1 << 31) || V >= (1 << 30)) return fail("invalid sizes");
+    if (dtype != kF16 && dtype != kBF16 && dtype != kF32) return fail("dtype must be float16, bfloat16 or float32");
+    if (((uintptr_t)a & 15) || ((uintptr_t)b & 15)) return fail("logits must be 16-byte aligned");
+    return 0;
+}
+
+}  // namespace
+
+NNLOSS_API const char* nn_loss_last_error(void) { return g_err.c_str(); }
+
+NNLOSS_API int nn_cross_entropy_fwd(const void* logits, const int64_t* targets, float* lse, float* rows, float* loss,
+                                    float* inv, int64_t R, int64_t V, int dtype, void* stream) {
+    if (int e = check_sizes(R, V, dtype, logits, logits)) return e;
+    if (!logits || !targets || !lse || !rows || !loss || !inv) return fail("null pointer argument");
+    const hipStream_t st = (hipStream_t)stream;
+    auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)R), dim3(kThreads), 0, st>>>(logits, (const long long*)targets, lse, rows, (int)V);
+        return launched("ce_fwd_kernel");
+    };
+    if (int e = dtype == kBF16 ? go(ce_fwd_kernel<kBF16>) : dtype == kF16 ? go(ce_fwd_kernel<kF16>) : go(ce_fwd_kernel<kF32>)) return e;
+    ce_mean_kernel<<<dim3(1), dim3(1024), 0, st>>>(rows, (const long long*)targets, loss, inv, (int)R);
+    return launched("ce_mean_kernel");
+}
+
+NNLOSS_API int nn_cross_entropy_bwd(const void* logits, const int64_t* targets, const float* lse, const float* inv,
+                                    const float* grad, void* dlogits, int64_t R, int64_t V, int dtype, void* stream) {
+    if (int e = check_sizes(R, V, dtype, logits, dlogits)) return e;
+    if (!logits || !targets || !lse || !inv || !grad || !dlogits) return fail("null pointer argument");
+    auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)R), dim3(kThreads), 0, (hipStream_t)stream>>>(logits, (const long long*)targets, lse, inv, grad, dlogits, (int)V);
+        return launched("ce_bwd_kernel");
+    };
+    return dtype == kBF16 ? go(ce_bwd_kernel<kBF16>) : dtype == kF16 ? go(ce_bwd_kernel<kF16>) : go(ce_bwd_kernel<kF32>);
+}

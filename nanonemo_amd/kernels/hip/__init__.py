@@ -28,7 +28,7 @@ _f32 = ctypes.c_float
 _sz = ctypes.c_size_t
 _i64p = ctypes.POINTER(ctypes.c_int64)
 
-# name -> (restype, argtypes); must match include/nanonemo_fa.h, nanonemo_rope.h, nanonemo_rmsnorm.h and nanonemo_linear.h
+# name -> (restype, argtypes); must match the headers in include/
 SIGNATURES: dict[str, tuple] = {
     "nn_fa_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _f32, _vp]),
     "nn_fa_fwd_strided": (
@@ -102,6 +102,10 @@ SIGNATURES: dict[str, tuple] = {
     "nn_swiglu_fwd": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nn_swiglu_bwd": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _vp]),
     "nn_linear_last_error": (ctypes.c_char_p, []),
+    # include/nanonemo_loss.h
+    "nn_cross_entropy_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
+    "nn_cross_entropy_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
+    "nn_loss_last_error": (ctypes.c_char_p, []),
 }
 
 ABI_VERSION = 11
@@ -199,6 +203,13 @@ def check_linear(rc: int) -> None:
     if rc != 0:
         msg = lib().nn_linear_last_error().decode(errors="replace")
         raise RuntimeError(msg or f"nanonemo_linear call failed with code {rc}")
+
+
+def check_loss(rc: int) -> None:
+    """Raise RuntimeError with the library's message when an nn_cross_entropy_* entry point returns non-zero."""
+    if rc != 0:
+        msg = lib().nn_loss_last_error().decode(errors="replace")
+        raise RuntimeError(msg or f"nanonemo_loss call failed with code {rc}")
 
 
 def check_rmsnorm(rc: int) -> None:

@@ -31,15 +31,16 @@ _DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
 _WGRAD_MOST = 6_000_000
 
 
-def plain(m: nn.Module, x: Tensor, width: int) -> bool:
-    """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width."""
+def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
+    """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width
+    (and of a multiple of 8 outputs, unless odd_rows)."""
     if type(m) is not nn.Linear or m.bias is not None or "forward" in m.__dict__:
         return False
     if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
         return False
     w = m.weight
     return (type(w) is nn.Parameter and w.dtype is torch.float32 and w.device == x.device and w.is_contiguous()
-            and w.shape[1] == width and w.shape[0] % 8 == 0 and width % 8 == 0 and w.data_ptr() % 16 == 0)
+            and w.shape[1] == width and (odd_rows or w.shape[0] % 8 == 0) and width % 8 == 0 and w.data_ptr() % 16 == 0)
 
 
 def eligible(x: Tensor) -> bool:
@@ -59,7 +60,7 @@ def can_project(x: Tensor, *layers: nn.Module) -> bool:
 def wgrad(dy: Tensor, x: Tensor, rows: list[int]) -> list[Tensor]:
     """dy^T x for dy (T, sum(rows)) and x (T, K), 16-bit with unit column strides: fp32, one (rows[i], K) tensor each."""
     (T, N), K = dy.shape, x.shape[1]
-    if N * K > _WGRAD_MOST:
+    if N * K > _WGRAD_MOST or N % 8:
         dw = torch.mm(dy.t(), x, out_dtype=torch.float32)
         return [dw] if len(rows) == 1 else [t.contiguous() for t in dw.split(rows)]
     out = [torch.empty((r, K), dtype=torch.float32, device=x.device) for r in rows]

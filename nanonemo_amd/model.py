@@ -276,6 +276,11 @@ class NanoNemo(nn.Module):
         for blk in self.blocks:
             x, delta = blk(x, self.rope_cos, self.rope_sin, delta)
         h = self.norm_out(x, delta)[0]
+        if targets is not None and self.cfg.any_hip and h.is_cuda:
+            from nanonemo_amd.kernels.hip import head
+
+            if head.can_fuse_head(h, self.lm_head, targets):  # both in this build's kernels, as one autograd node
+                return head.head_loss(h, self.lm_head, targets)
         logits = self.lm_head(h)
         loss = None
         if targets is not None:
