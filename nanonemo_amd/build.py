@@ -60,6 +60,29 @@ NO_NANS = ["-Xarch_device", "-fno-honor-nans"]
 HONOR_NANS = {"loss"}
 
 
+# The host side of the operations, a torch extension over the library (g++: it has no device code).
+HOST_SRC = PKG / "csrc" / "host.cpp"
+HOST_LIB = LIB_DIR / "nanonemo_host.so"
+
+
+def _host_command(out: str) -> list[str]:
+    """Compile the host module; it links the library beside it."""
+    import sysconfig
+
+    import torch
+
+    base = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc()).resolve().parents[1]
+    includes = [base / "include", base / "include" / "torch" / "csrc" / "api" / "include", rocm / "include", sysconfig.get_paths()["include"]]
+    libs = ["c10", "c10_hip", "torch", "torch_cpu", "torch_hip", "torch_python"]
+    return [
+        "g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        "-DTORCH_EXTENSION_NAME=nanonemo_host", "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *(a for p in includes for a in ("-isystem", str(p))), f"-I{ROOT / 'include'}", "-o", out, str(HOST_SRC),
+        f"-L{base / 'lib'}", f"-L{LIB_DIR}", "-lnanonemo_fa", *(f"-l{n}" for n in libs), "-Wl,-rpath,$ORIGIN",
+    ]
+
+
 def hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), "/opt/rocm/bin/hipcc", shutil.which("hipcc")):
         if cand and Path(cand).exists():
@@ -68,21 +91,21 @@ def hipcc() -> str:
 
 
 def _run(cmd: list[str], verbose: bool) -> None:
-    """One hipcc command; raises with its output if it fails."""
+    """One compiler command; raises with its output if it fails."""
     if verbose:
         print(" ".join(cmd), flush=True)
     p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     noise = "'-packed-fp32-ops' is not a recognized feature"
     log = "\n".join(l for l in p.stdout.splitlines() if noise not in l)
     if p.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({p.returncode}): {' '.join(cmd)}\n{log}")
+        raise RuntimeError(f"{Path(cmd[0]).name} failed ({p.returncode}): {' '.join(cmd)}\n{log}")
     if verbose and log.strip():
         print(log, flush=True)
 
 
 def build(verbose: bool = False) -> Path:
-    """Compile the HIP library and the timeline build of the attention kernels, every source in parallel (always
-    recompiles); return the library's path."""
+    """Compile the HIP library, the timeline build of the attention kernels and the host module, the HIP sources in
+    parallel (always recompiles); return the library's path."""
     LIB_DIR.mkdir(parents=True, exist_ok=True)
     with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor() as pool:
         jobs = []
@@ -99,6 +122,9 @@ def build(verbose: bool = False) -> Path:
             out = lib.with_suffix(".so.tmp")
             _run([hipcc(), f"--offload-arch={ARCH}", "-shared", "-o", str(out), *(obj for to, obj, _ in jobs if to == lib)], verbose)
             os.replace(out, lib)  # atomic: a process that already mapped the old file keeps it
+    out = HOST_LIB.with_suffix(".so.tmp")
+    _run(_host_command(str(out)), verbose)
+    os.replace(out, HOST_LIB)
     return LIB
 
 

@@ -1,4 +1,7 @@
-"""ctypes binding of the gfx950 HIP library (libnanonemo_fa.so, C ABI in include/nanonemo_fa.h).
+"""Loads the gfx950 HIP library (libnanonemo_fa.so, C ABI in include/) and the host module over it.
+
+The operations run through :func:`host` (csrc/host.cpp, a torch extension: checks, allocation and launches on torch
+tensors); :func:`lib` is the C ABI itself through ctypes, for callers that bring their own buffers.
 
 Replaces the reference's ``build(name)`` (/root/reference/nanonemo/kernels/cuda/__init__.py:15-18), which
 JIT-compiled a pybind11 torch extension. Here the library is built ahead of time by
@@ -16,6 +19,7 @@ from functools import cache
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parents[2] / "lib" / "libnanonemo_fa.so"
+HOST_PATH = LIB_PATH.with_name("nanonemo_host.so")
 
 DTYPE_F16 = 0
 DTYPE_BF16 = 1
@@ -129,6 +133,32 @@ def lib() -> ctypes.CDLL:
     return handle
 
 
+@cache
+def host():
+    """Load nanonemo_host.so once per process; it also registers the CUDA kernels of the torch.library ops."""
+    import importlib.util
+
+    import torch  # noqa: F401  (the module links libtorch)
+
+    lib()  # a missing library or another ABI is reported as such
+    if not HOST_PATH.exists():
+        raise RuntimeError(
+            f"host module {HOST_PATH} is not built; run `python -m nanonemo_amd.build` "
+            "(or __graft_entry__.build()) first. There is no other implementation."
+        )
+    spec = importlib.util.spec_from_file_location("nanonemo_host", HOST_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    return module
+
+
+def preload() -> None:
+    """Load the host module where it is built, so that the ops' CUDA kernels are registered with their schemas; an
+    unbuilt one is an error only when an operation runs."""
+    if HOST_PATH.exists() and LIB_PATH.exists():
+        host()
+
+
 def eager(*ts) -> bool:
     """Whether a public function may run its eager path: a plain autograd.Function around the library call instead
     of its torch.library op. The ops' dispatch (the dispatcher's Python kernel, the autograd.Function that
@@ -139,37 +169,7 @@ def eager(*ts) -> bool:
     take the ops too, whose fake impls and checks handle them."""
     import torch
 
-    if torch.compiler.is_compiling():
-        return False
-    for t in ts:
-        if type(t) is not torch.Tensor or not t.is_cuda:
-            return False
-    # Both queries are PyTorch internals; where this PyTorch lacks one, the ops take every call.
-    transforms = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
-    modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
-    if transforms is None or modes is None:
-        return False
-    return transforms() is None and not modes()
-
-
-def stream_of(t) -> int:
-    """PyTorch's current HIP stream on t's device, as the hipStream_t the library takes (the handle alone, without
-    building a torch.cuda.Stream object where this PyTorch offers that)."""
-    import torch
-
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        return raw(t.device.index)
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
-def on_device(t):
-    """A context that makes t's device current for a launch (a no-op when it already is)."""
-    import contextlib
-
-    import torch
-
-    return contextlib.nullcontext() if t.device.index == torch.cuda.current_device() else torch.cuda.device(t.device)
+    return not torch.compiler.is_compiling() and host().plain_cuda(*ts)
 
 
 def records(*ts) -> bool:
@@ -196,13 +196,6 @@ def check_rope(rc: int) -> None:
     if rc != 0:
         msg = lib().nn_rope_last_error().decode(errors="replace")
         raise RuntimeError(msg or f"nanonemo_rope call failed with code {rc}")
-
-
-def check_linear(rc: int) -> None:
-    """Raise RuntimeError with the library's message when an nn_linear_* entry point returns non-zero."""
-    if rc != 0:
-        msg = lib().nn_linear_last_error().decode(errors="replace")
-        raise RuntimeError(msg or f"nanonemo_linear call failed with code {rc}")
 
 
 def check_loss(rc: int) -> None:

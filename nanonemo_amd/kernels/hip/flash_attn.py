@@ -8,99 +8,27 @@ gradient of lse, :43-54) and the same public ``flash_attn(q, k, v) -> o`` (:57-6
 
 Differences from the reference, all widening: fp16 **and** bf16 inputs (the reference accepts fp16
 only, flash_attn.cu:344-346), and the compute is the HIP library behind a C ABI
-(include/nanonemo_fa.h) called through ctypes on PyTorch's current HIP stream. Every output and the
-backward workspace is allocated here by PyTorch's caching allocator; the library never allocates,
-synchronises or copies to the host, so both ops can be captured into a HIP graph. In eager mode the public
-functions reach the same launches through a plain autograd.Function instead of the ops' dispatch, which
-halves their host time (see "the eager path" below).
+(include/nanonemo_fa.h) called by the host module (csrc/host.cpp) on PyTorch's current HIP stream. Every
+output and the backward workspace is allocated there by PyTorch's caching allocator; the library never
+allocates, synchronises or copies to the host, so both ops can be captured into a HIP graph. On CUDA tensors
+the ops' kernels are the host module's (the bodies here serve other devices, which they refuse). In eager
+mode the public functions reach the same launches through a plain autograd.Function instead of the ops'
+dispatch (see "the eager path" below).
 """
 
 from __future__ import annotations
-
-import ctypes
-import math
 
 import torch
 from torch import Tensor
 from torch.autograd.function import once_differentiable
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check, lib, strides3
 from nanonemo_amd.kernels.hip import eager as _eager
-from nanonemo_amd.kernels.hip import on_device as _on
+from nanonemo_amd.kernels.hip import host, preload
 from nanonemo_amd.kernels.hip import records as _records
-from nanonemo_amd.kernels.hip import stream_of as _stream
-
-_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
-
-
-def _check_inputs(q: Tensor, k: Tensor, v: Tensor, seq_dim: int = 2) -> None:
-    """The reference's check_inputs (flash_attn.cu:342-356) with the dtype set widened to {fp16, bf16}.
-
-    ``seq_dim`` is 2 for the reference's (B, heads, T, hd) tensors and 1 for the (B, T, heads, hd)
-    tensors of the layout-fused ops; the head dimension is the other one of dims 1 and 2."""
-    head_dim_idx = 3 - seq_dim
-    if not (q.is_cuda and k.is_cuda and v.is_cuda):
-        raise RuntimeError("inputs must be CUDA tensors")
-    if q.dtype not in _DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
-        raise RuntimeError("inputs must be float16 or bfloat16 (all the same dtype)")
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise RuntimeError("expected (B, H, T, hd) / (B, KVH, T, hd)")
-    if q.size(0) != k.size(0) or q.size(seq_dim) != k.size(seq_dim) or k.shape != v.shape:
-        raise RuntimeError("K and V must share shape; Q must share batch and length")
-    if q.size(3) != k.size(3):
-        raise RuntimeError("Q and K must share head_dim")
-    if q.size(3) not in (32, 64):
-        raise RuntimeError("head_dim must be 32 or 64")
-    if k.size(head_dim_idx) == 0 or q.size(head_dim_idx) % k.size(head_dim_idx) != 0:
-        raise RuntimeError("query heads must group evenly over KV heads")
-    if q.device != k.device or q.device != v.device:
-        raise RuntimeError("inputs must be on the same device")
-    for t in (q, k, v):
-        if t.numel() and t.data_ptr() % 16 != 0:
-            raise RuntimeError("inputs must be 16-byte aligned")
 
 
 def _contig(t: Tensor) -> Tensor:
     return t if t.is_contiguous() else t.contiguous()
-
-
-def _strides(t: Tensor) -> tuple[int, int, int] | None:
-    """The {batch, head, row} element strides through which the kernels can read the (B, heads, T, hd) tensor t in
-    place, or None: unit hd stride, the others positive multiples of 8 elements (16-byte rows) with rows at least hd
-    apart and within the library's 32-bit row offsets, and a 16-byte aligned start. A dimension of size 1 has no
-    stride of its own; the dense one stands for it."""
-    B, H, T, D = t.shape
-    sb, sh, st, sd = t.stride()
-    st = st if T > 1 else D
-    sh = sh if H > 1 else T * st
-    sb = sb if B > 1 else H * sh
-    if sd != 1 or st < D or st % 8 or sh <= 0 or sh % 8 or sb <= 0 or sb % 8 or T * st >= 1 << 30 or t.data_ptr() % 16:
-        return None
-    return (sb, sh, st) if sb < 1 << 40 and sh * H < 1 << 40 else None
-
-
-def _in_place(*ts: Tensor) -> bool:
-    """Whether the library can read these (B, heads, T, hd) tensors in place, through strides they share (as
-    nn_fa_*_views takes k and v, and q and dO)."""
-    found = {_strides(t) for t in ts}
-    return None not in found and len(found) == 1
-
-
-def _readable(*ts: Tensor) -> tuple[Tensor, ...]:
-    """The tensors themselves where the library can read them in place together, else contiguous copies."""
-    if all(t.is_contiguous() for t in ts) or (all(t.dim() == 4 and t.numel() for t in ts) and _in_place(*ts)):
-        return ts
-    return tuple(t.contiguous() for t in ts)
-
-
-def _stride_array(*ts: Tensor) -> ctypes.Array:
-    """The strides argument of nn_fa_*_views, for tensors that are contiguous or that _readable left in place."""
-
-    def of(t: Tensor) -> tuple[int, int, int]:
-        _, H, T, D = t.shape
-        return (H * T * D, T * D, D) if t.is_contiguous() else _strides(t)
-
-    return (ctypes.c_int64 * (3 * len(ts)))(*(x for t in ts for x in of(t)))
 
 
 _CAPTURE_MSG = (
@@ -118,9 +46,9 @@ def _refuse_capture_with_autograd(where: str, *inputs: Tensor) -> None:
     while torch.compile traces (the check is a host query, and no capture runs at trace time)."""
     # A capture needs PyTorch's initialised HIP state: is_initialized is a flag read, where the capture query is a
     # runtime call, and this runs on every op call.
-    if not torch.cuda.is_initialized():
-        return
     if inputs and not (torch.is_grad_enabled() and any(t.requires_grad for t in inputs)):
+        return
+    if not torch.cuda.is_initialized():
         return
     if torch.compiler.is_compiling() or not torch.cuda.is_current_stream_capturing():
         return
@@ -134,47 +62,9 @@ def _refuse_capture_from_autograd_engine(where: str) -> None:
         _refuse_capture_with_autograd(where)
 
 
-def _launch_fwd(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
-    """Allocates (o, lse), contiguous, and launches the forward on checked inputs the library can read (_readable)."""
-    B, H, T, D = q.shape
-    dense = q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
-    o = torch.empty_like(q) if dense else torch.empty_like(q, memory_format=torch.contiguous_format)
-    lse = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
-    if B == 0 or T == 0 or H == 0:
-        return o, lse
-    ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr())
-    with _on(q):
-        if dense:
-            rc = lib().nn_fa_fwd(*ptrs, B, H, k.size(1), T, D, _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q))
-        else:
-            rc = lib().nn_fa_fwd_views(
-                *ptrs, B, H, k.size(1), T, D, _stride_array(q, k, o), _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q)
-            )
-    check(rc)
-    return o, lse
-
-
-def _prep(q: Tensor, k: Tensor, v: Tensor, seq_dim: int = 2) -> tuple[Tensor, Tensor, Tensor]:
-    """The forward's inputs as the launch takes them, checked: contiguous copies where needed. The (B, heads, T, hd)
-    forward reads strided views in place where it can: for a model that transposes its (B, T, heads, hd)
-    projections the three copies were 20 % of its forward + backward (B=32, T=1024, with the copy of d_o)."""
-    if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
-        if seq_dim == 2:
-            (q,), (k, v) = _readable(q), _readable(k, v)
-        else:
-            q, k, v = _contig(q), _contig(k), _contig(v)
-    _check_inputs(q, k, v, seq_dim)
-    return q, k, v
-
-
-def _fwd(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
-    """The forward on any strides: (o, lse)."""
-    return _launch_fwd(*_prep(q, k, v))
-
-
 @torch.library.custom_op("nanonemo::flash_attn", mutates_args=())
 def _flash_attn(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
-    return _fwd(q, k, v)
+    return host().fa_fwd(q, k, v)
 
 
 @_flash_attn.register_fake
@@ -186,47 +76,10 @@ def _(q, k, v):
     )
 
 
-def _launch_bwd(d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    """Allocates (dq, dk, dv), contiguous, and the workspace and launches the backward on checked inputs. q and d_o, and
-    k and v, are read in place where the library can (_readable); o and lse are contiguous."""
-    dense = q.is_contiguous() and d_o.is_contiguous() and k.is_contiguous() and v.is_contiguous()
-    if not dense:
-        (q, d_o), (k, v) = _readable(q, d_o), _readable(k, v)
-    B, H, T, D = q.shape
-    KVH = k.size(1)
-    if dense:
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    else:
-        dq, dk, dv = (torch.empty_like(t, memory_format=torch.contiguous_format) for t in (q, k, v))
-    if B == 0 or T == 0 or H == 0:
-        return dq, dk, dv
-    L = lib()
-    ws_bytes = L.nn_fa_bwd_workspace_size(B, H, KVH, T, D)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    args = (d_o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws_bytes, B, H, KVH, T, D)
-    with _on(q):
-        if dense:
-            rc = L.nn_fa_bwd(*args, _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q))
-        else:
-            rc = L.nn_fa_bwd_views(
-                *args, _stride_array(q, k, o, dq, dk), _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q)
-            )
-    check(rc)
-    return dq, dk, dv
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bwd", mutates_args=())
 def _flash_attn_bwd(d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     _refuse_capture_from_autograd_engine("flash_attn backward op")
-    o, lse = _contig(o), _contig(lse)
-    _check_inputs(q, k, v)
-    if d_o.shape != q.shape or d_o.dtype != q.dtype or o.shape != q.shape or o.dtype != q.dtype:
-        raise RuntimeError("d_o must be a contiguous float16/bfloat16 tensor shaped like q")
-    B, H, T, D = q.shape
-    if lse.shape != (B, H, T) or lse.dtype != torch.float32:
-        raise RuntimeError("lse must be a float32 tensor of shape (B, H, T)")
-    return _launch_bwd(d_o, q, k, v, o, lse)
+    return host().fa_bwd_op(d_o, q, k, v, o, lse)
 
 
 @_flash_attn_bwd.register_fake
@@ -272,8 +125,9 @@ _flash_attn.register_autograd(_backward, setup_context=_setup_context)
 class _FlashAttnFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v):
-        q, k, v = _prep(q, k, v)
-        o, lse = _launch_fwd(q, k, v)
+        if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):  # copies the backward would make again
+            (q,), (k, v) = host().readable(q), host().readable(k, v)
+        o, lse = host().fa_fwd(q, k, v)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.set_materialize_grads(False)
         return o
@@ -283,14 +137,14 @@ class _FlashAttnFn(torch.autograd.Function):
     def backward(ctx, d_o):
         _refuse_capture_with_autograd("flash_attn backward")
         q, k, v, o, lse = ctx.saved_tensors
-        return _launch_bwd(_d_out(d_o, o), q, k, v, o, lse)
+        return host().fa_bwd(_d_out(d_o, o), q, k, v, o, lse)
 
 
 def flash_attn(q: Tensor, k: Tensor, v: Tensor) -> Tensor:
     """Causal GQA attention. q: (B, H, T, hd), k/v: (B, KVH, T, hd), fp16 or bf16, H % KVH == 0, hd in {32, 64}."""
     _refuse_capture_with_autograd("flash_attn", q, k, v)
     if _eager(q, k, v):
-        return _FlashAttnFn.apply(q, k, v) if _records(q, k, v) else _fwd(q, k, v)[0]
+        return _FlashAttnFn.apply(q, k, v) if _records(q, k, v) else host().fa_fwd(q, k, v)[0]
     o, _ = _flash_attn(q, k, v)
     return o
 
@@ -306,31 +160,9 @@ def flash_attn(q: Tensor, k: Tensor, v: Tensor) -> Tensor:
 # lse stays (B, H, T). Not in the reference: an addition that the same model code can select.
 
 
-def _bthd_strides(t: Tensor) -> ctypes.Array:
-    B, T, Hh, D = t.shape
-    return strides3(T * Hh * D, D, Hh * D)
-
-
-def _launch_fwd_bthd(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
-    """Allocates (o, lse) and launches the projection-layout forward on contiguous, checked inputs."""
-    B, T, H, D = q.shape
-    o = torch.empty_like(q)
-    lse = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
-    if B == 0 or T == 0 or H == 0:
-        return o, lse
-    with _on(q):
-        rc = lib().nn_fa_fwd_strided(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-            B, H, k.size(2), T, D, _bthd_strides(q), _bthd_strides(k), _DTYPES[q.dtype], 1.0 / math.sqrt(D),
-            _stream(q),
-        )
-    check(rc)
-    return o, lse
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bthd", mutates_args=())
 def _flash_attn_bthd(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
-    return _launch_fwd_bthd(*_prep(q, k, v, seq_dim=1))
+    return host().bthd_fwd(q, k, v)
 
 
 @_flash_attn_bthd.register_fake
@@ -342,40 +174,12 @@ def _(q, k, v):
     )
 
 
-def _launch_bwd_bthd(d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    """Allocates (dq, dk, dv) and the workspace and launches the projection-layout backward on contiguous, checked
-    inputs."""
-    B, T, H, D = q.shape
-    KVH = k.size(2)
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    if B == 0 or T == 0 or H == 0:
-        return dq, dk, dv
-    L = lib()
-    ws_bytes = L.nn_fa_bwd_workspace_size(B, H, KVH, T, D)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    with _on(q):
-        rc = L.nn_fa_bwd_strided(
-            d_o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws_bytes,
-            B, H, KVH, T, D, _bthd_strides(q), _bthd_strides(k), _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q),
-        )
-    check(rc)
-    return dq, dk, dv
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bthd_bwd", mutates_args=())
 def _flash_attn_bthd_bwd(
     d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor
 ) -> tuple[Tensor, Tensor, Tensor]:
     _refuse_capture_from_autograd_engine("flash_attn_bthd backward op")
-    d_o, q, k, v, o, lse = (_contig(t) for t in (d_o, q, k, v, o, lse))
-    _check_inputs(q, k, v, seq_dim=1)
-    if d_o.shape != q.shape or d_o.dtype != q.dtype or o.shape != q.shape or o.dtype != q.dtype:
-        raise RuntimeError("d_o must be a contiguous float16/bfloat16 tensor shaped like q")
-    B, T, H, D = q.shape
-    if lse.shape != (B, H, T) or lse.dtype != torch.float32:
-        raise RuntimeError("lse must be a float32 tensor of shape (B, H, T)")
-    return _launch_bwd_bthd(d_o, q, k, v, o, lse)
+    return host().bthd_bwd_op(d_o, q, k, v, o, lse)
 
 
 @_flash_attn_bthd_bwd.register_fake
@@ -397,8 +201,8 @@ class _FlashAttnBthdFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v):
-        q, k, v = _prep(q, k, v, seq_dim=1)
-        o, lse = _launch_fwd_bthd(q, k, v)
+        q, k, v = _contig(q), _contig(k), _contig(v)
+        o, lse = host().bthd_fwd(q, k, v)
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.set_materialize_grads(False)
         return o
@@ -408,7 +212,7 @@ class _FlashAttnBthdFn(torch.autograd.Function):
     def backward(ctx, d_o):
         _refuse_capture_with_autograd("flash_attn_bthd backward")
         q, k, v, o, lse = ctx.saved_tensors
-        return _launch_bwd_bthd(_contig(_d_out(d_o, o)), q, k, v, o, lse)
+        return host().bthd_bwd(_d_out(d_o, o), q, k, v, o, lse)
 
 
 def flash_attn_bthd(q: Tensor, k: Tensor, v: Tensor) -> Tensor:
@@ -417,7 +221,7 @@ def flash_attn_bthd(q: Tensor, k: Tensor, v: Tensor) -> Tensor:
     if _eager(q, k, v):
         if _records(q, k, v):
             return _FlashAttnBthdFn.apply(q, k, v)
-        return _launch_fwd_bthd(*_prep(q, k, v, seq_dim=1))[0]
+        return host().bthd_fwd(q, k, v)[0]
     o, _ = _flash_attn_bthd(q, k, v)
     return o
 
@@ -443,33 +247,11 @@ def _check_tables(cos: Tensor, sin: Tensor, T: int, D: int, device: torch.device
     return _contig(cos), _contig(sin)
 
 
-def _prep_rope(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, ...]:
-    """Contiguous copies where needed and the checks of the RoPE-fused forward's inputs."""
-    q, k, v = _prep(q, k, v, seq_dim=1)
-    cos, sin = _check_tables(cos, sin, q.size(1), q.size(3), q.device)
-    return q, k, v, cos, sin
-
-
-def _launch_fwd_rope(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    """Allocates (o, lse, q_rot) and launches the RoPE-fused forward on contiguous, checked inputs."""
-    B, T, H, D = q.shape
-    o, q_rot = torch.empty_like(q), torch.empty_like(q)
-    lse = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
-    if B == 0 or T == 0 or H == 0:
-        return o, lse, q_rot
-    with _on(q):
-        rc = lib().nn_fa_fwd_rope_strided(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), q_rot.data_ptr(),
-            cos.data_ptr(), sin.data_ptr(), cos.shape[0], B, H, k.size(2), T, D, _bthd_strides(q), _bthd_strides(k),
-            _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream(q),
-        )
-    check(rc)
-    return o, lse, q_rot
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bthd_rope", mutates_args=())
 def _flash_attn_bthd_rope(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    return _launch_fwd_rope(*_prep_rope(q, k, v, cos, sin))
+    if q.is_cuda:
+        cos, sin = _check_tables(cos, sin, q.size(1), q.size(3), q.device)
+    return host().bthd_rope_fwd(q, k, v, cos, sin)
 
 
 @_flash_attn_bthd_rope.register_fake
@@ -482,44 +264,12 @@ def _(q, k, v, cos, sin):
     )
 
 
-def _launch_bwd_rope(
-    d_o: Tensor, q_rot: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, cos: Tensor, sin: Tensor
-) -> tuple[Tensor, Tensor, Tensor]:
-    """Allocates (dq of the unrotated q, dk, dv) and the workspace and launches the RoPE-fused backward on
-    contiguous, checked inputs."""
-    B, T, H, D = q_rot.shape
-    KVH = k.size(2)
-    dq, dk, dv = torch.empty_like(q_rot), torch.empty_like(k), torch.empty_like(v)
-    if B == 0 or T == 0 or H == 0:
-        return dq, dk, dv
-    L = lib()
-    ws_bytes = L.nn_fa_bwd_workspace_size(B, H, KVH, T, D)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q_rot.device)
-    with _on(q_rot):
-        rc = L.nn_fa_bwd_rope_strided(
-            d_o.data_ptr(), q_rot.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws_bytes, cos.data_ptr(), sin.data_ptr(),
-            cos.shape[0], B, H, KVH, T, D, _bthd_strides(q_rot), _bthd_strides(k), _DTYPES[q_rot.dtype],
-            1.0 / math.sqrt(D), _stream(q_rot),
-        )
-    check(rc)
-    return dq, dk, dv
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bthd_rope_bwd", mutates_args=())
 def _flash_attn_bthd_rope_bwd(
     d_o: Tensor, q_rot: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, cos: Tensor, sin: Tensor
 ) -> tuple[Tensor, Tensor, Tensor]:
     _refuse_capture_from_autograd_engine("flash_attn_bthd_rope backward op")
-    d_o, q_rot, k, v, o, lse = (_contig(t) for t in (d_o, q_rot, k, v, o, lse))
-    _check_inputs(q_rot, k, v, seq_dim=1)
-    if d_o.shape != q_rot.shape or d_o.dtype != q_rot.dtype or o.shape != q_rot.shape or o.dtype != q_rot.dtype:
-        raise RuntimeError("d_o must be a contiguous float16/bfloat16 tensor shaped like q")
-    B, T, H, D = q_rot.shape
-    if lse.shape != (B, H, T) or lse.dtype != torch.float32:
-        raise RuntimeError("lse must be a float32 tensor of shape (B, H, T)")
-    cos, sin = _check_tables(cos, sin, T, D, q_rot.device)
-    return _launch_bwd_rope(d_o, q_rot, k, v, o, lse, cos, sin)
+    return host().bthd_rope_bwd_op(d_o, q_rot, k, v, o, lse, cos, sin)
 
 
 @_flash_attn_bthd_rope_bwd.register_fake
@@ -550,8 +300,8 @@ class _FlashAttnBthdRopeFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, cos, sin):
-        q, k, v, cos, sin = _prep_rope(q, k, v, cos, sin)
-        o, lse, q_rot = _launch_fwd_rope(q, k, v, cos, sin)
+        k, v = _contig(k), _contig(v)
+        o, lse, q_rot = host().bthd_rope_fwd(q, k, v, cos, sin)
         ctx.save_for_backward(q_rot, k, v, o, lse, cos, sin)
         ctx.set_materialize_grads(False)
         return o
@@ -561,7 +311,7 @@ class _FlashAttnBthdRopeFn(torch.autograd.Function):
     def backward(ctx, d_o):
         _refuse_capture_with_autograd("flash_attn_bthd_rope backward")
         q_rot, k, v, o, lse, cos, sin = ctx.saved_tensors
-        dq, dk, dv = _launch_bwd_rope(_contig(_d_out(d_o, o)), q_rot, k, v, o, lse, cos, sin)
+        dq, dk, dv = host().bthd_rope_bwd(_d_out(d_o, o), q_rot, k, v, o, lse, cos, sin)
         return dq, dk, dv, None, None
 
 
@@ -572,6 +322,9 @@ def flash_attn_bthd_rope(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tens
     if _eager(q, k, v, cos, sin):
         if _records(q, k, v, cos, sin):
             return _FlashAttnBthdRopeFn.apply(q, k, v, cos, sin)
-        return _launch_fwd_rope(*_prep_rope(q, k, v, cos, sin))[0]
+        return host().bthd_rope_fwd(q, k, v, cos, sin)[0]
     o, _, _ = _flash_attn_bthd_rope(q, k, v, cos, sin)
     return o
+
+
+preload()

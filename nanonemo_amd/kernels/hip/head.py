@@ -12,10 +12,8 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check_loss, lib, on_device, stream_of
-from nanonemo_amd.kernels.hip.linear import cast_weights, eligible, plain, wgrad
-
-_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
+from nanonemo_amd.kernels.hip import host
+from nanonemo_amd.kernels.hip.linear import eligible, plain
 
 
 def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
@@ -28,13 +26,7 @@ def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
 class _HeadLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, targets):
-        (w16,) = cast_weights(x.dtype, (w,))
-        logits = x @ w16.t()
-        R, V = logits.shape
-        lse, rows, loss, inv = (torch.empty(n, dtype=torch.float32, device=x.device) for n in (R, R, (), ()))
-        with on_device(x):
-            check_loss(lib().nn_cross_entropy_fwd(logits.data_ptr(), targets.data_ptr(), lse.data_ptr(), rows.data_ptr(), loss.data_ptr(),
-                                                  inv.data_ptr(), R, V, _DTYPES[x.dtype], stream_of(x)))
+        logits, loss, w16, lse, inv = host().head_fwd(x, w, targets)
         ctx.save_for_backward(x, w16, w, targets, lse, inv)
         # The caller owns the logits and may change them in place before the backward, which then computes them again
         # from x: an alias that shares their version counter and not their graph, instead of a saved output, whose
@@ -50,20 +42,8 @@ class _HeadLoss(torch.autograd.Function):
         need_x, need_w, _ = ctx.needs_input_grad
         if torch.is_grad_enabled():
             return _replayed(x, w, targets, (need_x, need_w), dlogits, dloss)
-        if dloss is not None:
-            logits = ctx.logits if ctx.logits._version == ctx.version else x @ w16.t()
-            d = torch.empty_like(logits)
-            R, V = logits.shape
-            dloss = dloss.contiguous()
-            with on_device(x):
-                check_loss(lib().nn_cross_entropy_bwd(logits.data_ptr(), targets.data_ptr(), lse.data_ptr(), inv.data_ptr(), dloss.data_ptr(),
-                                                      d.data_ptr(), R, V, _DTYPES[x.dtype], stream_of(x)))
-            dlogits = d if dlogits is None else d.add_(dlogits)
-        if dlogits is None:
-            return None, None, None
-        dx = dlogits @ w16 if need_x else None
-        dw = wgrad(dlogits.contiguous(), x, [w.shape[0]])[0] if need_w else None
-        return dx, dw, None
+        logits = ctx.logits if ctx.logits._version == ctx.version else None
+        return (*host().head_bwd(dlogits, dloss, logits, x, w16, targets, lse, inv, need_x, need_w), None)
 
 
 def _replayed(x, w, targets, need, dlogits, dloss):

@@ -18,19 +18,14 @@ and the package's differentiable functions, so that what those support is what i
 
 from __future__ import annotations
 
-import ctypes
-import math
-
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check, check_linear, check_rope, lib, on_device, stream_of
+from nanonemo_amd.kernels.hip import host
 from nanonemo_amd.kernels.hip.flash_attn import flash_attn_bthd
-from nanonemo_amd.kernels.hip.linear import cast_weights, eligible, plain, wgrad
+from nanonemo_amd.kernels.hip.linear import eligible, plain
 from nanonemo_amd.kernels.hip.rope import rope_qk
-
-_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
 
 
 def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd: int, wq, wk, wv, wo) -> bool:
@@ -49,75 +44,22 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
     return not torch.cuda.is_current_stream_capturing()
 
 
-class _Shape:
-    """Sizes of a call, and the strides of its tensors for the library."""
-
-    def __init__(self, B: int, T: int, H: int, KVH: int, D: int):
-        self.B, self.T, self.H, self.KVH, self.D = B, T, H, KVH, D
-        self.nq, self.nk = H * D, KVH * D
-        n = self.n = self.nq + 2 * self.nk
-        dense, wide = (T * self.nq, D, self.nq), (T * n, D, n)  # {batch, head, row}: q, o and dO; ranges of the buffer
-        self.fwd = (ctypes.c_int64 * 9)(*dense, *wide, *dense)
-        self.bwd = (ctypes.c_int64 * 15)(*dense, *wide, *dense, *wide, *wide)
-        dense_r, wide_r = (dense[0], dense[2], D), (wide[0], wide[2], D)  # {batch, position, head}
-        self.rot = (ctypes.c_int64 * 12)(*wide_r, *dense_r, *wide_r, *wide_r)
-        self.unrot = (ctypes.c_int64 * 12)(*wide_r * 4)
-
-    def ranges(self, buf: Tensor) -> tuple[int, int, int]:
-        """Addresses of the q, k and v ranges of a (B T, n) buffer."""
-        p = buf.data_ptr()
-        return p, p + 2 * self.nq, p + 2 * (self.nq + self.nk)
-
-
 class _AttentionLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, cos, sin, B, T, H, KVH, wq, wk, wv, wo):
-        sh = _Shape(B, T, H, KVH, wq.shape[0] // H)
-        w, wo16 = cast_weights(x.dtype, (wq, wk, wv), (wo,))
-        qkv = x @ w.t()
-        q_rot = torch.empty((B, T, sh.nq), dtype=x.dtype, device=x.device)
-        o = torch.empty_like(q_rot)
-        lse = torch.empty((B, H, T), dtype=torch.float32, device=x.device)
-        L, dt, D = lib(), _DTYPES[x.dtype], sh.D
-        q, k, v = sh.ranges(qkv)
-        with on_device(x):
-            st = stream_of(x)
-            check_rope(L.nn_rope_qk_views(q, q_rot.data_ptr(), k, k, cos.data_ptr(), sin.data_ptr(), B, T, H, KVH, D, sh.rot,
-                                          cos.shape[0], dt, 0, st))
-            check(L.nn_fa_fwd_views(q_rot.data_ptr(), k, v, o.data_ptr(), lse.data_ptr(), B, H, KVH, T, D, sh.fwd, dt,
-                                    1.0 / math.sqrt(D), st))
-        y = o.view(B * T, sh.nq) @ wo16.t()
-        ctx.save_for_backward(x, cos, sin, qkv, q_rot, o, lse, w, wo16, wq, wk, wv, wo)
-        ctx.sh = sh
+        y, qkv, q, o, lse, w, wo16 = host().attention_layer_fwd(x, cos, sin, B, T, H, KVH, wq, wk, wv, wo)
+        ctx.save_for_backward(x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo)
+        ctx.sizes = (B, T, H, KVH)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, cos, sin, qkv, q_rot, o, lse, w, wo16, wq, wk, wv, wo = ctx.saved_tensors
-        sh, need = ctx.sh, ctx.needs_input_grad
-        B, T, H, KVH, D = sh.B, sh.T, sh.H, sh.KVH, sh.D
+        x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo = ctx.saved_tensors
+        need = ctx.needs_input_grad
         if torch.is_grad_enabled():
-            return _replayed(_modular, (x, wq, wk, wv, wo), (need[0], *need[7:]), dy, (cos, sin, B, T, H, KVH), at=7)
-        dy = dy.contiguous()
-        d_o = dy @ wo16
-        dwo = wgrad(dy, o.view(B * T, sh.nq), [wo.shape[0]])[0] if need[10] else None
-        if not (need[0] or any(need[7:10])):
-            return None, None, None, None, None, None, None, None, None, None, dwo
-        dqkv = torch.empty_like(qkv)
-        L, dt = lib(), _DTYPES[x.dtype]
-        ws_bytes = L.nn_fa_bwd_workspace_size(B, H, KVH, T, D)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        _, k, v = sh.ranges(qkv)
-        dq, dk, dv = sh.ranges(dqkv)
-        with on_device(x):
-            st = stream_of(x)
-            check(L.nn_fa_bwd_views(d_o.data_ptr(), q_rot.data_ptr(), k, v, o.data_ptr(), lse.data_ptr(), dq, dk, dv,
-                                    ws.data_ptr(), ws_bytes, B, H, KVH, T, D, sh.bwd, dt, 1.0 / math.sqrt(D), st))
-            check_rope(L.nn_rope_qk_views(dq, dq, dk, dk, cos.data_ptr(), sin.data_ptr(), B, T, H, KVH, D, sh.unrot,
-                                          cos.shape[0], dt, 1, st))
-        dx = dqkv @ w if need[0] else None
-        dws = wgrad(dqkv, x, [sh.nq, sh.nk, sh.nk]) if any(need[7:10]) else [None] * 3
-        return dx, None, None, None, None, None, None, *(g if n else None for g, n in zip(dws, need[7:10])), dwo
+            return _replayed(_modular, (x, wq, wk, wv, wo), (need[0], *need[7:]), dy, (cos, sin, *ctx.sizes), at=7)
+        dx, *dws = host().attention_layer_bwd(dy, x, cos, sin, qkv, q, o, lse, w, wo16, *ctx.sizes, need[0], any(need[7:10]), need[10])
+        return dx, None, None, None, None, None, None, *(g if n else None for g, n in zip(dws, need[7:]))
 
 
 def _modular(x, wq, wk, wv, wo, cos, sin, B, T, H, KVH):
@@ -161,34 +103,18 @@ def can_fuse_mlp(x: Tensor, w_gate, w_up, w_down) -> bool:
 class _MlpLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_gate, w_up, w_down):
-        wgu, wd = cast_weights(x.dtype, (w_gate, w_up), (w_down,))
-        gu = x @ wgu.t()
-        T, F_ = x.shape[0], w_gate.shape[0]
-        h = torch.empty((T, F_), dtype=x.dtype, device=x.device)
-        with on_device(x):
-            check_linear(lib().nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F_, _DTYPES[x.dtype], stream_of(x)))
-        y = h @ wd.t()
-        ctx.save_for_backward(x, gu, h, wgu, wd, w_gate, w_up, w_down)
+        y, gu, h, w, wd = host().mlp_fwd(x, w_gate, w_up, w_down)
+        ctx.save_for_backward(x, gu, h, w, wd, w_gate, w_up, w_down)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, gu, h, wgu, wd, w_gate, w_up, w_down = ctx.saved_tensors
+        x, gu, h, w, wd, w_gate, w_up, w_down = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():
             return _replayed(_modular_mlp, (x, w_gate, w_up, w_down), need, dy, (), at=1)
-        dy = dy.contiguous()
-        dwd = wgrad(dy, h, [w_down.shape[0]])[0] if need[3] else None
-        if not (need[0] or need[1] or need[2]):
-            return None, None, None, dwd
-        dh = dy @ wd
-        dgu = torch.empty_like(gu)
-        T, F_ = h.shape
-        with on_device(x):
-            check_linear(lib().nn_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), T, F_, _DTYPES[x.dtype], stream_of(x)))
-        dx = dgu @ wgu if need[0] else None
-        dwg, dwu = wgrad(dgu, x, [F_, F_]) if need[1] or need[2] else (None, None)
-        return dx, dwg if need[1] else None, dwu if need[2] else None, dwd
+        grads = host().mlp_bwd(dy, x, gu, h, w, wd, need[0], need[1] or need[2], need[3])
+        return tuple(g if n else None for g, n in zip(grads, need))
 
 
 def _modular_mlp(x, w_gate, w_up, w_down):

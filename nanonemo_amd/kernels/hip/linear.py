@@ -16,20 +16,14 @@ itself recorded (create_graph) runs differentiable torch products instead of the
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 from torch import Tensor, nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, check_linear, eager, lib, on_device, stream_of
+from nanonemo_amd.kernels.hip import eager, host
 
-_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
-# Above this many elements of dW the library's product fills the chip by itself and is the faster one (8192 tokens:
-# 2048 x 2048 at 16384 tokens 140 us here against 165 with its cast, 4096 x 4096 334 against 245).
-_WGRAD_MOST = 6_000_000
-
+_DTYPES = (torch.float16, torch.bfloat16)
 
 def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
     """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width
@@ -59,43 +53,7 @@ def can_project(x: Tensor, *layers: nn.Module) -> bool:
 
 def wgrad(dy: Tensor, x: Tensor, rows: list[int]) -> list[Tensor]:
     """dy^T x for dy (T, sum(rows)) and x (T, K), 16-bit with unit column strides: fp32, one (rows[i], K) tensor each."""
-    (T, N), K = dy.shape, x.shape[1]
-    if N * K > _WGRAD_MOST or N % 8:
-        dw = torch.mm(dy.t(), x, out_dtype=torch.float32)
-        return [dw] if len(rows) == 1 else [t.contiguous() for t in dw.split(rows)]
-    out = [torch.empty((r, K), dtype=torch.float32, device=x.device) for r in rows]
-    L, n = lib(), len(rows)
-    ws_bytes = L.nn_linear_wgrad_workspace_size(T, N, K)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-    with on_device(x):
-        rc = L.nn_linear_wgrad(
-            dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), T, N, K, n,
-            (ctypes.c_void_p * n)(*(t.data_ptr() for t in out)), (ctypes.c_int64 * n)(*rows),
-            ws.data_ptr() if ws_bytes else None, ws_bytes, _DTYPES[x.dtype], stream_of(x),
-        )
-    check_linear(rc)
-    return out
-
-
-def cast_weights(dtype: torch.dtype, *groups: tuple[Tensor, ...]) -> list[Tensor]:
-    """Each group of fp32 (N_i, K) weights stacked into one (sum N_i, K) tensor of a 16-bit dtype, in one launch."""
-    ws = [w for group in groups for w in group]
-    out, dst = [], []
-    for group in groups:
-        t = torch.empty((sum(w.shape[0] for w in group), group[0].shape[1]), dtype=dtype, device=group[0].device)
-        at = t.data_ptr()
-        for w in group:
-            dst.append(at)
-            at += 2 * w.numel()
-        out.append(t)
-    n = len(ws)
-    with on_device(ws[0]):
-        rc = lib().nn_linear_cast(
-            n, (ctypes.c_void_p * n)(*(w.data_ptr() for w in ws)), (ctypes.c_void_p * n)(*dst),
-            (ctypes.c_int64 * n)(*(w.numel() for w in ws)), _DTYPES[dtype], stream_of(ws[0]),
-        )
-    check_linear(rc)
-    return out
+    return host().wgrad(dy, x, rows)
 
 
 def stacked(grads: tuple[Tensor | None, ...], rows: list[int], like: Tensor) -> Tensor:
@@ -110,10 +68,9 @@ class _Projections(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, *ws):
-        (w16,) = cast_weights(x.dtype, ws)
+        y, w16 = host().project_fwd(x, ws)
         ctx.save_for_backward(x, w16, *ws)
         ctx.set_materialize_grads(False)
-        y = x @ w16.t()
         return (y,) if len(ws) == 1 else y.split([w.shape[0] for w in ws], dim=1)
 
     @staticmethod

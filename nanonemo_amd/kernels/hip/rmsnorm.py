@@ -18,53 +18,11 @@ import torch
 from torch import Tensor
 from torch.autograd.function import once_differentiable
 
-from nanonemo_amd.kernels.hip import check_rmsnorm, eager, lib, on_device, records, stream_of
-
-_CODES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
-
-
-def _code(dtype: torch.dtype) -> int:
-    if dtype not in _CODES:
-        raise RuntimeError(f"only float32, float16 and bfloat16 are supported, got {dtype}")
-    return _CODES[dtype]
-
-
-
-
-def _fwd_impl(
-    x: Tensor, delta: Tensor | None, weight: Tensor, eps: float, out_dtype: torch.dtype
-) -> tuple[Tensor, Tensor, Tensor]:
-    """Checks, allocates and launches the forward: (y, h, rstd). The body of the op and of the eager path."""
-    if not x.is_cuda:
-        raise RuntimeError("x must be a CUDA tensor")
-    x = x.contiguous()
-    delta = delta.contiguous() if delta is not None else None
-    weight = weight.contiguous()
-    if weight.dtype != torch.float32:
-        raise RuntimeError("weight must be contiguous float32")
-    if delta is not None and delta.shape != x.shape:
-        raise RuntimeError("delta must match x")
-    N = x.size(-1)
-    if weight.numel() != N:
-        raise RuntimeError("weight must have hidden-size elements")
-    M = x.numel() // N if N else 0
-    y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    h = torch.empty(x.shape, dtype=torch.promote_types(x.dtype, delta.dtype), device=x.device) if delta is not None \
-        else x.new_empty(0)
-    rstd = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
-    with on_device(x):
-        rc = lib().nn_add_rmsnorm_fwd(
-            x.data_ptr(), delta.data_ptr() if delta is not None else None, weight.data_ptr(), y.data_ptr(),
-            h.data_ptr() if delta is not None else None, rstd.data_ptr(), M, N, eps, _code(x.dtype),
-            _code(delta.dtype) if delta is not None else 0, _code(out_dtype), stream_of(x),
-        )
-    check_rmsnorm(rc)
-    return y, h, rstd
-
+from nanonemo_amd.kernels.hip import eager, host, preload, records
 
 @torch.library.custom_op("nanonemo::cuda_add_rms_norm_fwd", mutates_args=())
 def _fwd(x: Tensor, delta: Tensor | None, weight: Tensor, eps: float, out_dtype: torch.dtype) -> tuple[Tensor, Tensor, Tensor]:
-    return _fwd_impl(x, delta, weight, eps, out_dtype)
+    return host().norm_fwd(x, delta, weight, eps, out_dtype)
 
 
 @_fwd.register_fake
@@ -73,44 +31,12 @@ def _(x, delta, weight, eps, out_dtype):
     return x.new_empty(x.shape, dtype=out_dtype), h, x.new_empty(x.shape[:-1], dtype=torch.float32)
 
 
-def _bwd_impl(
-    dy: Tensor, dh: Tensor | None, h: Tensor, weight: Tensor, rstd: Tensor,
-    dx_dtype: torch.dtype, ddelta_dtype: torch.dtype | None,
-) -> tuple[Tensor, Tensor, Tensor]:
-    """Checks, allocates and launches the backward: (dx, ddelta, dw). The body of the op and of the eager path."""
-    dy, h, weight, rstd = dy.contiguous(), h.contiguous(), weight.contiguous(), rstd.contiguous()
-    dh = dh.contiguous() if dh is not None else None
-    if dy.shape != h.shape:
-        raise RuntimeError("dy and h must be contiguous, same shape")
-    if (dh is None) != (ddelta_dtype is None):
-        raise RuntimeError("dh and ddelta_dtype go together")
-    if dh is not None and dh.dtype != h.dtype:
-        raise RuntimeError("dh must be contiguous, h's dtype")
-    N = h.size(-1)
-    M = h.numel() // N if N else 0
-    dx = torch.empty(h.shape, dtype=dx_dtype, device=h.device)
-    dd = torch.empty(h.shape, dtype=ddelta_dtype, device=h.device) if dh is not None else h.new_empty(0)
-    dw = torch.empty(N, dtype=torch.float32, device=h.device)
-    L = lib()
-    ws_bytes = L.nn_add_rmsnorm_bwd_workspace_size(M, N)
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=h.device)
-    with on_device(h):
-        rc = L.nn_add_rmsnorm_bwd(
-            dy.data_ptr(), dh.data_ptr() if dh is not None else None, h.data_ptr(), weight.data_ptr(),
-            rstd.data_ptr(), dx.data_ptr(), dd.data_ptr() if dh is not None else None, dw.data_ptr(), ws.data_ptr(),
-            ws_bytes, M, N, _code(dy.dtype), _code(h.dtype), _code(dx_dtype),
-            _code(ddelta_dtype) if ddelta_dtype is not None else 0, stream_of(h),
-        )
-    check_rmsnorm(rc)
-    return dx, dd, dw.to(weight.dtype)
-
-
 @torch.library.custom_op("nanonemo::cuda_add_rms_norm_bwd", mutates_args=())
 def _bwd(
     dy: Tensor, dh: Tensor | None, h: Tensor, weight: Tensor, rstd: Tensor,
     dx_dtype: torch.dtype, ddelta_dtype: torch.dtype | None,
 ) -> tuple[Tensor, Tensor, Tensor]:
-    return _bwd_impl(dy, dh, h, weight, rstd, dx_dtype, ddelta_dtype)
+    return host().norm_bwd(dy, dh, h, weight, rstd, dx_dtype, ddelta_dtype)
 
 
 @_bwd.register_fake
@@ -158,7 +84,7 @@ class _AddRmsNormFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, delta, weight, eps, out_dtype):
-        y, h, rstd = _fwd_impl(x, delta, weight, eps, out_dtype)
+        y, h, rstd = host().norm_fwd(x, delta, weight, eps, out_dtype)
         _save(ctx, x, delta, weight, y, h, rstd)
         if delta is None:
             ctx.mark_non_differentiable(h)
@@ -167,7 +93,7 @@ class _AddRmsNormFn(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, dy, dh):
-        return _grads(ctx, dy, dh, _bwd_impl)
+        return _grads(ctx, dy, dh, host().norm_bwd)
 
 
 def add_rms_norm(x: Tensor, delta: Tensor | None, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
@@ -179,7 +105,10 @@ def add_rms_norm(x: Tensor, delta: Tensor | None, weight: Tensor, eps: float) ->
         if records(*ins):
             y, h = _AddRmsNormFn.apply(x, delta, weight, eps, out_dtype)
         else:
-            y, h, _ = _fwd_impl(x, delta, weight, eps, out_dtype)
+            y, h, _ = host().norm_fwd(x, delta, weight, eps, out_dtype)
     else:
         y, h, _ = _fwd(x, delta, weight, eps, out_dtype)
     return y, (x if delta is None else h)
+
+
+preload()

@@ -17,48 +17,12 @@ import torch
 from torch import Tensor
 from torch.autograd.function import once_differentiable
 
-from nanonemo_amd.kernels.hip import DTYPE_BF16, DTYPE_F16, DTYPE_F32, check_rope, eager, lib, on_device, records
-from nanonemo_amd.kernels.hip import stream_of, strides3
-
-_DTYPES = {torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16, torch.float32: DTYPE_F32}
-
-
-def _prep(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor]:
-    if not (q.is_cuda and k.is_cuda and cos.is_cuda and sin.is_cuda):
-        raise RuntimeError("inputs must be CUDA tensors")
-    if q.dim() != 4 or k.dim() != 4 or q.shape[0] != k.shape[0] or q.shape[1] != k.shape[1] or q.shape[3] != k.shape[3]:
-        raise RuntimeError("expected q (B, T, H, hd) and k (B, T, KVH, hd)")
-    if q.dtype not in _DTYPES or k.dtype != q.dtype:
-        raise RuntimeError("q and k must share a dtype in {float16, bfloat16, float32}")
-    D = q.shape[3]
-    if D % 16:
-        raise RuntimeError("head_dim must be a multiple of 16")
-    if cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape or cos.dim() != 2 \
-            or cos.shape[1] != D // 2 or cos.shape[0] < q.shape[1]:
-        raise RuntimeError("cos/sin must be float32 (T_max >= T, hd/2) tables")
-    q, k = q.contiguous(), k.contiguous()
-    return q, k, cos.contiguous(), sin.contiguous()
-
-
-def _call(fn_name: str, q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor]:
-    B, T, H, D = q.shape
-    KVH = k.shape[2]
-    qo, ko = torch.empty_like(q), torch.empty_like(k)
-    if q.numel() == 0 and k.numel() == 0:
-        return qo, ko
-    with on_device(q):
-        rc = getattr(lib(), fn_name)(
-            q.data_ptr(), qo.data_ptr(), k.data_ptr(), ko.data_ptr(), cos.data_ptr(), sin.data_ptr(),
-            B, T, H, KVH, D, strides3(T * H * D, H * D, D), strides3(T * KVH * D, KVH * D, D), cos.shape[0],
-            _DTYPES[q.dtype], stream_of(q),
-        )
-    check_rope(rc)
-    return qo, ko
+from nanonemo_amd.kernels.hip import eager, host, preload, records
 
 
 @torch.library.custom_op("nanonemo::rope_qk", mutates_args=())
 def _rope_qk(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor]:
-    return _call("nn_rope_qk", *_prep(q, k, cos, sin))
+    return host().rope(q, k, cos, sin, False)
 
 
 @_rope_qk.register_fake
@@ -68,7 +32,7 @@ def _(q, k, cos, sin):
 
 @torch.library.custom_op("nanonemo::rope_qk_bwd", mutates_args=())
 def _rope_qk_bwd(dq: Tensor, dk: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor]:
-    return _call("nn_rope_qk_bwd", *_prep(dq, dk, cos, sin))
+    return host().rope(dq, dk, cos, sin, True)
 
 
 @_rope_qk_bwd.register_fake
@@ -97,13 +61,13 @@ class _RopeQkFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, cos, sin):
         ctx.save_for_backward(cos, sin)
-        return _call("nn_rope_qk", *_prep(q, k, cos, sin))
+        return host().rope(q, k, cos, sin, False)
 
     @staticmethod
     @once_differentiable
     def backward(ctx, dq, dk):
         cos, sin = ctx.saved_tensors
-        gq, gk = _call("nn_rope_qk_bwd", *_prep(dq, dk, cos, sin))
+        gq, gk = host().rope(dq, dk, cos, sin, True)
         return gq, gk, None, None
 
 
@@ -111,7 +75,7 @@ def _rope(q: Tensor, k: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tenso
     if eager(q, k, cos, sin):
         if records(q, k, cos, sin):
             return _RopeQkFn.apply(q, k, cos, sin)
-        return _call("nn_rope_qk", *_prep(q, k, cos, sin))
+        return host().rope(q, k, cos, sin, False)
     return _rope_qk(q, k, cos, sin)
 
 
@@ -124,3 +88,6 @@ def rope_k(k: Tensor, cos: Tensor, sin: Tensor) -> Tensor:
     """Rotate k (B, T, KVH, hd) alone (the q half of the pass is folded into the attention op)."""
     q = k.new_empty(k.shape[0], k.shape[1], 0, k.shape[3])
     return _rope(q, k, cos, sin)[1]
+
+
+preload()

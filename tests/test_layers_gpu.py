@@ -126,8 +126,8 @@ def test_mlp_layer_matches_its_modules(shape, d, ff, dtype):
 @pytest.mark.parametrize("T, F", [(1, 8), (3, 104), (129, 2048)])
 def test_swiglu_matches_float64(T, F, dtype):
     from nanonemo_amd.kernels.hip import lib
-    from nanonemo_amd.kernels.hip.layers import _DTYPES
 
+    code = {torch.float16: 0, torch.bfloat16: 1}[dtype]
     g = torch.Generator(device="cuda").manual_seed(T + F)
     gu = (4 * torch.randn(T, 2 * F, device="cuda", generator=g)).to(dtype)
     edge = torch.tensor([0.0, -0.0, 60.0, -60.0, -1000.0, 1000.0, float("inf"), float("nan")], device="cuda").to(dtype)
@@ -135,8 +135,8 @@ def test_swiglu_matches_float64(T, F, dtype):
     dh = torch.randn(T, F, device="cuda", generator=g).to(dtype)
     h, dgu = torch.empty_like(dh), torch.empty_like(gu)
     st = torch.cuda.current_stream().cuda_stream
-    assert lib().nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F, _DTYPES[dtype], st) == 0
-    assert lib().nn_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), T, F, _DTYPES[dtype], st) == 0
+    assert lib().nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F, code, st) == 0
+    assert lib().nn_swiglu_bwd(dh.data_ptr(), gu.data_ptr(), dgu.data_ptr(), T, F, code, st) == 0
     x = gu.double().requires_grad_()
     ref = torch.nn.functional.silu(x[:, :F]) * x[:, F:]
     (rg,) = torch.autograd.grad(ref, x, dh.double())
