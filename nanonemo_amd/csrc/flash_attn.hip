@@ -604,21 +604,21 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
     // tile nqt - 1 - i / group in its first unit or on tile i / group - 1 in its second, whichever pair it is. The
     // pairs' blocks of one (batch, KV head) run on one XCD and start together, so they ask for the same Q / dO
     // tiles at about the same time and share them in that XCD's L2 (at most two tiles per head in flight).
-    auto iter_head = [&](int itn, int qtf) { (void)qtf; return itn % group; };
-    auto iter_tile = [&](int itn, int qtf) { return qtf == pj ? nqt - 1 - itn / group : qtf + itn / group; };
     // DMA iteration itn into this wave's slot: the Q / dO tiles and the -lse/scale, -D vectors.
     auto issue_it = [&](int itn, int qtf, u16* qs, u16* os, float* ls) {
         // Wave-uniform in fact; made uniform for the compiler only here, so that the tile addressing is
         // scalar without keeping scalar copies alive across the whole kernel.
         const int itu = __builtin_amdgcn_readfirstlane(itn), wu = __builtin_amdgcn_readfirstlane(wave);
         const int bu = __builtin_amdgcn_readfirstlane(b), ku = __builtin_amdgcn_readfirstlane(kvh);
-        const int hq = ku * group + iter_head(itu, qtf);
-        const size_t ro = ((size_t)bu * H + hq) * T;  // first row of the head's [T] vectors
+        const uint32_t iq = (uint32_t)itu / (uint32_t)group, ih = (uint32_t)itu - iq * (uint32_t)group;
+        const uint32_t hq = (uint32_t)(ku * group) + ih;
+        const size_t ro = (uint64_t)((uint32_t)(bu * H) + hq) * (uint32_t)T;  // first row of the head's [T] vectors
         const size_t qo = lq.at(bu, hq);
-        const int q0 = iter_tile(itu, qtf) * BM;
-        dma_rows<HD, BM, 1>(Q + qo, lq.st, q0, T, qs + wu * QT, 0, dfo);
-        dma_rows<HD, BM, 1>(dO + qo, lq.st, q0, T, os + wu * QT, 0, dfo);
-        const uint32_t lo = (uint32_t)min(lane, T - 1 - q0) * 4;  // rows past T repeat row T - 1
+        const uint32_t q0 = (uint32_t)(qtf == pj ? nqt - 1 - (int)iq : qtf + (int)iq) * BM;
+        const uint64_t at = qo + (uint64_t)q0 * (uint32_t)lq.st;
+        dma_tile<HD, BM, 1>(Q + at, lq.st, T - (int)q0, qs + wu * QT, 0, dfo);
+        dma_tile<HD, BM, 1>(dO + at, lq.st, T - (int)q0, os + wu * QT, 0, dfo);
+        const uint32_t lo = (uint32_t)min(lane, T - 1 - (int)q0) * 4;  // rows past T repeat row T - 1
         dma_vec64(nLvec + ro + q0, lo, ls + wu * 2 * BM);
         dma_vec64(nDvec + ro + q0, lo, ls + wu * 2 * BM + BM);
     };
@@ -699,8 +699,14 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
         const int nmine = active && wp < nsp ? (nsp - wp + WPP - 1) / WPP : 0;  // iterations ifirst + wp + WPP j
 
 
-        // Iteration itn -> 64-row query tile.
-        auto qbase_of = [&](int itn) { return iter_tile(itn, qt_first) * BM; };
+        // The unit's iterations on its last `group` and on its first: for the pair's first unit, which walks down,
+        // the last are on the diagonal (tile = unit) and the first on the last tile; for the second unit, up, the
+        // other way round. (A division for the tile itself, in every iteration before its first product, cost a single
+        // in-order wave about 40 instructions of 577; with the operand reads issued before the copies' addresses, and
+        // those in unsigned arithmetic, dK/dV is 2.5-5 % faster at every shape: 32.6 -> 31.7 us at B=8, T=1024, 389.5 ->
+        // 379.7 at T = 8192.)
+        auto at_low = [&](int itn) { return (unsigned)(itn - (unit == pj ? niter - group : 0)) < (unsigned)group; };
+        auto at_high = [&](int itn) { return (unsigned)(itn - (unit == pj ? 0 : niter - group)) < (unsigned)group; };
         auto issue = [&](int itn, u16* qs, u16* os, float* ls) { issue_it(itn, qt_first, qs, os, ls); };
         // Operands of one 32-query step: Q / dO rows (A operands) and -lse/scale, -D as the
         // accumulators' initial values (element i: query 32qh + (i/4)*8 + 4hh + i%4, the same for
@@ -743,11 +749,10 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
         // one, their copy instructions spread over the MFMAs (the CU's copy path accepts them only so
         // fast, and an in-order wave that issued them back to back would stall on it with its MFMA
         // pipe idle).
-        auto compute = [&](auto mask_tag, auto dma_tag, int qbase, const u16* qs, const u16* os, const float* ls,
+        auto compute = [&](auto mask_tag, auto dma_tag, const u16* qs, const u16* os, const float* ls,
                            int nitn, u16* nqs, u16* nos, float* nls) {
             constexpr bool MASK = decltype(mask_tag)::value;
             constexpr bool DMA = decltype(dma_tag)::value;
-            if constexpr (DMA) issue(nitn, nqs, nos, nls);
             const u16* qb_ = qs + wave * QT;
             const u16* ob_ = os + wave * QT;
             const float* lb_ = ls + wave * 2 * BM;
@@ -755,6 +760,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
             ColOps c[2];
             load_rows(0, qb_, ob_, lb_, r[0]);
             load_cols(0, qb_, ob_, c[0]);
+            if constexpr (DMA) issue(nitn, nqs, nos, nls);
 #pragma unroll
             for (int qh = 0; qh < 2; ++qh) {
                 // A masked iteration sits on the diagonal (its query tile is the unit: qbase == kb0), so
@@ -784,8 +790,7 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
                     // keys of every row before T, and their columns are never stored. Rows past T start
                     // from -inf (see below), so their p is 0 too.
                     if (MASK && sl == qh) {
-                        const int key = kb0 + 32 * sl + l32;
-                        const int qlo = key - qbase - 32 * qh - 4 * hh;  // offsets below this: future
+                        const int qlo = 32 * sl + l32 - 32 * qh - 4 * hh;  // offsets below this: future
 #pragma unroll
                         for (int i = 0; i < 16; ++i)
                             s[sl][i] = (i >> 2) * 8 + (i & 3) >= qlo ? s[sl][i] : -INFINITY;
@@ -821,15 +826,15 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
         };
         auto run = [&](auto dma_tag, int itn, const u16* qs, const u16* os, float* ls, int nitn, u16* nqs,
                        u16* nos, float* nls) {
-            const int qbase = qbase_of(itn);
+            const int itu = itn;
             // Rows past T (zero Q and dO rows; their -lse is row T - 1's, which with a zero score could
             // overflow p) start their scores from -inf instead, so their p is 0: patched in this wave's
             // copy of the -lse vector, which has landed.
-            if (qbase + BM > T && lane >= T - qbase) ls[wave * 2 * BM + lane] = -INFINITY;
-            if (kb0 + BNK - 1 > qbase)
-                compute(std::true_type{}, dma_tag, qbase, qs, os, ls, nitn, nqs, nos, nls);
+            if (T % BM != 0 && at_high(itu) && lane >= T % BM) ls[wave * 2 * BM + lane] = -INFINITY;
+            if (at_low(itu))
+                compute(std::true_type{}, dma_tag, qs, os, ls, nitn, nqs, nos, nls);
             else
-                compute(std::false_type{}, dma_tag, qbase, qs, os, ls, nitn, nqs, nos, nls);
+                compute(std::false_type{}, dma_tag, qs, os, ls, nitn, nqs, nos, nls);
         };
         // Double-buffered: this wave's iteration j uses buffer j % 2 while j + 1 streams into the other.
         // The DMA into a buffer is issued only after this wave's own reads of it (iteration j - 1)

@@ -168,15 +168,15 @@ __device__ inline DmaOffs<W, ROWS, NW> dma_offsets(int lane, int wave, int ld) {
 // Buffer resource word 3 for raw (unswizzled, stride 0) buffer access on gfx9-family parts.
 constexpr int kBufWord3 = 0x00020000;
 
-// Copies rows [r0, r0 + ROWS) of a [T][W] global matrix with row stride `ld` elements into a
-// swizzled row-major LDS tile, 16 bytes per lane. `g`, `ld`, `r0`, `T`, `lds` and `wave` are
+// Copies ROWS rows of W columns at g, row stride `ld` elements, into a swizzled row-major LDS tile, 16
+// bytes per lane; `left` rows (at least 1) remain in the matrix. `g`, `ld`, `left`, `lds` and `wave` are
 // wave-uniform, and `fo` holds this lane's offsets for stride `ld` (dma_offsets). The copies are
 // buffer loads: the tile's base and extent live in a scalar buffer descriptor and each lane adds its
-// 32-bit offset, so they cost no per-lane address arithmetic. The descriptor's extent ends at row
-// T - 1, so rows past it read as zeros (their results are masked by the callers). The LDS
+// 32-bit offset, so they cost no per-lane address arithmetic. The descriptor's extent ends at the last
+// row, so rows past it read as zeros (their results are masked by the callers). The LDS
 // destination of a copy is the uniform base + 16 * lane.
 template <int W, int ROWS, int NW>
-__device__ inline void dma_rows(const u16* __restrict__ g, int ld, int r0, int T, u16* lds, int wave,
+__device__ inline void dma_tile(const u16* __restrict__ g, int ld, int left, u16* lds, int wave,
                                 const DmaOffs<W, ROWS, NW>& fo) {
     constexpr int CH = W / 8, NCH = ROWS * CH;
     static_assert(NCH % (64 * NW) == 0 && 64 % CH == 0, "tile must split evenly over the block's waves");
@@ -184,11 +184,11 @@ __device__ inline void dma_rows(const u16* __restrict__ g, int ld, int r0, int T
     const int wu = __builtin_amdgcn_readfirstlane(wave);
     // readfirstlane yields an int: each half goes through uint32_t before widening, or a low word with
     // bit 31 set would sign-extend into the high word.
-    const uint64_t ga = reinterpret_cast<uint64_t>(g + (size_t)r0 * ld);
+    const uint64_t ga = reinterpret_cast<uint64_t>(g);
     const uint32_t ghi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(ga >> 32));
     const uint32_t glo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)ga);
     void* gt = reinterpret_cast<void*>(((uint64_t)ghi << 32) | glo);
-    const int nbytes = __builtin_amdgcn_readfirstlane(min(T - r0, ROWS) * ld * 2);
+    const int nbytes = __builtin_amdgcn_readfirstlane(min(left, ROWS) * ld * 2);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(gt, 0, nbytes, kBufWord3);
 #pragma unroll
     for (int it = 0; it < NCH / (64 * NW); ++it) {
@@ -196,6 +196,12 @@ __device__ inline void dma_rows(const u16* __restrict__ g, int ld, int r0, int T
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_AS(void, lds + k * 64 * 8), 16, fo.o[it], 0, 0, 0);
     }
 #endif
+}
+// The same for rows [r0, r0 + ROWS) of a [T][W] matrix at g.
+template <int W, int ROWS, int NW>
+__device__ inline void dma_rows(const u16* __restrict__ g, int ld, int r0, int T, u16* lds, int wave,
+                                const DmaOffs<W, ROWS, NW>& fo) {
+    dma_tile<W, ROWS, NW>(g + (size_t)r0 * ld, ld, T - r0, lds, wave, fo);
 }
 
 // Wait until this wave's vector-memory operations (including LDS DMA) have completed.
