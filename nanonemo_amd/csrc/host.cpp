@@ -363,7 +363,14 @@ struct Inner {
 // row counts are its too.
 constexpr int64_t kWgradMost = 6000000;
 
-std::vector<Tensor> wgrad(const Tensor& dy, const Tensor& x, const std::vector<int64_t>& rows) {
+// The tensor as the kernel reads it: rows of unit stride, 16-byte aligned (a gradient may arrive as a slice of anything).
+Tensor rows_aligned(const Tensor& t) {
+    const bool ok = t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) && (uintptr_t)t.data_ptr() % 16 == 0;
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+
+std::vector<Tensor> wgrad(const Tensor& dy_, const Tensor& x_, const std::vector<int64_t>& rows) {
+    const Tensor dy = rows_aligned(dy_), x = rows_aligned(x_);
     const int64_t T = dy.size(0), N = dy.size(1), K = x.size(1);
     const c10::DeviceGuard guard(x.device());
     if (N * K > kWgradMost || N % 8) {

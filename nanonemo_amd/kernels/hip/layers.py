@@ -35,6 +35,8 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
     d = x.shape[2]
     if not (plain(wq, x, d) and plain(wk, x, d) and plain(wv, x, d) and plain(wo, x, heads * hd)):
         return False
+    if x.shape[1] * (heads + 2 * kv_heads) * hd >= 1 << 30:  # the library's row offsets within a sequence
+        return False
     if wq.weight.shape[0] != heads * hd or wk.weight.shape[0] != kv_heads * hd or wv.weight.shape[0] != kv_heads * hd:
         return False
     for t in (cos, sin):
@@ -97,7 +99,8 @@ def can_fuse_mlp(x: Tensor, w_gate, w_up, w_down) -> bool:
     if not (plain(w_gate, x, d) and plain(w_up, x, d)):
         return False
     F_ = w_gate.weight.shape[0]
-    return w_up.weight.shape[0] == F_ and plain(w_down, x, F_) and not torch.cuda.is_current_stream_capturing()
+    return (w_up.weight.shape[0] == F_ and plain(w_down, x, F_) and x.numel() // d * F_ < 1 << 33  # the activation kernel's index
+            and not torch.cuda.is_current_stream_capturing())
 
 
 class _MlpLayer(torch.autograd.Function):

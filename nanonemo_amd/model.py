@@ -16,8 +16,12 @@ tied input/output embedding, GPT-2 style init with the residual projections scal
 ``rope_kernel="hip"`` rotates q and k with this build's RoPE kernel (nanonemo::rope_qk), ``rope_kernel="fused"``
 rotates k with it and q inside the layout-fused attention op (nanonemo::flash_attn_bthd_rope), and
 ``norm_kernel="hip"`` runs the residual add + RMSNorm on either side of attention as this build's fused
-kernel (nanonemo::cuda_add_rms_norm_fwd / _bwd, the reference's norm_kernel="cuda"); everything else
-is plain PyTorch.
+kernel (nanonemo::cuda_add_rms_norm_fwd / _bwd, the reference's norm_kernel="cuda").
+
+A model with any of them set also runs its linear layers, SwiGLU and cross entropy on this build's kernels where it is
+called eagerly on a GPU under 16-bit autocast (kernels/hip/linear.py, layers.py and head.py say exactly when; there the
+"hip_bthd" attention with either RoPE kernel is one autograd node, with q rotated by the RoPE kernel, whose result is
+bit-identical). Everything else, and every module whose layers carry hooks or are not plain nn.Linear, is PyTorch.
 """
 
 from __future__ import annotations

@@ -120,3 +120,17 @@ def test_only_untouched_layers_under_autocast_take_the_path():
         with torch.autograd.forward_ad.dual_level():
             assert not linear.can_project(x, _layers(32, (16,))[0])
         assert not linear.can_project(x, nn.Linear(32, 16, bias=False).cuda().bfloat16())
+
+
+@pytest.mark.parametrize("what", ["offset", "row stride", "column stride"])
+def test_wgrad_copies_what_the_kernel_cannot_read(what):
+    from nanonemo_amd.kernels.hip.linear import wgrad
+
+    T, N, K = 130, 64, 40
+    t = torch.randn(2 * T * (N + 4) + 3, device="cuda").bfloat16()
+    dy = {"offset": t[3 : 3 + T * N].view(T, N), "row stride": t[: T * (N + 4)].view(T, N + 4)[:, :N],
+          "column stride": t[: T * N].view(N, T).t()}[what]
+    x = torch.randn(T, K, device="cuda").bfloat16()
+    assert torch.equal(wgrad(dy, x, [N])[0], wgrad(dy.clone(memory_format=torch.contiguous_format), x, [N])[0])
+    (got,), (ref,) = wgrad(x, dy, [K]), wgrad(x, dy.clone(memory_format=torch.contiguous_format), [K])
+    assert torch.equal(got, ref)
