@@ -222,7 +222,7 @@ class MLP(nn.Module):
         self.w_gate = nn.Linear(cfg.d_model, cfg.d_ff, bias=False)
         self.w_up = nn.Linear(cfg.d_model, cfg.d_ff, bias=False)
         self.w_down = nn.Linear(cfg.d_ff, cfg.d_model, bias=False)
-        self.any_hip = cfg.any_hip
+        self.any_hip = cfg.any_hip and cfg.d_model % 8 == 0 and cfg.d_ff % 8 == 0  # (the kernels' rows of 16-byte vectors)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.any_hip and x.is_cuda:
