@@ -28,6 +28,11 @@ size_t nn_linear_wgrad_workspace_size(int64_t T, int64_t N, int64_t K);
  * 16-byte aligned), in one launch: a layer's weights at the start of its forward. */
 int nn_linear_cast(int n, const float* const* src, void* const* dst, const int64_t* count, int dtype, void* stream);
 
+/* The same for n (1 to 4) dense row-major matrices of rows[i] x cols[i] (multiples of 8), and each also transposed:
+ * dst_t[i][c * ldt[i] + r] = dst[i][r * cols[i] + c], ldt[i] a multiple of 8, at least rows[i]. */
+int nn_linear_cast_both(int n, const float* const* src, void* const* dst, void* const* dst_t, const int64_t* rows,
+                        const int64_t* cols, const int64_t* ldt, int dtype, void* stream);
+
 /* SwiGLU: h = silu(g) u with silu(g) = g / (1 + exp(-g)), in fp32 with one rounding. gu is [T][2 F] (a row's F values
  * of g, then its F values of u: the stacked product of the gate and up layers), h is [T][F]; dense, 16-byte aligned,
  * F a multiple of 8. The backward writes dgu = (dh u silu'(g), dh silu(g)), [T][2 F].

@@ -393,34 +393,48 @@ std::vector<Tensor> wgrad(const Tensor& dy_, const Tensor& x_, const std::vector
     return out;
 }
 
-// Each group of fp32 (N_i, K) weights stacked into one (sum N_i, K) 16-bit tensor, in one launch.
-std::vector<Tensor> cast_weights(const Tensor& like, const std::vector<std::vector<Tensor>>& groups) {
-    std::vector<Tensor> out;
+// Each group of fp32 (N_i, K) weights stacked into one (sum N_i, K) 16-bit tensor, in one launch: for the layers'
+// products, and for the products of their inputs' gradients (the same tensors, or, `turned`, transposed copies, seen as
+// (sum N_i, K), which the library multiplies by faster; every N_i is then a multiple of 8).
+struct Weights {
+    std::vector<Tensor> fwd, bwd;
+};
+Weights cast_weights(const Tensor& like, const std::vector<std::vector<Tensor>>& groups, bool turned) {
+    Weights out;
     std::vector<const float*> src;
-    std::vector<void*> dst;
-    std::vector<int64_t> count;
+    std::vector<void*> dst, dst_t;
+    std::vector<int64_t> count, rows, cols, ldt;
     for (const auto& g : groups) {
         int64_t N = 0;
+        const int64_t K = g[0].size(1);
         for (const Tensor& w : g) N += w.size(0);
-        out.push_back(empty_of(like, {N, g[0].size(1)}));
-        char* at = (char*)out.back().data_ptr();
+        out.fwd.push_back(empty_of(like, {N, K}));
+        const Tensor t = turned ? empty_of(like, {K, N}) : Tensor();
+        out.bwd.push_back(turned ? t.t() : out.fwd.back());
+        char *at = (char*)out.fwd.back().data_ptr(), *at_t = turned ? (char*)t.data_ptr() : nullptr;
         for (const Tensor& w : g) {
             src.push_back(w.data_ptr<float>());
             dst.push_back(at);
             count.push_back(w.numel());
             at += 2 * w.numel();
+            if (!turned) continue;
+            dst_t.push_back(at_t);
+            at_t += 2 * w.size(0);
+            rows.push_back(w.size(0)), cols.push_back(K), ldt.push_back(N);
         }
     }
-    lin_done(nn_linear_cast((int)src.size(), src.data(), dst.data(), count.data(), code(like), stream_of(like)));
+    const int n = (int)src.size(), dt = code(like);
+    lin_done(turned ? nn_linear_cast_both(n, src.data(), dst.data(), dst_t.data(), rows.data(), cols.data(), ldt.data(), dt, stream_of(like))
+                    : nn_linear_cast(n, src.data(), dst.data(), count.data(), dt, stream_of(like)));
     return out;
 }
 
-// Layers that share an input: (their outputs side by side, the stacked 16-bit weights).
-T2 project_fwd(const Tensor& x, const std::vector<Tensor>& ws) {
+// Layers that share an input: (their outputs side by side, the stacked 16-bit weights for the backward).
+T2 project_fwd(const Tensor& x, const std::vector<Tensor>& ws, bool turned) {
     const Inner inner;
     const c10::DeviceGuard guard(x.device());
-    Tensor w = cast_weights(x, {ws})[0];
-    return {at::mm(x, w.t()), w};
+    const Weights w = cast_weights(x, {ws}, turned);
+    return {at::mm(x, w.fwd[0].t()), w.bwd[0]};
 }
 
 // The attention layer (kernels/hip/layers.py): sizes, and the strides of its tensors for the library. q, k and v are
@@ -446,20 +460,21 @@ struct LayerShape {
 };
 
 std::vector<Tensor> attention_layer_fwd(const Tensor& x, const Tensor& cos, const Tensor& sin, int64_t B, int64_t T, int64_t H,
-                                        int64_t KVH, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wo) {
+                                        int64_t KVH, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wo,
+                                        bool turned) {
     const Inner inner;
     const c10::DeviceGuard guard(x.device());
     const LayerShape s(B, T, H, KVH, wq.size(0) / H);
     const int dt = code(x);
     void* st = stream_of(x);
-    auto w = cast_weights(x, {{wq, wk, wv}, {wo}});
-    Tensor qkv = at::mm(x, w[0].t());
+    const Weights w = cast_weights(x, {{wq, wk, wv}, {wo}}, turned);
+    Tensor qkv = at::mm(x, w.fwd[0].t());
     Tensor q = empty_of(x, {B * T, s.nq}), o = empty_of(x, {B * T, s.nq}), lse = empty_f32(x, {B, H, T});
     rope_done(nn_rope_qk_views(qkv.data_ptr(), q.data_ptr(), s.k(qkv), s.k(qkv), cos.data_ptr<float>(), sin.data_ptr<float>(), B, T, H,
                                KVH, s.D, s.rot, cos.size(0), dt, 0, st));
     fa_done(nn_fa_fwd_views(q.data_ptr(), s.k(qkv), s.v(qkv), o.data_ptr(), lse.data_ptr<float>(), B, H, KVH, T, s.D, s.fwd, dt,
                             scale_of(s.D), st));
-    return {at::mm(o, w[1].t()), qkv, q, o, lse, w[0], w[1]};
+    return {at::mm(o, w.fwd[1].t()), qkv, q, o, lse, w.bwd[0], w.bwd[1]};
 }
 
 // The gradients of x, wq, wk, wv and wo; undefined where not needed.
@@ -491,15 +506,15 @@ std::vector<OptTensor> attention_layer_bwd(const Tensor& dy_, const Tensor& x, c
     return out;
 }
 
-std::vector<Tensor> mlp_fwd(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down) {
+std::vector<Tensor> mlp_fwd(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down, bool turned) {
     const Inner inner;
     const c10::DeviceGuard guard(x.device());
-    auto w = cast_weights(x, {{w_gate, w_up}, {w_down}});
-    Tensor gu = at::mm(x, w[0].t());
+    const Weights w = cast_weights(x, {{w_gate, w_up}, {w_down}}, turned);
+    Tensor gu = at::mm(x, w.fwd[0].t());
     const int64_t T = x.size(0), F = w_gate.size(0);
     Tensor h = empty_of(x, {T, F});
     lin_done(nn_swiglu_fwd(gu.data_ptr(), h.data_ptr(), T, F, code(x), stream_of(x)));
-    return {at::mm(h, w[1].t()), gu, h, w[0], w[1]};
+    return {at::mm(h, w.fwd[1].t()), gu, h, w.bwd[0], w.bwd[1]};
 }
 
 // The gradients of x, w_gate, w_up and w_down; undefined where not needed.
@@ -523,20 +538,21 @@ std::vector<OptTensor> mlp_bwd(const Tensor& dy_, const Tensor& x, const Tensor&
     return out;
 }
 
-// (logits, loss, w16, lse, 1 / rows that count).
-std::vector<Tensor> head_fwd(const Tensor& x, const Tensor& w_, const Tensor& targets) {
+// (logits, loss, w16 for the backward, lse, 1 / rows that count).
+std::vector<Tensor> head_fwd(const Tensor& x, const Tensor& w_, const Tensor& targets, bool turned) {
     const Inner inner;
     const c10::DeviceGuard guard(x.device());
-    Tensor w = cast_weights(x, {{w_}})[0], logits = at::mm(x, w.t());
+    const Weights w = cast_weights(x, {{w_}}, turned && w_.size(0) % 8 == 0);
+    const Tensor logits = at::mm(x, w.fwd[0].t());
     const int64_t R = logits.size(0), V = logits.size(1);
     Tensor lse = empty_f32(x, {R}), rows = empty_f32(x, {R}), loss = empty_f32(x, {}), inv = empty_f32(x, {});
     loss_done(nn_cross_entropy_fwd(logits.data_ptr(), targets.data_ptr<int64_t>(), lse.data_ptr<float>(), rows.data_ptr<float>(),
                                    loss.data_ptr<float>(), inv.data_ptr<float>(), R, V, code(x), stream_of(x)));
-    return {logits, loss, w, lse, inv};
+    return {logits, loss, w.bwd[0], lse, inv};
 }
 
 // The gradients of x and w from those of the logits and of the loss (either may be missing); logits: the forward's, or
-// nothing to compute them again.
+// nothing to compute them again (by the forward's product, on rows).
 std::vector<OptTensor> head_bwd(const OptTensor& dlogits_, const OptTensor& dloss, const OptTensor& logits_, const Tensor& x,
                                 const Tensor& w, const Tensor& targets, const Tensor& lse, const Tensor& inv, bool need_x, bool need_w) {
     const Inner inner;
@@ -544,7 +560,7 @@ std::vector<OptTensor> head_bwd(const OptTensor& dlogits_, const OptTensor& dlos
     std::vector<OptTensor> out(2);
     Tensor d = dlogits_.has_value() ? contig(*dlogits_) : Tensor();
     if (dloss.has_value()) {
-        const Tensor logits = logits_.has_value() ? *logits_ : at::mm(x, w.t()), g = contig(*dloss);
+        const Tensor logits = logits_.has_value() ? *logits_ : at::mm(x, contig(w).t()), g = contig(*dloss);
         Tensor t = at::empty_like(logits);
         loss_done(nn_cross_entropy_bwd(logits.data_ptr(), targets.data_ptr<int64_t>(), lse.data_ptr<float>(), inv.data_ptr<float>(),
                                        g.data_ptr<float>(), t.data_ptr(), logits.size(0), logits.size(1), code(x), stream_of(x)));

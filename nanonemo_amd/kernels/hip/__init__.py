@@ -103,6 +103,9 @@ SIGNATURES: dict[str, tuple] = {
     ),
     "nn_linear_wgrad_workspace_size": (_sz, [_i64, _i64, _i64]),
     "nn_linear_cast": (_int, [_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _int, _vp]),
+    "nn_linear_cast_both": (
+        _int, [_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _i64p, _i64p, _int, _vp]
+    ),
     "nn_swiglu_fwd": (_int, [_vp, _vp, _i64, _i64, _int, _vp]),
     "nn_swiglu_bwd": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _vp]),
     "nn_linear_last_error": (ctypes.c_char_p, []),

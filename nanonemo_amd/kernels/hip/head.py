@@ -12,7 +12,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from nanonemo_amd.kernels.hip import host
+from nanonemo_amd.kernels.hip import host, records
 from nanonemo_amd.kernels.hip.linear import eligible, plain
 
 
@@ -25,8 +25,8 @@ def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
 
 class _HeadLoss(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w, targets):
-        logits, loss, w16, lse, inv = host().head_fwd(x, w, targets)
+    def forward(ctx, x, w, targets, turned):
+        logits, loss, w16, lse, inv = host().head_fwd(x, w, targets, turned)
         ctx.save_for_backward(x, w16, w, targets, lse, inv)
         # The caller owns the logits and may change them in place before the backward, which then computes them again
         # from x: an alias that shares their version counter and not their graph, instead of a saved output, whose
@@ -39,11 +39,11 @@ class _HeadLoss(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dlogits, dloss):
         x, w16, w, targets, lse, inv = ctx.saved_tensors
-        need_x, need_w, _ = ctx.needs_input_grad
+        need_x, need_w = ctx.needs_input_grad[:2]
         if torch.is_grad_enabled():
-            return _replayed(x, w, targets, (need_x, need_w), dlogits, dloss)
+            return *_replayed(x, w, targets, (need_x, need_w), dlogits, dloss), None
         logits = ctx.logits if ctx.logits._version == ctx.version else None
-        return (*host().head_bwd(dlogits, dloss, logits, x, w16, targets, lse, inv, need_x, need_w), None)
+        return (*host().head_bwd(dlogits, dloss, logits, x, w16, targets, lse, inv, need_x, need_w), None, None)
 
 
 def _replayed(x, w, targets, need, dlogits, dloss):
@@ -64,5 +64,5 @@ def _replayed(x, w, targets, need, dlogits, dloss):
 def head_loss(x: Tensor, layer: nn.Linear, targets: Tensor) -> tuple[Tensor, Tensor]:
     """(layer(x), the mean cross entropy of its rows against the targets) for calls that can_fuse_head."""
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
-    logits, loss = _HeadLoss.apply(flat, layer.weight, targets.reshape(-1).contiguous())
+    logits, loss = _HeadLoss.apply(flat, layer.weight, targets.reshape(-1).contiguous(), records(flat))
     return logits.view(*x.shape[:-1], logits.shape[1]), loss

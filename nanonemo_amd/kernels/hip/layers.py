@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from nanonemo_amd.kernels.hip import host
+from nanonemo_amd.kernels.hip import host, records
 from nanonemo_amd.kernels.hip.flash_attn import flash_attn_bthd
 from nanonemo_amd.kernels.hip.linear import eligible, plain
 from nanonemo_amd.kernels.hip.rope import rope_qk
@@ -48,8 +48,8 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
 
 class _AttentionLayer(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, cos, sin, B, T, H, KVH, wq, wk, wv, wo):
-        y, qkv, q, o, lse, w, wo16 = host().attention_layer_fwd(x, cos, sin, B, T, H, KVH, wq, wk, wv, wo)
+    def forward(ctx, x, cos, sin, B, T, H, KVH, wq, wk, wv, wo, turned):
+        y, qkv, q, o, lse, w, wo16 = host().attention_layer_fwd(x, cos, sin, B, T, H, KVH, wq, wk, wv, wo, turned)
         ctx.save_for_backward(x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo)
         ctx.sizes = (B, T, H, KVH)
         return y
@@ -59,9 +59,9 @@ class _AttentionLayer(torch.autograd.Function):
         x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():
-            return _replayed(_modular, (x, wq, wk, wv, wo), (need[0], *need[7:]), dy, (cos, sin, *ctx.sizes), at=7)
+            return _replayed(_modular, (x, wq, wk, wv, wo), (need[0], *need[7:11]), dy, (cos, sin, *ctx.sizes), at=7) + (None,)
         dx, *dws = host().attention_layer_bwd(dy, x, cos, sin, qkv, q, o, lse, w, wo16, *ctx.sizes, need[0], any(need[7:10]), need[10])
-        return dx, None, None, None, None, None, None, *(g if n else None for g, n in zip(dws, need[7:]))
+        return dx, None, None, None, None, None, None, *(g if n else None for g, n in zip(dws, need[7:11])), None
 
 
 def _modular(x, wq, wk, wv, wo, cos, sin, B, T, H, KVH):
@@ -87,7 +87,8 @@ def attention_layer(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: i
     """wo(attention(rope(wq x), rope(wk x), wv x)) on x (B, T, d) in the autocast dtype, for calls that can_fuse."""
     B, T, d = x.shape
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(B * T, d)
-    y = _AttentionLayer.apply(flat, cos, sin, B, T, heads, kv_heads, wq.weight, wk.weight, wv.weight, wo.weight)
+    y = _AttentionLayer.apply(flat, cos, sin, B, T, heads, kv_heads, wq.weight, wk.weight, wv.weight, wo.weight,
+                              records(flat, wq.weight, wk.weight, wv.weight))
     return y.view(B, T, -1)
 
 
@@ -105,19 +106,19 @@ def can_fuse_mlp(x: Tensor, w_gate, w_up, w_down) -> bool:
 
 class _MlpLayer(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w_gate, w_up, w_down):
-        y, gu, h, w, wd = host().mlp_fwd(x, w_gate, w_up, w_down)
+    def forward(ctx, x, w_gate, w_up, w_down, turned):
+        y, gu, h, w, wd = host().mlp_fwd(x, w_gate, w_up, w_down, turned)
         ctx.save_for_backward(x, gu, h, w, wd, w_gate, w_up, w_down)
         return y
 
     @staticmethod
     def backward(ctx, dy):
         x, gu, h, w, wd, w_gate, w_up, w_down = ctx.saved_tensors
-        need = ctx.needs_input_grad
+        need = ctx.needs_input_grad[:4]
         if torch.is_grad_enabled():
-            return _replayed(_modular_mlp, (x, w_gate, w_up, w_down), need, dy, (), at=1)
+            return _replayed(_modular_mlp, (x, w_gate, w_up, w_down), need, dy, (), at=1) + (None,)
         grads = host().mlp_bwd(dy, x, gu, h, w, wd, need[0], need[1] or need[2], need[3])
-        return tuple(g if n else None for g, n in zip(grads, need))
+        return *(g if n else None for g, n in zip(grads, need)), None
 
 
 def _modular_mlp(x, w_gate, w_up, w_down):
@@ -128,5 +129,5 @@ def _modular_mlp(x, w_gate, w_up, w_down):
 def mlp_layer(x: Tensor, w_gate: nn.Linear, w_up: nn.Linear, w_down: nn.Linear) -> Tensor:
     """w_down(silu(w_gate x) * w_up x) on x (..., d) in the autocast dtype, for calls that can_fuse_mlp."""
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
-    y = _MlpLayer.apply(flat, w_gate.weight, w_up.weight, w_down.weight)
+    y = _MlpLayer.apply(flat, w_gate.weight, w_up.weight, w_down.weight, records(flat, w_gate.weight, w_up.weight))
     return y.view(*x.shape[:-1], y.shape[1])

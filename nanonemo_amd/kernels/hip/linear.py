@@ -21,7 +21,7 @@ from torch import Tensor, nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
-from nanonemo_amd.kernels.hip import eager, host
+from nanonemo_amd.kernels.hip import eager, host, records
 
 _DTYPES = (torch.float16, torch.bfloat16)
 
@@ -67,8 +67,8 @@ class _Projections(torch.autograd.Function):
     """y_i = x W_i^T: x (T, K) 16-bit, W_i fp32, y_i the column ranges of one (T, sum N_i) product."""
 
     @staticmethod
-    def forward(ctx, x, *ws):
-        y, w16 = host().project_fwd(x, ws)
+    def forward(ctx, x, turned, *ws):
+        y, w16 = host().project_fwd(x, ws, turned)
         ctx.save_for_backward(x, w16, *ws)
         ctx.set_materialize_grads(False)
         return (y,) if len(ws) == 1 else y.split([w.shape[0] for w in ws], dim=1)
@@ -77,7 +77,7 @@ class _Projections(torch.autograd.Function):
     def backward(ctx, *dys):
         x, w16, *ws = ctx.saved_tensors
         rows = [w.shape[0] for w in ws]
-        need_w = any(ctx.needs_input_grad[1:])
+        need_w = any(ctx.needs_input_grad[2:])
         dy = stacked(dys, rows, x)
         if torch.is_grad_enabled():  # a recorded backward
             wd = torch.cat([w.to(x.dtype) for w in ws])
@@ -86,10 +86,10 @@ class _Projections(torch.autograd.Function):
         else:
             dx = dy @ w16 if ctx.needs_input_grad[0] else None
             dws = wgrad(dy, x, rows) if need_w else [None] * len(ws)
-        return dx, *(g if n else None for g, n in zip(dws, ctx.needs_input_grad[1:]))
+        return dx, None, *(g if n else None for g, n in zip(dws, ctx.needs_input_grad[2:]))
 
 
 def projections(x: Tensor, *layers: nn.Linear) -> tuple[Tensor, ...]:
     """The layers' outputs on x (..., K), in the autocast dtype, as (..., N_i) column ranges of one product."""
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
-    return tuple(y.view(*x.shape[:-1], y.shape[1]) for y in _Projections.apply(flat, *(m.weight for m in layers)))
+    return tuple(y.view(*x.shape[:-1], y.shape[1]) for y in _Projections.apply(flat, records(flat), *(m.weight for m in layers)))

@@ -134,3 +134,26 @@ def test_wgrad_copies_what_the_kernel_cannot_read(what):
     assert torch.equal(wgrad(dy, x, [N])[0], wgrad(dy.clone(memory_format=torch.contiguous_format), x, [N])[0])
     (got,), (ref,) = wgrad(x, dy, [K]), wgrad(x, dy.clone(memory_format=torch.contiguous_format), [K])
     assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shapes", [[(8, 8)], [(72, 56), (8, 200), (136, 64)], [(1280, 768), (64, 64), (128, 8), (16, 328)]])
+def test_cast_both_is_exact(shapes, dtype):
+    from nanonemo_amd.kernels import hip
+
+    ws = [torch.randn(s, device="cuda") for s in shapes]
+    dst = [torch.full(s, float("nan"), device="cuda", dtype=dtype) for s in shapes]
+    ldt = [r + 8 * (i % 2) for i, (r, _) in enumerate(shapes)]
+    turned = [torch.full((c, ld), float("nan"), device="cuda", dtype=dtype) for (_, c), ld in zip(shapes, ldt)]
+    n = len(ws)
+    ptrs = [(ctypes.c_void_p * n)(*(t.data_ptr() for t in ts)) for ts in (ws, dst, turned)]
+    sizes = [(ctypes.c_int64 * n)(*v) for v in ([r for r, _ in shapes], [c for _, c in shapes], ldt)]
+    stream = torch.cuda.current_stream().cuda_stream
+    code = hip.DTYPE_BF16 if dtype is torch.bfloat16 else hip.DTYPE_F16
+    assert hip.lib().nn_linear_cast_both(n, *ptrs, *sizes, code, stream) == 0
+    for w, d, t, (r, _) in zip(ws, dst, turned, shapes):
+        assert torch.equal(d, w.to(dtype))
+        assert torch.equal(t[:, :r], w.to(dtype).t())
+        assert t[:, r:].isnan().all()
+    sizes[0][0] = 4  # not a multiple of 8
+    assert hip.lib().nn_linear_cast_both(n, *ptrs, *sizes, code, stream) != 0
