@@ -3,8 +3,8 @@
 Replaces the reference's JIT build (/root/reference/nanonemo/kernels/cuda/__init__.py:15-18, which runs
 nvcc through torch.utils.cpp_extension.load on first use): here ``hipcc`` compiles
 ``nanonemo_amd/csrc/*.hip`` once, in-tree, into ``nanonemo_amd/lib/libnanonemo_fa.so``, a plain C-ABI
-shared library with no torch types in its signatures (include/*.h). The library is loaded with ctypes (nanonemo_amd/kernels/hip/__init__.py), so the same .so runs on any box with the ROCm
-runtime.
+shared library with no torch types in its signatures (include/*.h), and ``g++`` compiles ``csrc/host.cpp`` into
+``nanonemo_host.so``, the torch extension that calls it.
 
     python -m nanonemo_amd.build
 """

@@ -1,10 +1,11 @@
 """The model's attention layer and MLP as one call each under 16-bit autocast, forward and backward
 (/root/reference/nanonemo/model/layers.py:77-116,119-137).
 
-Attention: projections, rotary embedding, attention and output projection. The layer's own memory order lets every kernel read what the one before it wrote: q, k and v are column ranges of one
-product's (B T, (H + 2 KVH) hd) output, the rotation writes q to a tensor of its own and k over itself, the attention
-reads k and v where they lie (nn_fa_fwd_views), and the backward writes dq, dk and dv as column ranges of one buffer,
-rotates them back in place and hands it to one product for the input's gradient and one call for the three weights'.
+Attention: projections, rotary embedding, attention and output projection. The layer's own memory order lets every
+kernel read what the one before it wrote: q, k and v are column ranges of one product's (B T, (H + 2 KVH) hd) output, the
+rotation writes q to a tensor of its own and k over itself, the attention reads k and v where they lie (nn_fa_fwd_views),
+and the backward writes dq, dk and dv as column ranges of one buffer, rotates them back in place and hands it to one
+product for the input's gradient and one call for the three weights'.
 That is 6 launches forward and 9 to 11 backward, where the modules take 27 in all: a cast, a product and a rounding
 per weight each way, three input gradients added in 16 bits.
 
@@ -12,8 +13,12 @@ MLP: one product for gate and up, SwiGLU on its two halves (nn_swiglu_*), the do
 the gate's and up's weight gradients and one product for the input's gradient. 4 launches forward and 6 to 8 backward
 instead of 21.
 
-``can_fuse`` and ``can_fuse_mlp`` hold for the calls that ``linear.can_project`` describes, with every module of the layer untouched; the others run module by module. A backward that is itself recorded replays the layer through PyTorch's linear layers
-and the package's differentiable functions, so that what those support is what it supports.
+A layer's weights are rounded to 16 bits in one launch at the start of its forward; where a backward will be run
+(``turned``), a transposed copy is written beside them, which the products for the inputs' gradients read.
+
+``can_fuse`` and ``can_fuse_mlp`` hold for the calls that ``linear.can_project`` describes, with every module of the layer
+untouched; the others run module by module. A backward that is itself recorded replays the layer through PyTorch's linear
+layers and the package's differentiable functions, so that what those support is what it supports.
 """
 
 from __future__ import annotations

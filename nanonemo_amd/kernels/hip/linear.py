@@ -25,6 +25,7 @@ from nanonemo_amd.kernels.hip import eager, host, records
 
 _DTYPES = (torch.float16, torch.bfloat16)
 
+
 def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
     """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width
     (and of a multiple of 8 outputs, unless odd_rows)."""
