@@ -64,5 +64,9 @@ def _replayed(x, w, targets, need, dlogits, dloss):
 def head_loss(x: Tensor, layer: nn.Linear, targets: Tensor) -> tuple[Tensor, Tensor]:
     """(layer(x), the mean cross entropy of its rows against the targets) for calls that can_fuse_head."""
     flat = x.to(torch.get_autocast_dtype("cuda")).reshape(-1, x.shape[-1])
-    logits, loss = _HeadLoss.apply(flat, layer.weight, targets.reshape(-1).contiguous(), records(flat))
+    targets = targets.reshape(-1).contiguous()
+    if records(flat, layer.weight):
+        logits, loss = _HeadLoss.apply(flat, layer.weight, targets, records(flat))
+    else:  # nothing to keep for a backward (inference tensors have no version to keep either)
+        logits, loss = host().head_fwd(flat, layer.weight, targets, False)[:2]
     return logits.view(*x.shape[:-1], logits.shape[1]), loss

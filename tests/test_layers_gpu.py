@@ -122,6 +122,20 @@ def test_mlp_layer_matches_its_modules(shape, d, ff, dtype):
         torch.testing.assert_close(a, b, rtol=tol, atol=tol * b.abs().max().item(), msg=name)
 
 
+@pytest.mark.parametrize("kw", [dict(attn_kernel="hip_bthd", rope_kernel="hip", norm_kernel="hip"), dict(attn_kernel="hip")])
+def test_model_under_inference_mode(kw):
+    from nanonemo_amd.model import NanoNemo
+
+    torch.manual_seed(0)
+    m = NanoNemo(ModelConfig(n_layers=2, d_model=256, n_heads=4, n_kv_heads=2, d_ff=512, vocab_size=512, max_seq_len=96, **kw)).cuda()
+    idx = torch.randint(0, 512, (2, 96), device="cuda")
+    out = []
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+            out.append(m(idx, torch.roll(idx, -1, 1)))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T, F", [(1, 8), (3, 104), (129, 2048)])
 def test_swiglu_matches_float64(T, F, dtype):
