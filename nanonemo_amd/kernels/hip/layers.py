@@ -28,7 +28,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from nanonemo_amd.kernels.hip import host, records
-from nanonemo_amd.kernels.hip.flash_attn import flash_attn_bthd
+from nanonemo_amd.kernels.hip.flash_attn import _refuse_capture_with_autograd, flash_attn_bthd
 from nanonemo_amd.kernels.hip.linear import eligible, plain
 from nanonemo_amd.kernels.hip.rope import rope_qk
 
@@ -61,6 +61,7 @@ class _AttentionLayer(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        _refuse_capture_with_autograd("attention layer backward")
         x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():

@@ -30,3 +30,22 @@ def test_head_loss_under_inference_mode(host):
     with torch.inference_mode():
         got = head.head_loss(x, m, t)
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_attention_layer_backward_refuses_capture(monkeypatch):
+    # As the attention functions' backward does: a forward run eagerly and its backward under capture must not reach
+    # the launches. The guard comes before the saved tensors are read.
+    from nanonemo_amd.kernels.hip import layers
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+
+    class Ctx:
+        needs_input_grad = (True,) * 12
+
+        @property
+        def saved_tensors(self):
+            raise AssertionError("the guard must raise before the saved tensors are read")
+
+    with pytest.raises(RuntimeError, match="attention layer backward: capturing"):
+        layers._AttentionLayer.backward(Ctx(), torch.zeros(4, 8))
