@@ -3,7 +3,8 @@
 
 The loss reads the 16-bit logits once and its backward reads them once and writes their gradient, where F.cross_entropy
 on logits.float() moves an fp32 copy, its log-softmax and their gradients. ``can_fuse_head`` holds for calls that
-``linear.can_project`` describes with int64 targets; the others run module by module.
+``linear.can_project`` describes with int64 targets; the others run module by module. A target that is neither -100 nor in [0, V) makes the loss and its row's
+gradient NaN (F.cross_entropy ends the process with a device assertion).
 """
 
 from __future__ import annotations

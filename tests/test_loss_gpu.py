@@ -70,6 +70,15 @@ def test_cross_entropy_special_values_follow_torch(dtype):
     assert _call(base, t)[1].isnan()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("bad", [-1, 300, 1 << 40])
+def test_a_target_out_of_range_shows_in_the_loss_and_in_its_rows_gradient(dtype, bad):
+    logits = torch.randn(4, 300, device="cuda").to(dtype)
+    t = torch.tensor([0, bad, -100, 3], device="cuda")
+    _, loss, d = _call(logits, t)
+    assert loss.isnan() and d[1].isnan().all() and d[[0, 2, 3]].isfinite().all()
+
+
 @pytest.mark.parametrize("V", [512, 1003])
 def test_head_loss_matches_its_modules(V):
     from nanonemo_amd.kernels.hip import head
