@@ -17,7 +17,8 @@ extern "C" {
 int nn_cross_entropy_fwd(const void* logits, const int64_t* targets, float* lse, float* rows, float* loss, float* inv,
                          int64_t R, int64_t V, int dtype, void* stream);
 
-/* dlogits = (softmax(logits) - onehot(target)) * grad[0] * inv[0], zero for rows that do not count; lse and inv as the
+/* dlogits = (softmax(logits) - onehot(target)) * grad[0] * inv[0], zero for rows that do not count (NaN if their logits
+ * hold a NaN or +inf, as in PyTorch); lse and inv as the
  * forward wrote them, grad the gradient of the loss (one fp32), dlogits in the logits' dtype. NaN in a row whose target is
  * out of range. */
 int nn_cross_entropy_bwd(const void* logits, const int64_t* targets, const float* lse, const float* inv,

@@ -162,10 +162,10 @@ __global__ __launch_bounds__(kThreads) void ce_bwd_kernel(const void* __restrict
     const T* row = reinterpret_cast<const T*>(logits) + off;
     T* dst = reinterpret_cast<T*>(dlogits) + off;
     const long long t = targets[blockIdx.x];
-    const bool counts = t != kIgnore;
-    // A target out of range shows in its row's gradient as it does in the loss, so that no step is taken on it.
-    const float g = !counts ? 0.f : t >= 0 && t < V ? grad[0] * inv[0] : NAN, l = lse[blockIdx.x];
-    auto of = [&](float x, int j) { return counts ? (exp_diff(x, l) - (j == t ? 1.f : 0.f)) * g : 0.f; };
+    // A row that does not count has a zero gradient, or NaN where its logits hold one (or +inf), as in PyTorch. A
+    // target out of range shows in its row's gradient as it does in the loss, so that no step is taken on it.
+    const float g = t == kIgnore ? 0.f : t >= 0 && t < V ? grad[0] * inv[0] : NAN, l = lse[blockIdx.x];
+    auto of = [&](float x, int j) { return (exp_diff(x, l) - (j == t ? 1.f : 0.f)) * g; };
     const int head = R::head(row, V), nv = (V - head) / R::W, tail = head + nv * R::W, tid = threadIdx.x;
     if (tid < head) dst[tid] = R::round(of(R::one(row[tid]), tid));
     if (tid < V - tail) dst[tail + tid] = R::round(of(R::one(row[tail + tid]), tail + tid));

@@ -71,6 +71,20 @@ def test_cross_entropy_special_values_follow_torch(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_special_values_in_a_row_that_does_not_count_follow_torch(value, dtype):
+    logits = torch.randn(3, 300, device="cuda").to(dtype)
+    logits[1, 7] = value
+    t = torch.tensor([0, -100, 2], device="cuda")
+    _, loss, d = _call(logits, t)
+    x = logits.float().requires_grad_()
+    ref = F.cross_entropy(x, t)
+    (rg,) = torch.autograd.grad(ref, x)
+    assert torch.allclose(loss, ref.detach(), rtol=1e-5)
+    assert torch.equal(d.isnan(), rg.isnan()) and (d[1].isnan() | (d[1] == 0)).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("bad", [-1, 300, 1 << 40])
 def test_a_target_out_of_range_shows_in_the_loss_and_in_its_rows_gradient(dtype, bad):
     logits = torch.randn(4, 300, device="cuda").to(dtype)
