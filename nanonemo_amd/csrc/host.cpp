@@ -638,6 +638,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("head_fwd", head_fwd, nogil);
     m.def("head_bwd", head_bwd, nogil);
     m.def("plain_cuda", plain_cuda);
+    // A tensor's version counter (which its changes in place raise), without the tensor.
+    py::class_<c10::VariableVersion>(m, "Version")
+        .def(py::init([](const Tensor& t) { return t.unsafeGetTensorImpl()->version_counter(); }))
+        .def("current", &c10::VariableVersion::current_version);
     m.def("strides_of", strides_py);
     m.def("readable", readable_py, py::arg("a"), py::arg("b") = std::nullopt);
 }

@@ -28,22 +28,22 @@ class _HeadLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, targets, turned):
         logits, loss, w16, lse, inv = host().head_fwd(x, w, targets, turned)
-        ctx.save_for_backward(x, w16, w, targets, lse, inv)
         # The caller owns the logits and may change them in place before the backward, which then computes them again
-        # from x: an alias that shares their version counter and not their graph, instead of a saved output, whose
-        # change would be an error.
-        ctx.logits = logits.detach()
-        ctx.version = logits._version
+        # from x. Saved is an alias with a version of its own (saving the output would make such a change an error);
+        # whether the logits have changed is read from their own version, which holds on to no memory.
+        ctx.save_for_backward(x, w16, w, targets, lse, inv, logits.data)
+        ctx.version, ctx.at = host().Version(logits), logits._version
         ctx.set_materialize_grads(False)
         return logits, loss
 
     @staticmethod
     def backward(ctx, dlogits, dloss):
-        x, w16, w, targets, lse, inv = ctx.saved_tensors
+        x, w16, w, targets, lse, inv, logits = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad[:2]
         if torch.is_grad_enabled():
             return *_replayed(x, w, targets, (need_x, need_w), dlogits, dloss), None
-        logits = ctx.logits if ctx.logits._version == ctx.version else None
+        if ctx.version.current() != ctx.at:
+            logits = None
         return (*host().head_bwd(dlogits, dloss, logits, x, w16, targets, lse, inv, need_x, need_w), None, None)
 
 

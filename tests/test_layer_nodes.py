@@ -49,3 +49,26 @@ def test_attention_layer_backward_refuses_capture(monkeypatch):
 
     with pytest.raises(RuntimeError, match="attention layer backward: capturing"):
         layers._AttentionLayer.backward(Ctx(), torch.zeros(4, 8))
+
+
+def test_head_loss_keeps_nothing_past_its_backward(host):
+    # The logits are a saved tensor: autograd's hooks see them and a backward that does not retain the graph frees them,
+    # while the caller may still change the logits it was given before the backward.
+    from nanonemo_amd.kernels.hip import head
+
+    m, x, t = _head_inputs()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda v: packed.append(v) or v, lambda v: v):
+        logits, loss = head.head_loss(x, m, t)
+    assert logits.data_ptr() in [v.data_ptr() for v in packed]
+    node = loss.grad_fn
+    (g1,) = torch.autograd.grad(loss, m.weight, retain_graph=True)
+    assert not host.recomputed
+    with torch.no_grad():
+        logits.mul_(2.0)
+    (g2,) = torch.autograd.grad(loss, m.weight)
+    assert host.recomputed
+    torch.testing.assert_close(g1, g2)
+    assert not any(isinstance(v, torch.Tensor) and v.numel() >= logits.numel() for v in vars(node).values())
+    with pytest.raises(RuntimeError, match="freed"):
+        node.saved_tensors

@@ -126,6 +126,19 @@ def test_head_loss_matches_its_modules(V):
     assert torch.equal(out[0][2], out[0][-2]) and torch.equal(out[0][3], out[0][-1])
 
 
+def test_head_loss_frees_the_logits_with_the_backward():
+    from nanonemo_amd.kernels.hip import head
+
+    m = nn.Linear(64, 4096, bias=False).cuda()
+    x, t = torch.randn(2048, 64, device="cuda"), torch.randint(0, 4096, (2048,), device="cuda")
+    m.weight.grad = torch.zeros_like(m.weight)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        loss = head.head_loss(x, m, t)[1]
+    held = torch.cuda.memory_allocated()
+    loss.backward()
+    assert held - torch.cuda.memory_allocated() >= 2048 * 4096 * 2  # with loss still referenced
+
+
 def test_head_loss_second_derivative():
     from nanonemo_amd.kernels.hip import head
 
