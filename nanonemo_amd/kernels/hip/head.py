@@ -14,7 +14,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from nanonemo_amd.kernels.hip import host, records
-from nanonemo_amd.kernels.hip.linear import eligible, plain
+from nanonemo_amd.kernels.hip.linear import Stored, eligible, plain
 
 
 def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
@@ -31,26 +31,26 @@ class _HeadLoss(torch.autograd.Function):
         # The caller owns the logits and may change them in place before the backward, which then computes them again
         # from x. Saved is an alias with a version of its own (saving the output would make such a change an error);
         # whether the logits have changed is read from their own version, which holds on to no memory.
-        ctx.save_for_backward(x, w16, w, targets, lse, inv, logits.data)
-        ctx.version, ctx.at = host().Version(logits), logits._version
+        ctx.save_for_backward(x, w16, targets, lse, inv, logits.data)
+        ctx.weight, ctx.version, ctx.at = w, host().Version(logits), logits._version
         ctx.set_materialize_grads(False)
         return logits, loss
 
     @staticmethod
     def backward(ctx, dlogits, dloss):
-        x, w16, w, targets, lse, inv, logits = ctx.saved_tensors
+        x, w16, targets, lse, inv, logits = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad[:2]
         if torch.is_grad_enabled():
-            return *_replayed(x, w, targets, (need_x, need_w), dlogits, dloss), None
+            return *_replayed(x, ctx.weight, w16, targets, (need_x, need_w), dlogits, dloss), None
         if ctx.version.current() != ctx.at:
             logits = None
         return (*host().head_bwd(dlogits, dloss, logits, x, w16, targets, lse, inv, need_x, need_w), None, None)
 
 
-def _replayed(x, w, targets, need, dlogits, dloss):
-    """The gradients as recorded operations."""
+def _replayed(x, w, w16, targets, need, dlogits, dloss):
+    """The gradients as recorded operations on the forward's 16-bit copy of the weight."""
     with torch.enable_grad():
-        logits = F.linear(x, w.to(x.dtype))
+        logits = F.linear(x, Stored.apply(w, w16))
         outs, grads = [], []
         if dlogits is not None:
             outs.append(logits), grads.append(dlogits)

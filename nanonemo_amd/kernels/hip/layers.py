@@ -29,7 +29,7 @@ from torch import Tensor, nn
 
 from nanonemo_amd.kernels.hip import host, records
 from nanonemo_amd.kernels.hip.flash_attn import _refuse_capture_with_autograd, flash_attn_bthd
-from nanonemo_amd.kernels.hip.linear import eligible, plain
+from nanonemo_amd.kernels.hip.linear import Stored, eligible, plain
 from nanonemo_amd.kernels.hip.rope import rope_qk
 
 
@@ -55,37 +55,37 @@ class _AttentionLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, cos, sin, B, T, H, KVH, wq, wk, wv, wo, turned):
         y, qkv, q, o, lse, w, wo16 = host().attention_layer_fwd(x, cos, sin, B, T, H, KVH, wq, wk, wv, wo, turned)
-        ctx.save_for_backward(x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo)
-        ctx.sizes = (B, T, H, KVH)
+        ctx.save_for_backward(x, cos, sin, qkv, q, o, lse, w, wo16)
+        ctx.weights, ctx.sizes = (wq, wk, wv, wo), (B, T, H, KVH)
         return y
 
     @staticmethod
     def backward(ctx, dy):
         _refuse_capture_with_autograd("attention layer backward")
-        x, cos, sin, qkv, q, o, lse, w, wo16, wq, wk, wv, wo = ctx.saved_tensors
+        x, cos, sin, qkv, q, o, lse, w, wo16 = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():
-            return _replayed(_modular, (x, wq, wk, wv, wo), (need[0], *need[7:11]), dy, (cos, sin, *ctx.sizes), at=7) + (None,)
+            copies = (*w.split([m.shape[0] for m in ctx.weights[:3]]), wo16)
+            dx, *dws = _replayed(_modular, x, ctx.weights, copies, (need[0], *need[7:11]), dy, (cos, sin, *ctx.sizes))
+            return dx, None, None, None, None, None, None, *dws, None
         dx, *dws = host().attention_layer_bwd(dy, x, cos, sin, qkv, q, o, lse, w, wo16, *ctx.sizes, need[0], any(need[7:10]), need[10])
         return dx, None, None, None, None, None, None, *(g if n else None for g, n in zip(dws, need[7:11])), None
 
 
 def _modular(x, wq, wk, wv, wo, cos, sin, B, T, H, KVH):
-    """The layer through differentiable functions, on (B T, d) x, in x's dtype."""
+    """The layer through differentiable functions, on (B T, d) x and weights of x's dtype."""
     D = wq.shape[0] // H
-    q, k, v = (F.linear(x, w.to(x.dtype)).view(B, T, -1, D) for w in (wq, wk, wv))
+    q, k, v = (F.linear(x, w).view(B, T, -1, D) for w in (wq, wk, wv))
     q, k = rope_qk(q, k, cos, sin)
-    return F.linear(flash_attn_bthd(q, k, v).view(B * T, H * D), wo.to(x.dtype))
+    return F.linear(flash_attn_bthd(q, k, v).view(B * T, H * D), wo)
 
 
-def _replayed(fn, ins, need, dy, extra, at: int) -> tuple:
-    """The gradients of fn(*ins, *extra) as recorded operations: x's first, then None up to position ``at``, then the
-    weights'."""
+def _replayed(fn, x, weights, copies, need, dy, extra=()) -> list:
+    """The gradients of fn(x, *weights, *extra) as recorded operations on the forward's 16-bit copies of the weights."""
     with torch.enable_grad():
-        y = fn(*ins, *extra)
-        grads = iter(torch.autograd.grad(y, [t for t, n in zip(ins, need) if n], dy, create_graph=True))
-    out = [next(grads) if n else None for n in need]
-    return (out[0], *[None] * (at - 1), *out[1:])
+        y = fn(x, *(Stored.apply(w, c) for w, c in zip(weights, copies)), *extra)
+        grads = iter(torch.autograd.grad(y, [t for t, n in zip((x, *weights), need) if n], dy, create_graph=True))
+    return [next(grads) if n else None for n in need]
 
 
 def attention_layer(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, wq: nn.Linear, wk: nn.Linear,
@@ -114,22 +114,23 @@ class _MlpLayer(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_gate, w_up, w_down, turned):
         y, gu, h, w, wd = host().mlp_fwd(x, w_gate, w_up, w_down, turned)
-        ctx.save_for_backward(x, gu, h, w, wd, w_gate, w_up, w_down)
+        ctx.save_for_backward(x, gu, h, w, wd)
+        ctx.weights = (w_gate, w_up, w_down)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, gu, h, w, wd, w_gate, w_up, w_down = ctx.saved_tensors
+        x, gu, h, w, wd = ctx.saved_tensors
         need = ctx.needs_input_grad[:4]
         if torch.is_grad_enabled():
-            return _replayed(_modular_mlp, (x, w_gate, w_up, w_down), need, dy, (), at=1) + (None,)
+            return *_replayed(_modular_mlp, x, ctx.weights, (*w.chunk(2), wd), need, dy), None
         grads = host().mlp_bwd(dy, x, gu, h, w, wd, need[0], need[1] or need[2], need[3])
         return *(g if n else None for g, n in zip(grads, need)), None
 
 
 def _modular_mlp(x, w_gate, w_up, w_down):
-    """The MLP through differentiable functions, in x's dtype."""
-    return F.linear(F.silu(F.linear(x, w_gate.to(x.dtype))) * F.linear(x, w_up.to(x.dtype)), w_down.to(x.dtype))
+    """The MLP through differentiable functions, on weights of x's dtype."""
+    return F.linear(F.silu(F.linear(x, w_gate)) * F.linear(x, w_up), w_down)
 
 
 def mlp_layer(x: Tensor, w_gate: nn.Linear, w_up: nn.Linear, w_down: nn.Linear) -> Tensor:

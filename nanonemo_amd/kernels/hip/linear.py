@@ -64,29 +64,45 @@ def stacked(grads: tuple[Tensor | None, ...], rows: list[int], like: Tensor) -> 
     return torch.cat([like.new_zeros(like.shape[0], r) if g is None else g for g, r in zip(grads, rows)], dim=1)
 
 
+class Stored(torch.autograd.Function):
+    """The 16-bit copy that a forward made of a weight, as a function of the weight. A recorded backward computes with it:
+    its derivatives reach the parameter, and its values are the forward's whatever has become of the parameter since
+    (the nodes do not save the fp32 parameters, so changing one between forward and backward is no error, as with
+    autocast's nn.Linear, which keeps the same copy)."""
+
+    @staticmethod
+    def forward(ctx, w, copy):
+        return copy.detach()
+
+    @staticmethod
+    def backward(ctx, g):
+        return g.float(), None
+
+
 class _Projections(torch.autograd.Function):
     """y_i = x W_i^T: x (T, K) 16-bit, W_i fp32, y_i the column ranges of one (T, sum N_i) product."""
 
     @staticmethod
     def forward(ctx, x, turned, *ws):
         y, w16 = host().project_fwd(x, ws, turned)
-        ctx.save_for_backward(x, w16, *ws)
+        ctx.save_for_backward(x, w16)
+        ctx.weights = ws
         ctx.set_materialize_grads(False)
         return (y,) if len(ws) == 1 else y.split([w.shape[0] for w in ws], dim=1)
 
     @staticmethod
     def backward(ctx, *dys):
-        x, w16, *ws = ctx.saved_tensors
-        rows = [w.shape[0] for w in ws]
+        x, w16 = ctx.saved_tensors
+        rows = [w.shape[0] for w in ctx.weights]
         need_w = any(ctx.needs_input_grad[2:])
         dy = stacked(dys, rows, x)
         if torch.is_grad_enabled():  # a recorded backward
-            wd = torch.cat([w.to(x.dtype) for w in ws])
+            wd = torch.cat([Stored.apply(w, c) for w, c in zip(ctx.weights, w16.split(rows))])
             dx = dy @ wd if ctx.needs_input_grad[0] else None
-            dws = (dy.t() @ x).float().split(rows) if need_w else [None] * len(ws)
+            dws = (dy.t() @ x).float().split(rows) if need_w else [None] * len(rows)
         else:
             dx = dy @ w16 if ctx.needs_input_grad[0] else None
-            dws = wgrad(dy, x, rows) if need_w else [None] * len(ws)
+            dws = wgrad(dy, x, rows) if need_w else [None] * len(rows)
         return dx, None, *(g if n else None for g, n in zip(dws, ctx.needs_input_grad[2:]))
 
 

@@ -69,6 +69,44 @@ def test_head_loss_keeps_nothing_past_its_backward(host):
     (g2,) = torch.autograd.grad(loss, m.weight)
     assert host.recomputed
     torch.testing.assert_close(g1, g2)
-    assert not any(isinstance(v, torch.Tensor) and v.numel() >= logits.numel() for v in vars(node).values())
+    assert not any(isinstance(v, torch.Tensor) and v is not m.weight for v in vars(node).values())
     with pytest.raises(RuntimeError, match="freed"):
         node.saved_tensors
+
+
+def _mlp(d=16, ff=24):
+    torch.manual_seed(0)
+    gate, up, down = nn.Linear(d, ff, bias=False), nn.Linear(d, ff, bias=False), nn.Linear(ff, d, bias=False)
+    return torch.randn(3, 5, d, dtype=torch.bfloat16).requires_grad_(), (gate, up, down)
+
+
+def _calls():
+    """The fused calls: (output, its input, its layers)."""
+    from nanonemo_amd.kernels.hip import head, layers, linear
+
+    x, ws = _mlp()
+    yield "mlp", lambda: layers.mlp_layer(x, *ws), x, ws
+    yield "projections", lambda: torch.cat(linear.projections(x, *ws[:2]), -1), x, ws[:2]
+    yield "projection", lambda: linear.projections(x, ws[0])[0], x, ws[:1]
+    t = torch.randint(0, 24, (3, 5))
+    yield "head", lambda: head.head_loss(x, ws[0], t)[1], x, ws[:1]
+
+
+def test_weights_may_change_between_forward_and_backward(host):
+    # As with autocast's nn.Linear, which keeps 16-bit copies: the backward, recorded or not, is the forward's.
+    for name, f, x, ws in _calls():
+        params = [m.weight for m in ws]
+        ref = torch.autograd.grad(f().float().sum(), (x, *params))
+        for recorded in (False, True):
+            out, kept = f().float().sum(), [p.detach().clone() for p in params]
+            with torch.no_grad():
+                for p in params:
+                    p.mul_(1.5)
+            got = torch.autograd.grad(out, (x, *params), create_graph=recorded)
+            with torch.no_grad():
+                for p, k in zip(params, kept):
+                    p.copy_(k)
+            for a, b in zip(got, ref):
+                torch.testing.assert_close(a, b, rtol=2e-2, atol=2e-2 * b.abs().max().item(), msg=f"{name} {recorded}")
+            if recorded:  # and second derivatives reach the parameters
+                assert any(g is not None for g in torch.autograd.grad(got[0].float().square().sum(), params, allow_unused=True)), name
