@@ -574,6 +574,21 @@ std::vector<OptTensor> head_bwd(const OptTensor& dlogits_, const OptTensor& dlos
 
 // ---- routing ------------------------------------------------------------------------------------
 
+// Whether the tensor's values lie at its address, as dense values of its own type: not inside a transform's wrapper
+// (vmap, is_grads_batched, torch.func.grad, functionalization), not a lazy zero, negation or conjugate, not sparse,
+// nested or a subclass with its own dispatch.
+bool ordinary(const Tensor& t) {
+    using K = c10::DispatchKey;
+    static constexpr c10::DispatchKeySet wrapped({K::Python, K::Batched, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Functionalize,
+                                                  K::ZeroTensor, K::Negative, K::Conjugate});
+    return !t.key_set().has_any(wrapped) && !t.is_nested() && t.layout() == at::kStrided;
+}
+bool ordinary_py(const py::args& ts) {
+    for (py::handle t : ts)
+        if (!ordinary(THPVariable_Unpack(t.ptr()))) return false;
+    return true;
+}
+
 // Whether every argument is a plain CUDA tensor and neither a torch.func transform nor a Python dispatch mode is
 // active (see kernels/hip/__init__.py, eager).
 bool plain_cuda(const py::args& ts) {
@@ -638,6 +653,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("head_fwd", head_fwd, nogil);
     m.def("head_bwd", head_bwd, nogil);
     m.def("plain_cuda", plain_cuda);
+    m.def("ordinary", ordinary_py);
     // A tensor's version counter (which its changes in place raise), without the tensor.
     py::class_<c10::VariableVersion>(m, "Version")
         .def(py::init([](const Tensor& t) { return t.unsafeGetTensorImpl()->version_counter(); }))

@@ -40,7 +40,7 @@ class _HeadLoss(torch.autograd.Function):
     def backward(ctx, dlogits, dloss):
         x, w16, targets, lse, inv, logits = ctx.saved_tensors
         need_x, need_w = ctx.needs_input_grad[:2]
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not host().ordinary(*(g for g in (dlogits, dloss) if g is not None)):
             return *_replayed(x, ctx.weight, w16, targets, (need_x, need_w), dlogits, dloss), None
         if ctx.version.current() != ctx.at:
             logits = None
@@ -48,7 +48,8 @@ class _HeadLoss(torch.autograd.Function):
 
 
 def _replayed(x, w, w16, targets, need, dlogits, dloss):
-    """The gradients as recorded operations on the forward's 16-bit copy of the weight."""
+    """The gradients as torch operations, recorded if the backward is, on the forward's 16-bit copy of the weight."""
+    record = torch.is_grad_enabled()
     with torch.enable_grad():
         logits = F.linear(x, Stored.apply(w, w16))
         outs, grads = [], []
@@ -58,7 +59,7 @@ def _replayed(x, w, w16, targets, need, dlogits, dloss):
             outs.append(F.cross_entropy(logits.float(), targets)), grads.append(dloss)
         if not outs:
             return None, None, None
-        found = iter(torch.autograd.grad(outs, [t for t, n in zip((x, w), need) if n], grads, create_graph=True))
+        found = iter(torch.autograd.grad(outs, [t for t, n in zip((x, w), need) if n], grads, create_graph=record))
     return next(found) if need[0] else None, next(found) if need[1] else None, None
 
 

@@ -17,8 +17,9 @@ A layer's weights are rounded to 16 bits in one launch at the start of its forwa
 (``turned``), a transposed copy is written beside them, which the products for the inputs' gradients read.
 
 ``can_fuse`` and ``can_fuse_mlp`` hold for the calls that ``linear.can_project`` describes, with every module of the layer
-untouched; the others run module by module. A backward that is itself recorded replays the layer through PyTorch's linear
-layers and the package's differentiable functions, so that what those support is what it supports.
+untouched; the others run module by module. A backward that is itself recorded, or is handed gradients that the kernels
+cannot read by address (is_grads_batched), replays the layer through PyTorch's linear layers and the package's
+differentiable functions, so that what those support is what it supports.
 """
 
 from __future__ import annotations
@@ -64,7 +65,7 @@ class _AttentionLayer(torch.autograd.Function):
         _refuse_capture_with_autograd("attention layer backward")
         x, cos, sin, qkv, q, o, lse, w, wo16 = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not host().ordinary(dy):
             copies = (*w.split([m.shape[0] for m in ctx.weights[:3]]), wo16)
             dx, *dws = _replayed(_modular, x, ctx.weights, copies, (need[0], *need[7:11]), dy, (cos, sin, *ctx.sizes))
             return dx, None, None, None, None, None, None, *dws, None
@@ -81,10 +82,12 @@ def _modular(x, wq, wk, wv, wo, cos, sin, B, T, H, KVH):
 
 
 def _replayed(fn, x, weights, copies, need, dy, extra=()) -> list:
-    """The gradients of fn(x, *weights, *extra) as recorded operations on the forward's 16-bit copies of the weights."""
+    """The gradients of fn(x, *weights, *extra) as torch operations, recorded if the backward is, on the forward's 16-bit
+    copies of the weights."""
+    record = torch.is_grad_enabled()
     with torch.enable_grad():
         y = fn(x, *(Stored.apply(w, c) for w, c in zip(weights, copies)), *extra)
-        grads = iter(torch.autograd.grad(y, [t for t, n in zip((x, *weights), need) if n], dy, create_graph=True))
+        grads = iter(torch.autograd.grad(y, [t for t, n in zip((x, *weights), need) if n], dy, create_graph=record))
     return [next(grads) if n else None for n in need]
 
 
@@ -122,7 +125,7 @@ class _MlpLayer(torch.autograd.Function):
     def backward(ctx, dy):
         x, gu, h, w, wd = ctx.saved_tensors
         need = ctx.needs_input_grad[:4]
-        if torch.is_grad_enabled():
+        if torch.is_grad_enabled() or not host().ordinary(dy):
             return *_replayed(_modular_mlp, x, ctx.weights, (*w.chunk(2), wd), need, dy), None
         grads = host().mlp_bwd(dy, x, gu, h, w, wd, need[0], need[1] or need[2], need[3])
         return *(g if n else None for g, n in zip(grads, need)), None

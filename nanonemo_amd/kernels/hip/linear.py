@@ -11,7 +11,8 @@ which 10 would do).
 ``can_project(x, layers)`` says whether the call can take this path: plain CUDA tensors and untouched fp32
 ``nn.Linear`` layers under 16-bit autocast, in eager mode. Everything else (hooks, parametrizations, other module or
 tensor types, torch.compile, torch.func, forward-mode AD, no autocast) keeps calling the modules. A backward that is
-itself recorded (create_graph) runs differentiable torch products instead of the kernel.
+itself recorded (create_graph), or is handed gradients that the kernel cannot read by address (is_grads_batched), runs
+differentiable torch products instead of the kernel.
 """
 
 from __future__ import annotations
@@ -96,7 +97,7 @@ class _Projections(torch.autograd.Function):
         rows = [w.shape[0] for w in ctx.weights]
         need_w = any(ctx.needs_input_grad[2:])
         dy = stacked(dys, rows, x)
-        if torch.is_grad_enabled():  # a recorded backward
+        if torch.is_grad_enabled() or not host().ordinary(dy):  # a recorded backward, or batched gradients
             wd = torch.cat([Stored.apply(w, c) for w, c in zip(ctx.weights, w16.split(rows))])
             dx = dy @ wd if ctx.needs_input_grad[0] else None
             dws = (dy.t() @ x).float().split(rows) if need_w else [None] * len(rows)

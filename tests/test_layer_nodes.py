@@ -110,3 +110,31 @@ def test_weights_may_change_between_forward_and_backward(host):
                 torch.testing.assert_close(a, b, rtol=2e-2, atol=2e-2 * b.abs().max().item(), msg=f"{name} {recorded}")
             if recorded:  # and second derivatives reach the parameters
                 assert any(g is not None for g in torch.autograd.grad(got[0].float().square().sum(), params, allow_unused=True)), name
+
+
+def test_batched_gradients_pass_through_the_layers(host):
+    # torch.autograd.grad(..., is_grads_batched=True) hands the backward tensors without storage of their own: they take
+    # the replay, as they took the modules' backward.
+    for name, f, x, ws in _calls():
+        ins = (x, *(m.weight for m in ws))
+        y = f()
+        dys = torch.randn(4, *y.shape, dtype=y.dtype) if y.dim() else torch.tensor([0.5, -1.0, 2.0])
+        got = torch.autograd.grad(y, ins, dys, is_grads_batched=True, retain_graph=True)
+        for i, dy in enumerate(dys):
+            for a, b in zip(got, torch.autograd.grad(y, ins, dy, retain_graph=True)):
+                torch.testing.assert_close(a[i], b, rtol=2e-2, atol=2e-2 * b.abs().max().item(), msg=name)
+
+
+def test_ordinary_tells_tensors_that_can_be_read_by_address():
+    from nanonemo_amd.kernels.hip import host
+
+    o = host().ordinary
+    t = torch.randn(3, 4)
+    assert o(t) and o(t.t()) and o(t.requires_grad_()) and o()
+    assert not o(torch._efficientzerotensor(3)) and not o(torch.nested.nested_tensor([t.detach(), t.detach()])) and not o(t.detach().to_sparse())
+    assert not o(torch.randn(3, dtype=torch.complex64).conj().imag) and not o(t, torch.randn(3, dtype=torch.complex64).conj())
+    seen = []
+    torch.func.vmap(lambda a: seen.append(o(a)) or a)(t.detach())
+    torch.func.grad(lambda a: seen.append(o(a)) or a.sum())(t.detach())
+    torch._vmap_internals._vmap(lambda a: seen.append(o(a)) or a, 0)(t.detach())
+    assert seen == [False, False, False]
