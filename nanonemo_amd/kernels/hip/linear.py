@@ -10,9 +10,9 @@ which 10 would do).
 
 ``can_project(x, layers)`` says whether the call can take this path: plain CUDA tensors and untouched fp32
 ``nn.Linear`` layers under 16-bit autocast, in eager mode. Everything else (hooks, parametrizations, other module or
-tensor types, torch.compile, torch.func, forward-mode AD, no autocast) keeps calling the modules. A backward that is
-itself recorded (create_graph), or is handed gradients that the kernel cannot read by address (is_grads_batched), runs
-differentiable torch products instead of the kernel.
+tensor types, torch.compile, torch.func, dispatch and function modes, forward-mode AD, no autocast) keeps calling the
+modules. A backward that is itself recorded (create_graph), or is handed gradients that the kernel cannot read by
+address (is_grads_batched), runs differentiable torch products instead of the kernel.
 """
 
 from __future__ import annotations
@@ -21,6 +21,7 @@ import torch
 from torch import Tensor, nn
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
+from torch.utils._device import DeviceContext
 
 from nanonemo_amd.kernels.hip import eager, host, records
 
@@ -39,13 +40,18 @@ def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
             and w.shape[1] == width and (odd_rows or w.shape[0] % 8 == 0) and width % 8 == 0 and w.data_ptr() % 16 == 0)
 
 
+def function_mode() -> bool:
+    """Whether a TorchFunctionMode is active that may intercept the modules' functions (torch.device's does not)."""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 def eligible(x: Tensor) -> bool:
     """Whether a layer called on x now may run on this build's kernels (see above), whatever its modules."""
     if not eager(x) or not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") not in _DTYPES:
         return False
     if x.dim() < 2 or x.numel() == 0 or not x.is_floating_point() or x.dtype is torch.float64:
         return False
-    return not (torch.jit.is_tracing() or forward_ad._current_level >= 0 or _module._has_any_global_hook())
+    return not (torch.jit.is_tracing() or function_mode() or forward_ad._current_level >= 0 or _module._has_any_global_hook())
 
 
 def can_project(x: Tensor, *layers: nn.Module) -> bool:

@@ -138,3 +138,21 @@ def test_ordinary_tells_tensors_that_can_be_read_by_address():
     torch.func.grad(lambda a: seen.append(o(a)) or a.sum())(t.detach())
     torch._vmap_internals._vmap(lambda a: seen.append(o(a)) or a, 0)(t.detach())
     assert seen == [False, False, False]
+
+
+def test_function_modes_see_the_modules():
+    # A TorchFunctionMode may replace F.linear or F.cross_entropy: the layers then run module by module. The mode behind
+    # torch.set_default_device and `with torch.device(...)` replaces factories only.
+    from nanonemo_amd.kernels.hip import linear
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not linear.function_mode()
+    with torch.device("cpu"):
+        assert not linear.function_mode()
+        with Mode():
+            assert linear.function_mode()
+    with Mode():
+        assert linear.function_mode()
