@@ -589,11 +589,12 @@ bool ordinary_py(const py::args& ts) {
     return true;
 }
 
-// Whether every argument is a plain CUDA tensor and neither a torch.func transform nor a Python dispatch mode is
+// Whether every argument is a plain (ordinary, no subclass) CUDA tensor and neither a torch.func transform nor a Python dispatch mode is
 // active (see kernels/hip/__init__.py, eager).
 bool plain_cuda(const py::args& ts) {
     for (py::handle t : ts)
-        if (!THPVariable_CheckExact(t.ptr()) || !THPVariable_Unpack(t.ptr()).is_cuda()) return false;
+        if (!THPVariable_CheckExact(t.ptr()) || !THPVariable_Unpack(t.ptr()).is_cuda() || !ordinary(THPVariable_Unpack(t.ptr())))
+            return false;
     // (a torch.func transform puts its key into the thread's set while its stack is not empty)
     return c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
            !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);

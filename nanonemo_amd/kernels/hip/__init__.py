@@ -169,7 +169,8 @@ def eager(*ts) -> bool:
     host time per forward + backward; the eager paths call the same launch code, so their results are the same
     bits. True only for plain CUDA tensors outside torch.compile tracing, torch.func transforms and dispatch modes,
     which need the ops (an opaque traced node, a transform rule, the op visible to the mode); meta and CPU tensors
-    take the ops too, whose fake impls and checks handle them."""
+    take the ops too, whose fake impls and checks handle them, and so do sparse, nested and lazily negated ones, which the
+    dispatcher resolves or refuses."""
     import torch
 
     return not torch.compiler.is_compiling() and host().plain_cuda(*ts)

@@ -110,6 +110,7 @@ def test_only_untouched_layers_under_autocast_take_the_path():
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert linear.can_project(x, m)
         assert not linear.can_project(x.cpu(), m) and not linear.can_project(x.double(), m) and not linear.can_project(x[:0], m)
+        assert not linear.can_project(torch.nested.nested_tensor([x, x]), m)
         h = m.register_forward_hook(lambda *_: None)
         assert not linear.can_project(x, m)
         h.remove()
