@@ -69,6 +69,12 @@ Tensor empty_f32(const Tensor& like, at::IntArrayRef shape) { return at::empty(s
 Tensor bytes(const Tensor& like, size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
 float scale_of(int64_t D) { return (float)(1.0 / std::sqrt((double)D)); }
 
+// The library reads raw addresses on x's device.
+void check_on_device(const Tensor& x, std::initializer_list<const Tensor*> others) {
+    need(x.is_cuda(), "inputs must be CUDA tensors");
+    for (const Tensor* t : others) need(t->device() == x.device(), "inputs must be CUDA tensors on the same device");
+}
+
 // ---- attention ----------------------------------------------------------------------------------
 
 // The reference's check_inputs (flash_attn.cu:342-356) with the dtypes widened to {fp16, bf16}. seq is 2 for
@@ -249,6 +255,7 @@ void refuse_capture_from_engine(const char* where) {
 }
 void check_backward(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, int seq) {
     check_attention(q, k, v, seq);
+    check_on_device(q, {&d_o, &o, &lse});
     need(d_o.sizes() == q.sizes() && d_o.scalar_type() == q.scalar_type() && o.sizes() == q.sizes() && o.scalar_type() == q.scalar_type(),
          "d_o must be a contiguous float16/bfloat16 tensor shaped like q");
     need(lse.sizes() == at::IntArrayRef({q.size(0), q.size(3 - seq), q.size(seq)}) && lse.scalar_type() == at::kFloat,
@@ -280,7 +287,7 @@ T3 bthd_rope_bwd_op(const Tensor& d_o, const Tensor& q_, const Tensor& k_, const
 // ---- RoPE ---------------------------------------------------------------------------------------
 
 T2 rope(const Tensor& q_, const Tensor& k_, const Tensor& cos_, const Tensor& sin_, bool inverse) {
-    need(q_.is_cuda() && k_.is_cuda() && cos_.is_cuda() && sin_.is_cuda(), "inputs must be CUDA tensors");
+    check_on_device(q_, {&k_, &cos_, &sin_});
     need(q_.dim() == 4 && k_.dim() == 4 && q_.size(0) == k_.size(0) && q_.size(1) == k_.size(1) && q_.size(3) == k_.size(3),
          "expected q (B, T, H, hd) and k (B, T, KVH, hd)");
     need(code(q_) >= 0 && k_.scalar_type() == q_.scalar_type(), "q and k must share a dtype in {float16, bfloat16, float32}");
@@ -313,6 +320,7 @@ int norm_code(at::ScalarType t) {
 T3 norm_fwd(const Tensor& x_, const OptTensor& delta_, const Tensor& weight_, double eps, at::ScalarType out_dtype) {
     need(x_.is_cuda(), "x must be a CUDA tensor");
     const bool has = delta_.has_value();
+    check_on_device(x_, {&weight_, has ? &*delta_ : &x_});
     const Tensor x = contig(x_), w = contig(weight_), delta = has ? contig(*delta_) : Tensor();
     need(w.scalar_type() == at::kFloat, "weight must be contiguous float32");
     if (has) need(delta.sizes() == x.sizes(), "delta must match x");
@@ -332,11 +340,13 @@ T3 norm_fwd(const Tensor& x_, const OptTensor& delta_, const Tensor& weight_, do
 T3 norm_bwd(const Tensor& dy_, const OptTensor& dh_, const Tensor& h_, const Tensor& weight_, const Tensor& rstd_,
             at::ScalarType dx_dtype, std::optional<at::ScalarType> ddelta_dtype) {
     const bool has = dh_.has_value();
+    check_on_device(h_, {&dy_, &weight_, &rstd_, has ? &*dh_ : &h_});
     const Tensor dy = contig(dy_), h = contig(h_), w = contig(weight_), rstd = contig(rstd_), dh = has ? contig(*dh_) : Tensor();
     need(dy.sizes() == h.sizes(), "dy and h must be contiguous, same shape");
     need(has == ddelta_dtype.has_value(), "dh and ddelta_dtype go together");
     if (has) need(dh.scalar_type() == h.scalar_type(), "dh must be contiguous, h's dtype");
     const int64_t N = h.size(-1), M = N ? h.numel() / N : 0;
+    need(w.numel() == N && (N == 0 || rstd.numel() == M), "weight must have hidden-size elements and rstd one per row");
     Tensor dx = at::empty(h.sizes(), h.options().dtype(dx_dtype));
     Tensor dd = has ? at::empty(h.sizes(), h.options().dtype(*ddelta_dtype)) : empty_of(h, {0});
     Tensor dw = empty_f32(h, {N});

@@ -534,3 +534,13 @@ def test_eager_path_routing_without_a_gpu():
     assert records(cpu, g) and not records(cpu)
     with torch.no_grad():
         assert not records(g)
+
+
+def test_norm_backward_op_refuses_host_tensors():
+    # Before anything is allocated or launched: the library would read host addresses on the GPU.
+    from nanonemo_amd.kernels.hip import rmsnorm  # noqa: F401  (registers the ops)
+
+    t, w, r = torch.ones(4, 64), torch.ones(64), torch.ones(4)
+    for dh in (None, t):
+        with pytest.raises(RuntimeError, match="must be CUDA tensors"):
+            torch.ops.nanonemo.cuda_add_rms_norm_bwd(t, dh, t, w, r, torch.float32, None if dh is None else torch.float32)

@@ -203,3 +203,36 @@ def test_eager_path_under_activation_checkpointing():
     gb = torch.autograd.grad(checkpoint(fa.flash_attn_bthd, *b, use_reentrant=False), b, do)
     for x, y in zip(ga, gb):
         assert torch.equal(x, y)
+
+
+def test_tensors_of_another_device_are_refused_before_any_launch():
+    # the library would read a host address on the GPU
+    import nanonemo_amd.kernels.hip.flash_attn as fa
+    from nanonemo_amd.kernels.hip import rmsnorm, rope  # noqa: F401
+    from nanonemo_amd.model import rope_tables
+
+    ops, f32 = torch.ops.nanonemo, torch.float32
+    x, w = torch.randn(8, 64, device=DEV), torch.ones(64, device=DEV)
+    with pytest.raises(RuntimeError, match="CUDA tensors"):
+        rmsnorm.add_rms_norm(x, None, w.cpu(), 1e-5)
+    with pytest.raises(RuntimeError, match="CUDA tensors"):
+        rmsnorm.add_rms_norm(x, x.cpu(), w, 1e-5)
+    r = torch.ones(8, device=DEV)
+    for bad in range(5):
+        a = [t.cpu() if i == bad else t for i, t in enumerate((x, x, x, w, r))]
+        with pytest.raises(RuntimeError, match="CUDA tensors"):
+            ops.cuda_add_rms_norm_bwd(*a, f32, f32)
+    with pytest.raises(RuntimeError, match="one per row"):
+        ops.cuda_add_rms_norm_bwd(x, x, x, w, r[:4], f32, f32)
+    q = torch.randn(1, 2, 16, 64, device=DEV).bfloat16()
+    o, lse = ops.flash_attn(q, q, q)
+    for bad in ((q.cpu(), o, lse), (q, o.cpu(), lse), (q, o, lse.cpu())):
+        with pytest.raises(RuntimeError, match="CUDA tensors"):
+            ops.flash_attn_bwd(bad[0], q, q, q, *bad[1:])
+    t = q.transpose(1, 2).contiguous()
+    cos, sin = rope_tables(64, 16, 10000.0)  # host tables
+    for f in (lambda: rope.rope_qk(t, t, cos, sin), lambda: rope.rope_qk(t, t, cos.to(DEV), sin), lambda: fa.flash_attn_bthd_rope(t, t, t, cos, sin),
+              lambda: fa.flash_attn_bthd_rope(t, t, t, cos.to(DEV), sin), lambda: ops.flash_attn_bthd_rope(t, t, t, cos, sin),
+              lambda: ops.flash_attn_bthd_rope_bwd(t, t, t, t, t, lse, cos, sin)):
+        with pytest.raises(RuntimeError, match="CUDA tensors|inputs' device"):
+            f()
