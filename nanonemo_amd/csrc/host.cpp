@@ -22,6 +22,7 @@
 
 #include <array>
 #include <cmath>
+#include <functional>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -246,9 +247,10 @@ T3 bthd_rope_bwd(const Tensor& d_o_, const Tensor& q_, const Tensor& k_, const T
 
 // The backward ops as the dispatcher calls them. A capture of the autograd engine's backward is refused (such a capture
 // once ended in a host fault and no cause has been shown); capture without autograd is not affected.
-void refuse_capture_from_engine(const char* where) {
-    if (!torch::autograd::get_current_node() || c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None) return;
-    raise(std::string(where) + ": capturing this op into a HIP graph while autograd records it (torch.cuda.graph around the "
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+void refuse_capture_from_engine(const std::string& where, const std::function<bool()>& captures = capturing) {
+    if (!torch::autograd::get_current_node() || !captures()) return;
+    raise(where + ": capturing this op into a HIP graph while autograd records it (torch.cuda.graph around the "
           "forward and its autograd backward, or torch.compile(mode='reduce-overhead')) is not supported: such a capture once "
           "ended in a host fault in capture_end and no cause has been shown. Capture the C ABI calls (nn_fa_fwd / nn_fa_bwd / "
           "nn_fa_bwd_noalloc) instead, or run the ops eagerly (torch.compile(fullgraph=True) without graphs is supported).");
@@ -669,6 +671,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::class_<c10::VariableVersion>(m, "Version")
         .def(py::init([](const Tensor& t) { return t.unsafeGetTensorImpl()->version_counter(); }))
         .def("current", &c10::VariableVersion::current_version);
+    m.def("check_tables", check_tables);
+    m.def("refuse_capture_from_engine", [](const std::string& where, bool captures) {
+        refuse_capture_from_engine(where, [captures] { return captures; });
+    });
     m.def("strides_of", strides_py);
     m.def("readable", readable_py, py::arg("a"), py::arg("b") = std::nullopt);
 }

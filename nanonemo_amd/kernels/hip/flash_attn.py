@@ -55,13 +55,6 @@ def _refuse_capture_with_autograd(where: str, *inputs: Tensor) -> None:
     raise RuntimeError(_CAPTURE_MSG.format(where))
 
 
-def _refuse_capture_from_autograd_engine(where: str) -> None:
-    """In the backward ops' bodies: raise when the autograd engine runs them (directly, or inside a compiled
-    backward such as torch.compile's mode='reduce-overhead' records) while the current stream is capturing."""
-    if torch._C._current_autograd_node() is not None:
-        _refuse_capture_with_autograd(where)
-
-
 @torch.library.custom_op("nanonemo::flash_attn", mutates_args=())
 def _flash_attn(q: Tensor, k: Tensor, v: Tensor) -> tuple[Tensor, Tensor]:
     return host().fa_fwd(q, k, v)
@@ -78,7 +71,6 @@ def _(q, k, v):
 
 @torch.library.custom_op("nanonemo::flash_attn_bwd", mutates_args=())
 def _flash_attn_bwd(d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    _refuse_capture_from_autograd_engine("flash_attn backward op")
     return host().fa_bwd_op(d_o, q, k, v, o, lse)
 
 
@@ -178,7 +170,6 @@ def _(q, k, v):
 def _flash_attn_bthd_bwd(
     d_o: Tensor, q: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor
 ) -> tuple[Tensor, Tensor, Tensor]:
-    _refuse_capture_from_autograd_engine("flash_attn_bthd backward op")
     return host().bthd_bwd_op(d_o, q, k, v, o, lse)
 
 
@@ -236,21 +227,8 @@ def flash_attn_bthd(q: Tensor, k: Tensor, v: Tensor) -> Tensor:
 # output are not propagated (the model uses neither), as the reference ignores lse's.
 
 
-def _check_tables(cos: Tensor, sin: Tensor, T: int, D: int, device: torch.device) -> tuple[Tensor, Tensor]:
-    """The RoPE tables: float32 (T_max >= T, hd/2), on the inputs' GPU. Checked before any launch, since the
-    library reads them through raw device pointers (a host table would be read as device memory)."""
-    if not (cos.is_cuda and sin.is_cuda) or cos.device != device or sin.device != device:
-        raise RuntimeError("cos/sin must be float32 (T_max >= T, hd/2) tables on the inputs' device")
-    if cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape or cos.dim() != 2 \
-            or cos.shape[1] != D // 2 or cos.shape[0] < T:
-        raise RuntimeError("cos/sin must be float32 (T_max >= T, hd/2) tables on the inputs' device")
-    return _contig(cos), _contig(sin)
-
-
 @torch.library.custom_op("nanonemo::flash_attn_bthd_rope", mutates_args=())
 def _flash_attn_bthd_rope(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, Tensor, Tensor]:
-    if q.is_cuda:
-        cos, sin = _check_tables(cos, sin, q.size(1), q.size(3), q.device)
     return host().bthd_rope_fwd(q, k, v, cos, sin)
 
 
@@ -268,7 +246,6 @@ def _(q, k, v, cos, sin):
 def _flash_attn_bthd_rope_bwd(
     d_o: Tensor, q_rot: Tensor, k: Tensor, v: Tensor, o: Tensor, lse: Tensor, cos: Tensor, sin: Tensor
 ) -> tuple[Tensor, Tensor, Tensor]:
-    _refuse_capture_from_autograd_engine("flash_attn_bthd_rope backward op")
     return host().bthd_rope_bwd_op(d_o, q_rot, k, v, o, lse, cos, sin)
 
 

@@ -490,37 +490,37 @@ def test_capture_guard_is_off_when_not_capturing():
 
 def test_rope_fused_ops_reject_host_tables():
     # cos / sin must be GPU tensors on q's device; a host table would reach the library as a host address.
-    from nanonemo_amd.kernels.hip import flash_attn as fa
+    from nanonemo_amd.kernels.hip import host
 
     cos = torch.zeros(8, 32)
     with pytest.raises(RuntimeError, match="inputs' device"):
-        fa._check_tables(cos, cos, 8, 64, torch.device("cuda", 0))
+        host().check_tables(cos, cos, 8, 64, torch.device("cuda", 0))
     with pytest.raises(RuntimeError, match="inputs' device"):
-        fa._check_tables(cos, cos.clone(), 8, 64, torch.device("cpu"))  # CPU "inputs" still need CUDA tables
+        host().check_tables(cos, cos.clone(), 8, 64, torch.device("cpu"))  # CPU "inputs" still need CUDA tables
 
 
-def test_backward_ops_refuse_capture_only_inside_the_autograd_engine(monkeypatch):
+def test_backward_ops_refuse_capture_only_inside_the_autograd_engine():
     # The backward ops' own guard: a capture driven by the autograd engine (eager autograd, or a compiled backward
     # as mode="reduce-overhead" records) is refused; the same call outside the engine is not (a manual op pair).
-    from nanonemo_amd.kernels.hip import flash_attn as fa
+    from nanonemo_amd.kernels.hip import host
 
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
-    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
-    fa._refuse_capture_from_autograd_engine("outside the engine")  # returns
+    host().refuse_capture_from_engine("outside the engine", True)  # returns
 
     class F(torch.autograd.Function):
         @staticmethod
-        def forward(ctx, a):
+        def forward(ctx, a, captures):
+            ctx.captures = captures
             return a * 2
 
         @staticmethod
         def backward(ctx, g):
-            fa._refuse_capture_from_autograd_engine("inside the engine")
-            return g
+            host().refuse_capture_from_engine("inside the engine", ctx.captures)
+            return g, None
 
     x = torch.ones(3, requires_grad=True)
+    F.apply(x, False).sum().backward()  # not capturing
     with pytest.raises(RuntimeError, match="inside the engine: capturing"):
-        F.apply(x).sum().backward()
+        F.apply(x, True).sum().backward()
 
 
 def test_eager_path_routing_without_a_gpu():
