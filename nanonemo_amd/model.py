@@ -224,13 +224,20 @@ class MLP(nn.Module):
         self.w_down = nn.Linear(cfg.d_ff, cfg.d_model, bias=False)
         self.any_hip = cfg.any_hip and cfg.d_model % 8 == 0 and cfg.d_ff % 8 == 0  # (the kernels' rows of 16-byte vectors)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if self.any_hip and x.is_cuda:
-            from nanonemo_amd.kernels.hip import layers
+    @torch.jit.unused
+    def _fused(self, x: torch.Tensor) -> torch.Tensor | None:
+        """The whole MLP in this build's kernels, as one autograd node, for the calls that can be."""
+        from nanonemo_amd.kernels.hip import layers
 
-            ws = (self.w_gate, self.w_up, self.w_down)
-            if layers.can_fuse_mlp(x, *ws):
-                return layers.mlp_layer(x, *ws)
+        ws = (self.w_gate, self.w_up, self.w_down)
+        return layers.mlp_layer(x, *ws) if layers.can_fuse_mlp(x, *ws) else None
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        # (a scripted module, and one traced symbolically, whose x is no tensor, is the modules)
+        if not torch.jit.is_scripting() and self.any_hip and isinstance(x, torch.Tensor) and x.is_cuda:
+            y = self._fused(x)
+            if y is not None:
+                return y
         return self.w_down(F.silu(self.w_gate(x)) * self.w_up(x))
 
 

@@ -123,3 +123,15 @@ def test_unknown_attention_kernel_is_rejected():
 def test_unknown_neighbour_kernel_is_rejected(field):
     with pytest.raises(ValueError):
         ModelConfig(**{field: "triton"})
+
+
+@pytest.mark.parametrize("kw", [{}, dict(attn_kernel="hip")])
+@pytest.mark.parametrize("how", ["script", "symbolic_trace"])
+def test_mlp_can_be_scripted_and_traced_symbolically(how, kw):
+    # both are the modules, whatever kernels an eager call would take
+    from nanonemo_amd.model import MLP
+
+    m = MLP(ModelConfig(**SMALL, **kw))
+    x = torch.randn(3, SMALL["d_model"])
+    got = torch.jit.script(m) if how == "script" else torch.fx.symbolic_trace(m)
+    assert torch.equal(got(x), m(x))
