@@ -382,16 +382,18 @@ Tensor rows_aligned(const Tensor& t) {
 }
 
 std::vector<Tensor> wgrad(const Tensor& dy_, const Tensor& x_, const std::vector<int64_t>& rows) {
-    const Tensor dy = rows_aligned(dy_), x = rows_aligned(x_);
-    const int64_t T = dy.size(0), N = dy.size(1), K = x.size(1);
-    const c10::DeviceGuard guard(x.device());
+    const int64_t T = dy_.size(0), N = dy_.size(1), K = x_.size(1);
+    const c10::DeviceGuard guard(x_.device());
     if (N * K > kWgradMost || N % 8) {
-        Tensor dw = at::mm(dy.t(), x, at::kFloat);
+        // (dense rows are the library's to read whatever their width; an odd vocabulary's are not 16-byte aligned)
+        auto dense = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0 ? t : rows_aligned(t); };
+        Tensor dw = at::mm(dense(dy_).t(), dense(x_), at::kFloat);
         if (rows.size() == 1) return {dw};
         std::vector<Tensor> out = dw.split_with_sizes(rows);
         for (Tensor& t : out) t = t.clone();
         return out;
     }
+    const Tensor dy = rows_aligned(dy_), x = rows_aligned(x_);
     std::vector<Tensor> out;
     std::vector<float*> p;
     for (int64_t r : rows) {

@@ -37,6 +37,25 @@ def test_wgrad_matches_float64(T, N, K, dtype):
     assert ((got.double() - ref).abs() <= bound).all()
 
 
+def test_wgrad_of_an_odd_number_of_columns_copies_nothing():
+    # the output layer's gradient for a vocabulary that is no multiple of 8: 0.8 GB at 8192 x 50257
+    from nanonemo_amd.kernels.hip.linear import wgrad
+
+    T, N, K = 2048, 4099, 64
+    dy, x = (torch.randn(T, n, device="cuda").bfloat16() for n in (N, K))
+    wgrad(dy, x, [N])  # the library's own workspace
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    (got,) = wgrad(dy, x, [N])
+    assert torch.cuda.max_memory_allocated() - before < dy.nbytes
+    # any other layout is read as well: column slices, columns in memory order, a start off the 16-byte grid
+    wide = torch.full((T, N + 7), float("nan"), device="cuda").bfloat16()
+    off = torch.empty(T * N + 1, device="cuda", dtype=torch.bfloat16)[1:].view(T, N)
+    for like in (wide[:, 3 : 3 + N], torch.empty(N, T, device="cuda", dtype=torch.bfloat16).t(), off):
+        assert torch.equal(wgrad(like.copy_(dy), x, [N])[0], got)
+
+
 def test_wgrad_rejects_bad_arguments_before_any_launch():
     from nanonemo_amd.kernels.hip import lib
 
