@@ -12,7 +12,7 @@
 extern "C" {
 #endif
 
-/* logits: [R][V] dense; targets: int64 [R]. Writes lse[R] (logsumexp, fp32), rows[R] (scratch: the rows' losses),
+/* logits: [R][V] dense, R < 2^24; targets: int64 [R]. Writes lse[R] (logsumexp, fp32), rows[R] (scratch: the rows' losses),
  * loss[1] and inv[1] = 1 / number of rows that count. Deterministic. */
 int nn_cross_entropy_fwd(const void* logits, const int64_t* targets, float* lse, float* rows, float* loss, float* inv,
                          int64_t R, int64_t V, int dtype, void* stream);

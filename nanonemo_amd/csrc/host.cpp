@@ -374,17 +374,21 @@ struct Inner {
 // 16384 tokens 140 us in this build's kernel against 165 with the cast, 4096 x 4096 over 8192 334 against 245); odd
 // row counts are its too.
 constexpr int64_t kWgradMost = 6000000;
+// Whether dW (N, K) over T rows is the kernel's; so are only row counts within its 32-bit index.
+bool wgrad_takes(int64_t T, int64_t N, int64_t K) { return N * K <= kWgradMost && N % 8 == 0 && T < (int64_t)1 << 30; }
 
-// The tensor as the kernel reads it: rows of unit stride, 16-byte aligned (a gradient may arrive as a slice of anything).
+// The tensor as the kernel reads it: rows of unit stride within its 32-bit offsets, 16-byte aligned (a gradient may
+// arrive as a slice of anything).
 Tensor rows_aligned(const Tensor& t) {
-    const bool ok = t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) && (uintptr_t)t.data_ptr() % 16 == 0;
+    const bool ok = t.stride(1) == 1 && t.stride(0) % 8 == 0 && t.stride(0) >= t.size(1) && t.stride(0) < (1 << 23) &&
+                    (uintptr_t)t.data_ptr() % 16 == 0;
     return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 std::vector<Tensor> wgrad(const Tensor& dy_, const Tensor& x_, const std::vector<int64_t>& rows) {
     const int64_t T = dy_.size(0), N = dy_.size(1), K = x_.size(1);
     const c10::DeviceGuard guard(x_.device());
-    if (N * K > kWgradMost || N % 8) {
+    if (!wgrad_takes(T, N, K)) {
         // (dense rows are the library's to read whatever their width; an odd vocabulary's are not 16-byte aligned)
         auto dense = [](const Tensor& t) { return t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0 ? t : rows_aligned(t); };
         Tensor dw = at::mm(dense(dy_).t(), dense(x_), at::kFloat);
@@ -660,6 +664,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("norm_fwd", norm_fwd, nogil);
     m.def("norm_bwd", norm_bwd, nogil);
     m.def("wgrad", wgrad, nogil);
+    m.def("wgrad_takes", wgrad_takes);
+    m.def("rows_aligned", rows_aligned);
     m.def("project_fwd", project_fwd, nogil);
     m.def("attention_layer_fwd", attention_layer_fwd, nogil);
     m.def("attention_layer_bwd", attention_layer_bwd, nogil);

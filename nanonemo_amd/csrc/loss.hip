@@ -200,7 +200,8 @@ int launched(const char* what) {
 
 int check_sizes(int64_t R, int64_t V, int dtype, const void* a, const void* b) {
     g_err.clear();
-    if (R < 1 || V < 1 || R >= ((int64_t)1 << 31) || V >= (1 << 30)) return fail("invalid sizes");
+    // (a block per row: a launch holds fewer than 2^32 threads)
+    if (R < 1 || V < 1 || R >= ((int64_t)1 << 32) / kThreads || V >= (1 << 30)) return fail("invalid sizes");
     if (dtype != kF16 && dtype != kBF16 && dtype != kF32) return fail("dtype must be float16, bfloat16 or float32");
     if (((uintptr_t)a & 15) || ((uintptr_t)b & 15)) return fail("logits must be 16-byte aligned");
     return 0;

@@ -21,6 +21,7 @@ def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
     """Whether ``head_loss`` can stand for F.cross_entropy(layer(x).float(), targets), rows flattened."""
     return (eligible(x) and x.dim() >= 2 and plain(layer, x, x.shape[-1], odd_rows=True) and type(targets) is Tensor
             and targets.dtype is torch.int64 and targets.device == x.device and targets.numel() == x.numel() // x.shape[-1]
+            and targets.numel() < 1 << 24  # a block per row, and a launch ends at 2^32 threads
             and not torch.cuda.is_current_stream_capturing())
 
 

@@ -41,13 +41,15 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
     d = x.shape[2]
     if not (plain(wq, x, d) and plain(wk, x, d) and plain(wv, x, d) and plain(wo, x, heads * hd)):
         return False
-    if x.shape[1] * (heads + 2 * kv_heads) * hd >= 1 << 30:  # the library's row offsets within a sequence
+    B, T = x.shape[:2]
+    # the library's row offsets within a sequence, and the rotation kernel's index
+    if T * (heads + 2 * kv_heads) * hd >= 1 << 30 or B * T * (heads + kv_heads) * (hd // 16) >= 1 << 31:
         return False
     if wq.weight.shape[0] != heads * hd or wk.weight.shape[0] != kv_heads * hd or wv.weight.shape[0] != kv_heads * hd:
         return False
     for t in (cos, sin):
         if type(t) is not Tensor or t.dtype is not torch.float32 or t.device != x.device or t.requires_grad \
-                or t.dim() != 2 or t.shape[0] < x.shape[1] or t.shape[1] != hd // 2 or not t.is_contiguous():
+                or t.dim() != 2 or t.shape[0] < T or t.shape[1] != hd // 2 or not t.is_contiguous():
             return False
     return not torch.cuda.is_current_stream_capturing()
 

@@ -37,7 +37,8 @@ def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
         return False
     w = m.weight
     return (type(w) is nn.Parameter and w.dtype is torch.float32 and w.device == x.device and w.is_contiguous()
-            and w.shape[1] == width and (odd_rows or w.shape[0] % 8 == 0) and width % 8 == 0 and w.data_ptr() % 16 == 0)
+            and w.shape[1] == width and (odd_rows or w.shape[0] % 8 == 0) and width % 8 == 0 and w.data_ptr() % 16 == 0
+            and w.numel() < 1 << 31)  # the cast kernel's index, for up to four weights
 
 
 def function_mode() -> bool:

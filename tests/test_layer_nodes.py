@@ -156,3 +156,36 @@ def test_function_modes_see_the_modules():
             assert linear.function_mode()
     with Mode():
         assert linear.function_mode()
+
+
+def test_calls_past_the_kernels_indices_keep_the_modules(monkeypatch):
+    # Sizes only (expanded tensors hold one value): no call that the modules answer may end in the library's refusal.
+    from types import SimpleNamespace
+
+    from nanonemo_amd.kernels import hip
+    from nanonemo_amd.kernels.hip import head, host, layers, linear
+
+    for m in (head, layers):
+        monkeypatch.setattr(m, "eligible", lambda x: True)
+        monkeypatch.setattr(m, "plain", lambda *_, **__: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    one = torch.zeros(1, dtype=torch.bfloat16)
+    rows = lambda n, d: one.expand(n, d)  # noqa: E731
+    for n, takes in (((1 << 24) - 1, True), (1 << 24, False)):  # a block per row, 2^32 threads in a launch
+        assert head.can_fuse_head(rows(n, 8), None, torch.zeros(1, dtype=torch.int64).expand(n)) is takes
+    assert hip.lib().nn_cross_entropy_fwd(*[None] * 6, 1 << 24, 8, 1, None) != 0 and b"invalid sizes" in hip.lib().nn_loss_last_error()
+    H, KVH, hd, T = 12, 4, 64, 1024
+    w = SimpleNamespace(weight=rows(H * hd, 64)), SimpleNamespace(weight=rows(KVH * hd, 64))
+    cos = torch.zeros(T, hd // 2)
+    for B, takes in (((1 << 31) // (T * (H + KVH) * (hd // 16)) - 1, True), ((1 << 31) // (T * (H + KVH) * (hd // 16)), False)):
+        assert layers.can_fuse(one.expand(B, T, 64), cos, cos, H, KVH, hd, w[0], w[1], w[1], w[0]) is takes
+    assert host().wgrad_takes((1 << 30) - 1, 8, 8) and not host().wgrad_takes(1 << 30, 8, 8)
+    assert host().wgrad_takes(0, 8, 750000) and not host().wgrad_takes(64, 8, 750001) and not host().wgrad_takes(64, 12, 8)
+    storage = torch.zeros(3 * (1 << 23) + 8, dtype=torch.bfloat16)
+    near, far = (storage.as_strided((4, 8), (ld, 1)) for ld in ((1 << 23) - 8, 1 << 23))
+    assert host().rows_aligned(near).data_ptr() == storage.data_ptr() and host().rows_aligned(far).is_contiguous()
+
+    layer = nn.Linear(8, 8, bias=False)
+    for n, takes in (((1 << 31) // 64 - 8, True), ((1 << 31) // 64, False)):
+        layer.weight = nn.Parameter(torch.empty(n, 64, device="meta"))
+        assert linear.plain(layer, torch.empty(1, device="meta"), 64) is takes
