@@ -3,8 +3,8 @@
 
 The loss reads the 16-bit logits once and its backward reads them once and writes their gradient, where F.cross_entropy
 on logits.float() moves an fp32 copy, its log-softmax and their gradients. ``can_fuse_head`` holds for calls that
-``linear.can_project`` describes with int64 targets; the others run module by module. A target that is neither -100 nor in [0, V) makes the loss and its row's
-gradient NaN (F.cross_entropy ends the process with a device assertion).
+``linear.can_project`` describes with int64 targets; the others run module by module. A target that is neither -100 nor in
+[0, V) makes the loss and its row's gradient NaN (F.cross_entropy ends the process with a device assertion).
 """
 
 from __future__ import annotations
@@ -21,8 +21,7 @@ def can_fuse_head(x: Tensor, layer: nn.Module, targets: Tensor) -> bool:
     """Whether ``head_loss`` can stand for F.cross_entropy(layer(x).float(), targets), rows flattened."""
     return (eligible(x) and x.dim() >= 2 and plain(layer, x, x.shape[-1], odd_rows=True) and type(targets) is Tensor
             and targets.dtype is torch.int64 and targets.device == x.device and targets.numel() == x.numel() // x.shape[-1]
-            and targets.numel() < 1 << 24  # a block per row, and a launch ends at 2^32 threads
-            and not torch.cuda.is_current_stream_capturing())
+            and targets.numel() < 1 << 24)  # a block per row, and a launch ends at 2^32 threads
 
 
 class _HeadLoss(torch.autograd.Function):

@@ -51,7 +51,7 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
         if type(t) is not Tensor or t.dtype is not torch.float32 or t.device != x.device or t.requires_grad \
                 or t.dim() != 2 or t.shape[0] < T or t.shape[1] != hd // 2 or not t.is_contiguous():
             return False
-    return not torch.cuda.is_current_stream_capturing()
+    return True
 
 
 class _AttentionLayer(torch.autograd.Function):
@@ -111,8 +111,7 @@ def can_fuse_mlp(x: Tensor, w_gate, w_up, w_down) -> bool:
     if not (plain(w_gate, x, d) and plain(w_up, x, d)):
         return False
     F_ = w_gate.weight.shape[0]
-    return (w_up.weight.shape[0] == F_ and plain(w_down, x, F_) and x.numel() // d * F_ < 1 << 33  # the activation kernel's index
-            and not torch.cuda.is_current_stream_capturing())
+    return (w_up.weight.shape[0] == F_ and plain(w_down, x, F_) and x.numel() // d * F_ < 1 << 33)  # the activation kernel's index
 
 
 class _MlpLayer(torch.autograd.Function):

@@ -168,7 +168,6 @@ def test_calls_past_the_kernels_indices_keep_the_modules(monkeypatch):
     for m in (head, layers):
         monkeypatch.setattr(m, "eligible", lambda x: True)
         monkeypatch.setattr(m, "plain", lambda *_, **__: True)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     one = torch.zeros(1, dtype=torch.bfloat16)
     rows = lambda n, d: one.expand(n, d)  # noqa: E731
     for n, takes in (((1 << 24) - 1, True), (1 << 24, False)):  # a block per row, 2^32 threads in a launch
@@ -189,3 +188,15 @@ def test_calls_past_the_kernels_indices_keep_the_modules(monkeypatch):
     for n, takes in (((1 << 31) // 64 - 8, True), ((1 << 31) // 64, False)):
         layer.weight = nn.Parameter(torch.empty(n, 64, device="meta"))
         assert linear.plain(layer, torch.empty(1, device="meta"), 64) is takes
+
+
+def test_stream_capture_keeps_the_modules(monkeypatch):
+    from nanonemo_amd.kernels.hip import linear
+
+    monkeypatch.setattr(linear, "eager", lambda *_: True)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *_: True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda *_: torch.bfloat16)
+    m, x, _ = _head_inputs()
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        assert linear.can_project(x, m) is not capturing
