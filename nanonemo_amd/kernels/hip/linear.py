@@ -10,8 +10,8 @@ which 10 would do).
 
 ``can_project(x, layers)`` says whether the call can take this path: plain CUDA tensors and untouched fp32
 ``nn.Linear`` layers under 16-bit autocast, in eager mode. Everything else (hooks, parametrizations, other module or
-tensor types, torch.compile, torch.func, dispatch and function modes, forward-mode AD, stream capture, no autocast) keeps
-calling the modules. A backward that is itself recorded (create_graph), or is handed gradients that the kernel cannot read by
+tensor types, torch.compile, torch.func, dispatch and function modes, forward-mode AD, no autocast, a stream capture with
+gradients enabled) keeps calling the modules. A backward that is itself recorded (create_graph), or is handed gradients that the kernel cannot read by
 address (is_grads_batched), runs differentiable torch products instead of the kernel.
 """
 
@@ -53,7 +53,7 @@ def eligible(x: Tensor) -> bool:
     if x.dim() < 2 or x.numel() == 0 or not x.is_floating_point() or x.dtype is torch.float64:
         return False
     return not (torch.jit.is_tracing() or function_mode() or forward_ad._current_level >= 0 or _module._has_any_global_hook()
-                or torch.cuda.is_current_stream_capturing())
+                or torch.is_grad_enabled() and torch.cuda.is_current_stream_capturing())
 
 
 def can_project(x: Tensor, *layers: nn.Module) -> bool:

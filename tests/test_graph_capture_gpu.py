@@ -4,7 +4,8 @@ common.py:30-54, and that compile(mode="reduce-overhead") relies on, trainer.py:
 The library allocates, frees, synchronises and memsets nothing, so its calls can be captured. Here the
 calls themselves are captured with torch.cuda.graph on buffers allocated beforehand (no autograd inside
 the capture): one nn_fa_fwd + nn_fa_bwd pair (also at a shape whose dK/dV work is split, which adds the
-partial-sum kernel), and the RoPE and fused add + RMSNorm kernels beside it.
+partial-sum kernel), and the RoPE and fused add + RMSNorm kernels beside it. The model's forward without autograd is
+captured as a program would capture it, outputs allocated inside.
 Each graph is replayed several times with eager work and synchronisations in between, outputs poisoned
 before every replay; every replay must equal the eager result bit for bit.
 """
@@ -108,3 +109,37 @@ def test_captured_rope_and_rmsnorm_c_abi_calls_replay_bit_identically():
                                            1, 2, 2, 1, stream))
 
     _replays_match(launch, [qo, ko, y, h, rstd, dx, dd, dw])
+
+
+@pytest.mark.parametrize("attn, rope", [("hip_bthd", "hip"), ("hip", "hip")])
+def test_captured_evaluation_replays_the_eager_result(attn, rope):
+    from nanonemo_amd.model import ModelConfig, NanoNemo
+
+    print(f"\n[case] graph capture of the model's forward without autograd, {attn} {rope}", flush=True)
+    torch.manual_seed(0)
+    m = NanoNemo(ModelConfig(n_layers=2, vocab_size=1024, attn_kernel=attn, rope_kernel=rope, norm_kernel="hip")).cuda()
+    idx = torch.randint(0, 1024, (2, 256), device="cuda")
+    targets = torch.roll(idx, -1, 1)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, cache_enabled=False):
+            return m(idx, targets)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = run()
+    for i in range(4):
+        idx.copy_(torch.randint(0, 1024, idx.shape, device="cuda"))
+        targets.copy_(torch.roll(idx, -1, 1))
+        ref = run()
+        for t in outs:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, ref)), f"replay {i}"

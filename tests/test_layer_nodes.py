@@ -190,7 +190,8 @@ def test_calls_past_the_kernels_indices_keep_the_modules(monkeypatch):
         assert linear.plain(layer, torch.empty(1, device="meta"), 64) is takes
 
 
-def test_stream_capture_keeps_the_modules(monkeypatch):
+def test_stream_capture_with_gradients_keeps_the_modules(monkeypatch):
+    # (without them the captured call is the eager one, and so are its results)
     from nanonemo_amd.kernels.hip import linear
 
     monkeypatch.setattr(linear, "eager", lambda *_: True)
@@ -200,3 +201,5 @@ def test_stream_capture_keeps_the_modules(monkeypatch):
     for capturing in (False, True):
         monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
         assert linear.can_project(x, m) is not capturing
+        with torch.no_grad():
+            assert linear.can_project(x, m)
