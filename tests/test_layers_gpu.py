@@ -1,4 +1,4 @@
-"""GPU tests of the fused layers (kernels/hip/layers.py) against the same modules run one by one."""
+"""GPU tests of the fused layers (kernels/hip/layers.py) against the same modules run one by one and against float64."""
 
 from __future__ import annotations
 
@@ -56,6 +56,54 @@ def test_attention_layer_matches_its_modules(B, T, H, KVH, hd, dtype):
         torch.testing.assert_close(a, b, rtol=tol, atol=tol * b.abs().max().item(), msg=name)
     with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
         assert torch.equal(m(x, cos, sin), got[0])
+
+
+def _rel(a, b):
+    """The 2-norm of a - b over b's, in float64."""
+    return ((a.double() - b).norm() / b.norm()).item()
+
+
+def _attention64(x, cos, sin, H, KVH, wq, wk, wv, wo):
+    B, T, _ = x.shape
+    c, s = cos[:T, None].double(), sin[:T, None].double()
+
+    def rot(t):
+        a, b = t.chunk(2, -1)
+        return torch.cat((a * c - b * s, a * s + b * c), -1)
+
+    q, k, v = ((x @ w.t()).view(B, T, h, -1) for w, h in ((wq, H), (wk, KVH), (wv, KVH)))
+    q, k, v = rot(q).transpose(1, 2), rot(k).transpose(1, 2), v.transpose(1, 2)
+    k, v = (t.repeat_interleave(H // KVH, 1) for t in (k, v))
+    future = torch.ones(T, T, dtype=torch.bool, device=x.device).triu(1)
+    p = ((q @ k.transpose(2, 3)) / q.shape[-1] ** 0.5).masked_fill(future, -float("inf")).softmax(-1)
+    return (p @ v).transpose(1, 2).reshape(B, T, -1) @ wo.t()
+
+
+# The 16-bit roundings on the longest path to an output or gradient: each moves its tensor by at most u in the 2-norm
+# (u = 2^-8 in bf16, 2^-11 in fp16), the products that follow carry that on as they carry the tensor, and independent
+# roundings add up in squares, so n of them give at most sqrt(n) u.
+def _assert_close_to_float64(names, got, modules, exact, n, dtype):
+    u = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for name, a, b, ref in zip(names, got, modules, exact):
+        mine, theirs = _rel(a, ref), _rel(b, ref)
+        print(f"  {name}: {mine:.2e}, modules {theirs:.2e}, bound {n**0.5 * u:.2e}", flush=True)
+        assert mine <= n**0.5 * u, name
+        assert mine <= 1.1 * theirs, name  # no term may be worse than in the modules, which round more
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B, T, H, KVH, hd", [(2, 200, 12, 4, 64), (3, 65, 2, 2, 64), (1, 1030, 8, 2, 32)])
+def test_attention_layer_matches_float64(B, T, H, KVH, hd, dtype):
+    print(f"\n[case] attention layer against float64 B={B} T={T} H={H} KVH={KVH} hd={hd} {dtype}", flush=True)
+    m, (cos, sin) = _attention(H, KVH, hd, T, rope_kernel="hip")
+    x = torch.randn(B, T, H * hd, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(B, T, H * hd, device="cuda").to(dtype)
+    ins = [t.detach().double().requires_grad_() for t in (x, m.wq.weight, m.wk.weight, m.wv.weight, m.wo.weight)]
+    y = _attention64(ins[0], cos, sin, H, KVH, *ins[1:])
+    exact = (y.detach(), *torch.autograd.grad(y, ins, dy.double()))
+    # dwq, dwk: weights, product, rotation of q and of k; P and O; the output weight, dO, dS, dq or dk, its rotation
+    _assert_close_to_float64(("y", "dx", "dwq", "dwk", "dwv", "dwo"), _run(m, (x, cos, sin), dy, dtype),
+                             _run(_modules_only(m), (x, cos, sin), dy, dtype), exact, 13, dtype)
 
 
 def test_attention_layer_frozen_parts_and_repeated_backward():
@@ -120,6 +168,21 @@ def test_mlp_layer_matches_its_modules(shape, d, ff, dtype):
     for name, a, b in zip(("y", "dx", "dw_gate", "dw_up", "dw_down"), got, ref):
         assert a.shape == b.shape and a.dtype == b.dtype, name
         torch.testing.assert_close(a, b, rtol=tol, atol=tol * b.abs().max().item(), msg=name)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows, d, ff", [(400, 96, 264), (700, 768, 2048), (105, 40, 72)])
+def test_mlp_layer_matches_float64(rows, d, ff, dtype):
+    print(f"\n[case] MLP layer against float64 {rows} d={d} ff={ff} {dtype}", flush=True)
+    m = _mlp(d, ff)
+    x = torch.randn(rows, d, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(rows, d, device="cuda").to(dtype)
+    ins = [t.detach().double().requires_grad_() for t in (x, m.w_gate.weight, m.w_up.weight, m.w_down.weight)]
+    y = (torch.nn.functional.silu(ins[0] @ ins[1].t()) * (ins[0] @ ins[2].t())) @ ins[3].t()
+    exact = (y.detach(), *torch.autograd.grad(y, ins, dy.double()))
+    # dx: the gate's and up's weights and products, the down weight, dh, dgate and dup, dx
+    _assert_close_to_float64(("y", "dx", "dw_gate", "dw_up", "dw_down"), _run(m, (x,), dy, dtype), _run(_modules_only(m), (x,), dy, dtype),
+                             exact, 9, dtype)
 
 
 @pytest.mark.parametrize("kw", [dict(attn_kernel="hip_bthd", rope_kernel="hip", norm_kernel="hip"), dict(attn_kernel="hip")])
