@@ -826,12 +826,11 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkdv_kernel(
         };
         auto run = [&](auto dma_tag, int itn, const u16* qs, const u16* os, float* ls, int nitn, u16* nqs,
                        u16* nos, float* nls) {
-            const int itu = itn;
             // Rows past T (zero Q and dO rows; their -lse is row T - 1's, which with a zero score could
             // overflow p) start their scores from -inf instead, so their p is 0: patched in this wave's
             // copy of the -lse vector, which has landed.
-            if (T % BM != 0 && at_high(itu) && lane >= T % BM) ls[wave * 2 * BM + lane] = -INFINITY;
-            if (at_low(itu))
+            if (T % BM != 0 && at_high(itn) && lane >= T % BM) ls[wave * 2 * BM + lane] = -INFINITY;
+            if (at_low(itn))
                 compute(std::true_type{}, dma_tag, qs, os, ls, nitn, nqs, nos, nls);
             else
                 compute(std::false_type{}, dma_tag, qs, os, ls, nitn, nqs, nos, nls);

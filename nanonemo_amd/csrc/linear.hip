@@ -77,7 +77,7 @@ struct Operand {
 // store instruction covers 32 consecutive floats of two rows. Four stages of 32 KB, three in flight.
 // Bound: a stage is 512 MFMA cycles per SIMD beside 64 KB of transposing LDS reads (about 580 cycles per CU) and the
 // scalar work of its copies; it takes about 1300. Measured with the sum kernel, against the library's bf16 product
-// and cast, 8192 tokens: 768 x 768 22 us (51), 1280 x 768 26 (55), 4096 x 768 66 (83), 768 x 2048 37 (66); an earlier
+// and cast, 8192 tokens: 768 x 768 22 us (51), 1280 x 768 27 (54), 4096 x 768 61 (82), 768 x 2048 38 (65); an earlier
 // form with two 64 KB buffers and branching edge tests: 24, 30, 77, 48.
 template <int DT>
 __global__ __launch_bounds__(512, 2) void wgrad_kernel(const u16* __restrict__ dY, long long ldy,
