@@ -153,10 +153,22 @@ T2 fa_fwd(Tensor q, Tensor k, Tensor v) {
     return {o, lse};
 }
 
-// On inputs the forward checked; o and lse contiguous.
-T3 fa_bwd(Tensor d_o, Tensor q, Tensor k, Tensor v, const Tensor& o, const Tensor& lse) {
+// The backwards check what they are given like the forwards: a saved tensor is what the caller's saved-tensor hooks made
+// of it, and the library reads raw addresses.
+void check_backward(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, int seq) {
+    check_attention(q, k, v, seq);
+    check_on_device(q, {&d_o, &o, &lse});
+    need(d_o.sizes() == q.sizes() && d_o.scalar_type() == q.scalar_type() && o.sizes() == q.sizes() && o.scalar_type() == q.scalar_type(),
+         "d_o must be a contiguous float16/bfloat16 tensor shaped like q");
+    need(lse.sizes() == at::IntArrayRef({q.size(0), q.size(3 - seq), q.size(seq)}) && lse.scalar_type() == at::kFloat,
+         "lse must be a float32 tensor of shape (B, H, T)");
+}
+
+T3 fa_bwd(Tensor d_o, Tensor q, Tensor k, Tensor v, const Tensor& o_, const Tensor& lse_) {
     make_readable({&q, &d_o});
     make_readable({&k, &v});
+    check_backward(d_o, q, k, v, o_, lse_, 2);
+    const Tensor o = contig(o_), lse = contig(lse_);
     const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3), KVH = k.size(1);
     Tensor dq = empty_of(q, q.sizes()), dk = empty_of(k, k.sizes()), dv = empty_of(v, v.sizes());
     if (empty_problem(q)) return {dq, dk, dv};
@@ -191,8 +203,9 @@ T2 bthd_fwd(const Tensor& q_, const Tensor& k_, const Tensor& v_) {
     return {o, lse};
 }
 
-T3 bthd_bwd(const Tensor& d_o_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o, const Tensor& lse) {
-    const Tensor d_o = contig(d_o_), q = contig(q_), k = contig(k_), v = contig(v_);
+T3 bthd_bwd(const Tensor& d_o_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_, const Tensor& lse_) {
+    const Tensor d_o = contig(d_o_), q = contig(q_), k = contig(k_), v = contig(v_), o = contig(o_), lse = contig(lse_);
+    check_backward(d_o, q, k, v, o, lse, 1);
     const int64_t B = q.size(0), T = q.size(1), H = q.size(2), D = q.size(3), KVH = k.size(2);
     Tensor dq = empty_of(q, q.sizes()), dk = empty_of(k, k.sizes()), dv = empty_of(v, v.sizes());
     if (empty_problem(q)) return {dq, dk, dv};
@@ -229,9 +242,12 @@ T3 bthd_rope_fwd(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Ten
     return {o, lse, q_rot};
 }
 
-T3 bthd_rope_bwd(const Tensor& d_o_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o, const Tensor& lse,
+T3 bthd_rope_bwd(const Tensor& d_o_, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_, const Tensor& lse_,
                  const Tensor& cos_, const Tensor& sin_) {
-    const Tensor d_o = contig(d_o_), q = contig(q_), k = contig(k_), v = contig(v_), cos = contig(cos_), sin = contig(sin_);
+    const Tensor d_o = contig(d_o_), q = contig(q_), k = contig(k_), v = contig(v_), o = contig(o_), lse = contig(lse_);
+    check_backward(d_o, q, k, v, o, lse, 1);
+    check_tables(cos_, sin_, q.size(1), q.size(3), q.device());
+    const Tensor cos = contig(cos_), sin = contig(sin_);
     const int64_t B = q.size(0), T = q.size(1), H = q.size(2), D = q.size(3), KVH = k.size(2);
     Tensor dq = empty_of(q, q.sizes()), dk = empty_of(k, k.sizes()), dv = empty_of(v, v.sizes());
     if (empty_problem(q)) return {dq, dk, dv};
@@ -255,35 +271,18 @@ void refuse_capture_from_engine(const std::string& where, const std::function<bo
           "ended in a host fault in capture_end and no cause has been shown. Capture the C ABI calls (nn_fa_fwd / nn_fa_bwd / "
           "nn_fa_bwd_noalloc) instead, or run the ops eagerly (torch.compile(fullgraph=True) without graphs is supported).");
 }
-void check_backward(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, int seq) {
-    check_attention(q, k, v, seq);
-    check_on_device(q, {&d_o, &o, &lse});
-    need(d_o.sizes() == q.sizes() && d_o.scalar_type() == q.scalar_type() && o.sizes() == q.sizes() && o.scalar_type() == q.scalar_type(),
-         "d_o must be a contiguous float16/bfloat16 tensor shaped like q");
-    need(lse.sizes() == at::IntArrayRef({q.size(0), q.size(3 - seq), q.size(seq)}) && lse.scalar_type() == at::kFloat,
-         "lse must be a float32 tensor of shape (B, H, T)");
-}
-T3 fa_bwd_op(const Tensor& d_o, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o, const Tensor& lse) {
+T3 fa_bwd_op(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse) {
     refuse_capture_from_engine("flash_attn backward op");
-    Tensor q = q_, k = k_, v = v_;
-    make_readable({&q});
-    make_readable({&k, &v});
-    check_backward(d_o, q, k, v, o, lse, 2);
-    return fa_bwd(d_o, q, k, v, contig(o), contig(lse));
+    return fa_bwd(d_o, q, k, v, o, lse);
 }
-T3 bthd_bwd_op(const Tensor& d_o, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o, const Tensor& lse) {
+T3 bthd_bwd_op(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse) {
     refuse_capture_from_engine("flash_attn_bthd backward op");
-    const Tensor q = contig(q_), k = contig(k_), v = contig(v_);
-    check_backward(d_o, q, k, v, o, lse, 1);
-    return bthd_bwd(d_o, q, k, v, contig(o), contig(lse));
+    return bthd_bwd(d_o, q, k, v, o, lse);
 }
-T3 bthd_rope_bwd_op(const Tensor& d_o, const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o, const Tensor& lse,
+T3 bthd_rope_bwd_op(const Tensor& d_o, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse,
                     const Tensor& cos, const Tensor& sin) {
     refuse_capture_from_engine("flash_attn_bthd_rope backward op");
-    const Tensor q = contig(q_), k = contig(k_), v = contig(v_);
-    check_backward(d_o, q, k, v, o, lse, 1);
-    check_tables(cos, sin, q.size(1), q.size(3), q.device());
-    return bthd_rope_bwd(d_o, q, k, v, contig(o), contig(lse), cos, sin);
+    return bthd_rope_bwd(d_o, q, k, v, o, lse, cos, sin);
 }
 
 // ---- RoPE ---------------------------------------------------------------------------------------
@@ -370,6 +369,14 @@ struct Inner {
     c10::impl::ExcludeDispatchKeyGuard no_autocast{c10::DispatchKeySet(c10::DispatchKey::AutocastCUDA)};
 };
 
+// A tensor that the forward saved, as the kernels read it (see check_backward).
+Tensor saved(const Tensor& t, const Tensor& x, at::IntArrayRef sizes, at::ScalarType type) {
+    need(t.device() == x.device() && t.scalar_type() == type && t.sizes() == sizes,
+         "a saved tensor is not what the forward saved: another device, type or shape");
+    return contig(t);
+}
+Tensor saved(const Tensor& t, const Tensor& x, at::IntArrayRef sizes) { return saved(t, x, sizes, x.scalar_type()); }
+
 // Above this many elements of dW the library's product fills the chip by itself and is the faster one (2048 x 2048 over
 // 16384 tokens 140 us in this build's kernel against 165 with the cast, 4096 x 4096 over 8192 334 against 245); odd
 // row counts are its too.
@@ -386,6 +393,9 @@ Tensor rows_aligned(const Tensor& t) {
 }
 
 std::vector<Tensor> wgrad(const Tensor& dy_, const Tensor& x_, const std::vector<int64_t>& rows) {
+    check_on_device(x_, {&dy_});
+    need(dy_.dim() == 2 && x_.dim() == 2 && dy_.size(0) == x_.size(0) && dy_.scalar_type() == x_.scalar_type() && code(x_) >= 0 && code(x_) < 2,
+         "expected float16 or bfloat16 gradients (T, N) and inputs (T, K)");
     const int64_t T = dy_.size(0), N = dy_.size(1), K = x_.size(1);
     const c10::DeviceGuard guard(x_.device());
     if (!wgrad_takes(T, N, K)) {
@@ -425,7 +435,11 @@ Weights cast_weights(const Tensor& like, const std::vector<std::vector<Tensor>>&
     for (const auto& g : groups) {
         int64_t N = 0;
         const int64_t K = g[0].size(1);
-        for (const Tensor& w : g) N += w.size(0);
+        for (const Tensor& w : g) {
+            check_on_device(like, {&w});
+            need(w.dim() == 2 && w.size(1) == K && w.is_contiguous(), "weights must be contiguous and of one width");
+            N += w.size(0);
+        }
         out.fwd.push_back(empty_of(like, {N, K}));
         const Tensor t = turned ? empty_of(like, {K, N}) : Tensor();
         out.bwd.push_back(turned ? t.t() : out.fwd.back());
@@ -483,6 +497,7 @@ std::vector<Tensor> attention_layer_fwd(const Tensor& x, const Tensor& cos, cons
     const Inner inner;
     const c10::DeviceGuard guard(x.device());
     const LayerShape s(B, T, H, KVH, wq.size(0) / H);
+    check_tables(cos, sin, T, s.D, x.device());
     const int dt = code(x);
     void* st = stream_of(x);
     const Weights w = cast_weights(x, {{wq, wk, wv}, {wo}}, turned);
@@ -496,12 +511,16 @@ std::vector<Tensor> attention_layer_fwd(const Tensor& x, const Tensor& cos, cons
 }
 
 // The gradients of x, wq, wk, wv and wo; undefined where not needed.
-std::vector<OptTensor> attention_layer_bwd(const Tensor& dy_, const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& qkv,
-                                           const Tensor& q, const Tensor& o, const Tensor& lse, const Tensor& w, const Tensor& wo,
+std::vector<OptTensor> attention_layer_bwd(const Tensor& dy_, const Tensor& x, const Tensor& cos_, const Tensor& sin_, const Tensor& qkv_,
+                                           const Tensor& q_, const Tensor& o_, const Tensor& lse_, const Tensor& w, const Tensor& wo,
                                            int64_t B, int64_t T, int64_t H, int64_t KVH, bool need_x, bool need_qkv, bool need_o) {
     const Inner inner;
+    check_on_device(x, {&dy_});
     const c10::DeviceGuard guard(x.device());
-    const LayerShape s(B, T, H, KVH, q.size(1) / H);
+    const LayerShape s(B, T, H, KVH, wo.size(1) / H);
+    check_tables(cos_, sin_, T, s.D, x.device());
+    const Tensor cos = contig(cos_), sin = contig(sin_), lse = saved(lse_, x, {B, H, T}, at::kFloat);
+    const Tensor qkv = saved(qkv_, x, {B * T, s.n}), q = saved(q_, x, {B * T, s.nq}), o = saved(o_, x, {B * T, s.nq});
     const int dt = code(x);
     void* st = stream_of(x);
     const Tensor dy = contig(dy_);
@@ -536,12 +555,13 @@ std::vector<Tensor> mlp_fwd(const Tensor& x, const Tensor& w_gate, const Tensor&
 }
 
 // The gradients of x, w_gate, w_up and w_down; undefined where not needed.
-std::vector<OptTensor> mlp_bwd(const Tensor& dy_, const Tensor& x, const Tensor& gu, const Tensor& h, const Tensor& w, const Tensor& w_down,
+std::vector<OptTensor> mlp_bwd(const Tensor& dy_, const Tensor& x, const Tensor& gu_, const Tensor& h_, const Tensor& w, const Tensor& w_down,
                                bool need_x, bool need_gu, bool need_down) {
     const Inner inner;
+    check_on_device(x, {&dy_});
     const c10::DeviceGuard guard(x.device());
-    const Tensor dy = contig(dy_);
-    const int64_t T = x.size(0), F = h.size(1);
+    const int64_t T = x.size(0), F = w_down.size(1);
+    const Tensor dy = contig(dy_), gu = saved(gu_, x, {T, 2 * F}), h = saved(h_, x, {T, F});
     std::vector<OptTensor> out(4);
     Tensor dh = need_x || need_gu ? at::mm(dy, w_down) : Tensor();
     if (need_down) out[3] = wgrad(dy, h, {w_down.size(0)})[0];
@@ -559,6 +579,8 @@ std::vector<OptTensor> mlp_bwd(const Tensor& dy_, const Tensor& x, const Tensor&
 // (logits, loss, w16 for the backward, lse, 1 / rows that count).
 std::vector<Tensor> head_fwd(const Tensor& x, const Tensor& w_, const Tensor& targets, bool turned) {
     const Inner inner;
+    check_on_device(x, {&targets});
+    need(targets.is_contiguous() && targets.numel() == x.size(0), "expected one contiguous target per row");
     const c10::DeviceGuard guard(x.device());
     const Weights w = cast_weights(x, {{w_}}, turned && w_.size(0) % 8 == 0);
     const Tensor logits = at::mm(x, w.fwd[0].t());
@@ -572,21 +594,24 @@ std::vector<Tensor> head_fwd(const Tensor& x, const Tensor& w_, const Tensor& ta
 // The gradients of x and w from those of the logits and of the loss (either may be missing); logits: the forward's, or
 // nothing to compute them again (by the forward's product, on rows).
 std::vector<OptTensor> head_bwd(const OptTensor& dlogits_, const OptTensor& dloss, const OptTensor& logits_, const Tensor& x,
-                                const Tensor& w, const Tensor& targets, const Tensor& lse, const Tensor& inv, bool need_x, bool need_w) {
+                                const Tensor& w, const Tensor& targets_, const Tensor& lse_, const Tensor& inv_, bool need_x, bool need_w) {
     const Inner inner;
+    check_on_device(x, {});
     const c10::DeviceGuard guard(x.device());
+    const int64_t R = x.size(0), V = w.size(0);
     std::vector<OptTensor> out(2);
-    Tensor d = dlogits_.has_value() ? contig(*dlogits_) : Tensor();
+    Tensor d = dlogits_.has_value() ? saved(*dlogits_, x, {R, V}) : Tensor();
     if (dloss.has_value()) {
-        const Tensor logits = logits_.has_value() ? *logits_ : at::mm(x, contig(w).t()), g = contig(*dloss);
+        const Tensor targets = saved(targets_, x, {R}, at::kLong), lse = saved(lse_, x, {R}, at::kFloat), inv = saved(inv_, x, {}, at::kFloat);
+        const Tensor logits = logits_.has_value() ? saved(*logits_, x, {R, V}) : at::mm(x, contig(w).t()), g = saved(*dloss, x, {}, at::kFloat);
         Tensor t = at::empty_like(logits);
         loss_done(nn_cross_entropy_bwd(logits.data_ptr(), targets.data_ptr<int64_t>(), lse.data_ptr<float>(), inv.data_ptr<float>(),
-                                       g.data_ptr<float>(), t.data_ptr(), logits.size(0), logits.size(1), code(x), stream_of(x)));
+                                       g.data_ptr<float>(), t.data_ptr(), R, V, code(x), stream_of(x)));
         d = d.defined() ? t.add_(d) : t;
     }
     if (!d.defined()) return out;
     if (need_x) out[0] = at::mm(d, w);
-    if (need_w) out[1] = wgrad(d, x, {w.size(0)})[0];
+    if (need_w) out[1] = wgrad(d, x, {V})[0];
     return out;
 }
 

@@ -544,3 +544,23 @@ def test_norm_backward_op_refuses_host_tensors():
     for dh in (None, t):
         with pytest.raises(RuntimeError, match="must be CUDA tensors"):
             torch.ops.nanonemo.cuda_add_rms_norm_bwd(t, dh, t, w, r, torch.float32, None if dh is None else torch.float32)
+
+
+def test_host_functions_refuse_host_tensors():
+    # Before anything is launched, in the layers' functions and in the backwards that autograd's saved tensors reach.
+    from nanonemo_amd.kernels.hip import host
+
+    h, bf = host(), torch.bfloat16
+    x, w, w16, lse = torch.ones(16, 64, dtype=bf), torch.ones(64, 64), torch.ones(64, 64, dtype=bf), torch.ones(1, 1, 16)
+    cos, t, one = torch.ones(16, 32), torch.zeros(16, dtype=torch.int64), torch.ones(())
+    qkv, gu, q4 = torch.ones(16, 192, dtype=bf), torch.ones(16, 128, dtype=bf), torch.ones(1, 16, 1, 64, dtype=bf)
+    qt = q4.transpose(1, 2)
+    for f in (lambda: h.wgrad(x, x, [64]), lambda: h.project_fwd(x, [w], True), lambda: h.mlp_fwd(x, w, w, w, False),
+              lambda: h.mlp_bwd(x, x, gu, x, torch.cat([w16, w16]), w16, True, True, True),
+              lambda: h.attention_layer_fwd(x, cos, cos, 1, 16, 1, 1, w, w, w, w, True),
+              lambda: h.attention_layer_bwd(x, x, cos, cos, qkv, x, x, lse, torch.cat([w16] * 3), w16, 1, 16, 1, 1, True, True, True),
+              lambda: h.head_fwd(x, w, t, False), lambda: h.head_bwd(x, one, x, x, w16, t, one.expand(16), one, True, True),
+              lambda: h.fa_bwd(qt, qt, qt, qt, qt, lse), lambda: h.bthd_bwd(q4, q4, q4, q4, q4, lse),
+              lambda: h.bthd_rope_bwd(q4, q4, q4, q4, q4, lse, cos, cos)):
+        with pytest.raises(RuntimeError, match="must be CUDA tensors|on the inputs' device"):
+            f()

@@ -225,3 +225,49 @@ def test_swiglu_matches_float64(T, F, dtype):
         # silu'(g) cancels near its zero at g = -1.28: its fp32 error is a few 2^-24 of 1
         assert ((a.double() - b)[ok].abs() <= eps * b[ok].abs() + tiny + 1e-6).all()
         assert torch.equal(a.isnan(), b.isnan())
+
+
+def _saved_through(unpack, f):
+    """The gradients of f() = (output, inputs) with every saved tensor passed through unpack."""
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y, ins = f()
+    return torch.autograd.grad(y.float().square().sum(), ins)
+
+
+@pytest.mark.parametrize("what", ["attention layer", "mlp", "head", "projection", "flash_attn", "flash_attn_bthd", "flash_attn_bthd_rope"])
+def test_saved_tensors_are_checked_like_inputs(what):
+    # what a saved-tensor hook hands back reaches the kernels by address: dense or not it is read rightly, and a host tensor
+    # or another type is an error before any launch
+    from nanonemo_amd.kernels.hip import flash_attn as fa
+    from nanonemo_amd.kernels.hip import head, layers, linear
+
+    torch.manual_seed(1)
+    m, (cos, sin) = _attention(4, 2, 64, 70, rope_kernel="hip")
+    mlp, x = _mlp(256, 264), torch.randn(2, 70, 256, device="cuda").bfloat16().requires_grad_()
+    targets = torch.randint(0, 264, (2, 70), device="cuda")
+    q, k, v = (torch.randn(2, 70, h, 64, device="cuda").bfloat16().requires_grad_() for h in (4, 2, 2))
+
+    def f():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            if what == "attention layer":
+                return layers.attention_layer(x, cos, sin, 4, 2, m.wq, m.wk, m.wv, m.wo), (x, *m.parameters())
+            if what == "mlp":
+                return layers.mlp_layer(x, mlp.w_gate, mlp.w_up, mlp.w_down), (x, *mlp.parameters())
+            if what == "head":
+                return head.head_loss(x, mlp.w_gate, targets)[1], (x, mlp.w_gate.weight)
+            if what == "projection":
+                return linear.projections(x, mlp.w_gate)[0], (x, mlp.w_gate.weight)
+        if what == "flash_attn":
+            return fa.flash_attn(*(t.transpose(1, 2) for t in (q, k, v))), (q, k, v)
+        return (fa.flash_attn_bthd(q, k, v) if what == "flash_attn_bthd" else fa.flash_attn_bthd_rope(q, k, v, cos, sin)), (q, k, v)
+
+    def spread(t):  # the same values, every second element of a buffer
+        return t if t.dim() == 0 else torch.stack((t, t), -1)[..., 0]
+
+    ref = _saved_through(lambda t: t, f)
+    for a, b in zip(_saved_through(spread, f), ref):
+        # (the library may take another product for other strides: two bf16 roundings apart)
+        assert torch.equal(a, b) or not what.startswith("flash") and _rel(a, b.double()) < 2 * 2.0**-8
+    for bad in (lambda t: t.cpu(), lambda t: t.float() if t.dtype == torch.bfloat16 else t):
+        with pytest.raises(RuntimeError):
+            _saved_through(bad, f)
