@@ -38,10 +38,9 @@ def can_fuse(x: Tensor, cos: Tensor, sin: Tensor, heads: int, kv_heads: int, hd:
     """Whether ``attention_layer`` can stand for the layer's modules called on x."""
     if not eligible(x) or x.dim() != 3 or hd not in (32, 64):
         return False
-    d = x.shape[2]
+    B, T, d = x.shape
     if not (plain(wq, x, d) and plain(wk, x, d) and plain(wv, x, d) and plain(wo, x, heads * hd)):
         return False
-    B, T = x.shape[:2]
     # the library's row offsets within a sequence, and the rotation kernel's index
     if T * (heads + 2 * kv_heads) * hd >= 1 << 30 or B * T * (heads + kv_heads) * (hd // 16) >= 1 << 31:
         return False

@@ -31,19 +31,24 @@ _DTYPES = (torch.float16, torch.bfloat16)
 def plain(m: nn.Module, x: Tensor, width: int, odd_rows: bool = False) -> bool:
     """Whether m is an untouched bias-free nn.Linear with an fp32 weight on x's device for inputs of this width
     (and of a multiple of 8 outputs, unless odd_rows)."""
-    if type(m) is not nn.Linear or m.bias is not None or "forward" in m.__dict__:
+    if type(m) is not nn.Linear or "forward" in m.__dict__:
         return False
     if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
         return False
-    w = m.weight
-    return (type(w) is nn.Parameter and w.dtype is torch.float32 and w.device == x.device and w.is_contiguous()
-            and w.shape[1] == width and (odd_rows or w.shape[0] % 8 == 0) and width % 8 == 0 and w.data_ptr() % 16 == 0
-            and w.numel() < 1 << 31)  # the cast kernel's index, for up to four weights
+    own = m._parameters  # (read directly: a module's attribute lookup takes longer than the rest of this test)
+    w = own.get("weight")
+    if type(w) is not nn.Parameter or own.get("bias", m) is not None or w.dtype is not torch.float32 or w.device != x.device \
+            or not w.is_contiguous():
+        return False
+    n, k = w.shape
+    return (k == width and (odd_rows or n % 8 == 0) and k % 8 == 0 and n * k < 1 << 31  # the cast kernel's index, for four weights
+            and w.data_ptr() % 16 == 0)
 
 
 def function_mode() -> bool:
     """Whether a TorchFunctionMode is active that may intercept the modules' functions (torch.device's does not)."""
-    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+    n = torch._C._len_torch_function_stack()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
 
 
 def eligible(x: Tensor) -> bool:
