@@ -64,7 +64,9 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_de
 int code(at::ScalarType t) { return t == at::kHalf ? 0 : t == at::kBFloat16 ? 1 : t == at::kFloat ? 2 : -1; }
 int code(const Tensor& t) { return code(t.scalar_type()); }
 
-Tensor contig(const Tensor& t) { return t.is_contiguous() ? t : t.contiguous(); }
+// The tensor's values at its address: a gradient may come as a lazy negation of what lies there.
+Tensor real_values(const Tensor& t) { return t.is_neg() ? t.resolve_neg() : t; }
+Tensor contig(const Tensor& t) { return t.is_contiguous() && !t.is_neg() ? t : real_values(t).contiguous(); }
 Tensor empty_of(const Tensor& like, at::IntArrayRef shape) { return at::empty(shape, like.options()); }
 Tensor empty_f32(const Tensor& like, at::IntArrayRef shape) { return at::empty(shape, like.options().dtype(at::kFloat)); }
 Tensor bytes(const Tensor& like, size_t n) { return at::empty({(int64_t)n}, like.options().dtype(at::kByte)); }
@@ -117,7 +119,10 @@ S3 known_strides(const Tensor& t) { return t.is_contiguous() ? dense_strides(t) 
 // (as it takes k and v, and q and dO).
 void make_readable(std::initializer_list<Tensor*> ts) {
     bool dense = true;
-    for (Tensor* t : ts) dense = dense && t->is_contiguous();
+    for (Tensor* t : ts) {
+        *t = real_values(*t);
+        dense = dense && t->is_contiguous();
+    }
     if (dense) return;
     std::optional<S3> first;
     bool ok = true;

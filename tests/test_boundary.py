@@ -564,3 +564,12 @@ def test_host_functions_refuse_host_tensors():
               lambda: h.bthd_rope_bwd(q4, q4, q4, q4, q4, lse, cos, cos)):
         with pytest.raises(RuntimeError, match="must be CUDA tensors|on the inputs' device"):
             f()
+
+
+def test_lazy_negations_are_resolved_before_a_kernel_reads_them():
+    from nanonemo_amd.kernels.hip import host
+
+    t = torch.randn(1, 2, 16, 32, dtype=torch.complex64).conj().imag
+    assert t.is_neg()
+    for out in (*host().readable(t), *host().readable(t, t)):
+        assert not out.is_neg() and torch.equal(out, t)

@@ -236,3 +236,26 @@ def test_tensors_of_another_device_are_refused_before_any_launch():
               lambda: ops.flash_attn_bthd_rope_bwd(t, t, t, t, t, lse, cos, sin)):
         with pytest.raises(RuntimeError, match="CUDA tensors|inputs' device"):
             f()
+
+
+def test_lazily_negated_gradients():
+    # the imaginary part of a conjugate is a view that negates when it is read
+    import nanonemo_amd.kernels.hip.flash_attn as fa
+    from nanonemo_amd.kernels.hip import rmsnorm, rope
+    from nanonemo_amd.model import rope_tables
+
+    cos, sin = (t.to(DEV) for t in rope_tables(64, 16, 10000.0))
+    x, w = torch.randn(1, 16, 2, 64, device=DEV), torch.ones(64, device=DEV)
+    q = x.bfloat16()
+    for a, f in ((q, lambda a: fa.flash_attn(*[a.transpose(1, 2)] * 3).transpose(1, 2)), (q, lambda a: fa.flash_attn_bthd(a, a, a)),
+                 (q, lambda a: fa.flash_attn_bthd_rope(a, a, a, cos, sin)), (x, lambda a: rope.rope_k(a, cos, sin)),
+                 (x, lambda a: rmsnorm.add_rms_norm(a, None, w, 1e-5)[0])):
+        a = a.clone().requires_grad_()
+        y = f(a)
+        g = torch.randn(*y.shape, dtype=torch.complex64, device=DEV).conj().imag
+        if y.dtype == torch.float32:
+            assert g.is_neg()
+        else:
+            g = torch._neg_view(torch.randn_like(y))
+        got = torch.autograd.grad(y, a, g, retain_graph=True)[0]
+        assert torch.equal(got, torch.autograd.grad(y, a, g.resolve_neg())[0])
